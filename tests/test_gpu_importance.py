@@ -51,6 +51,32 @@ def test_residual_crop_scores_int16(dev, mode):
     assert_bits_equal(got, want, f"mode {mode}")
 
 
+@pytest.mark.parametrize("H,W,C,ph,pw,prev,offset", [
+    (16, 16, 3, 16, 16, True, 0),       # one patch: fewer chunks than threads
+    (32, 1600, 3, 16, 16, True, 0),     # more chunks than one round of the workgroup
+    (28, 32, 4, 14, 8, False, 0),       # another patch shape in whole chunks, no previous frame
+    (32, 48, 3, 16, 8, True, 0),        # 24-byte patch rows: the general kernel
+    (32, 32, 3, 16, 16, True, 1),       # frames off 16-byte alignment: the general kernel
+])
+@pytest.mark.parametrize("mode", [OI.RMS, OI.ENERGY, OI.L2])
+def test_residual_score_uint8_layouts(dev, H, W, C, ph, pw, prev, offset, mode):
+    """uint8 frames in and out of the streaming kernel's layouts, bit for bit, extreme differences included."""
+    rng = np.random.default_rng(H + W + mode)
+    curr = rng.choice([0, 1, 254, 255], (2, H, W, C)).astype(np.uint8)
+    old = rng.choice([0, 255], (2, H, W, C)).astype(np.uint8) if prev else None
+
+    def place(a):
+        if a is None:
+            return None
+        buf = torch.empty(a.size + offset, dtype=torch.uint8, device=dev)
+        t = buf[offset:].view(a.shape)
+        t.copy_(torch.from_numpy(a))
+        return t
+
+    got = K.patch_residual_score(place(curr), place(old), (ph, pw), MODES[mode])
+    assert_bits_equal(got, OI.patch_residual_score(curr, old, ph, pw, mode), f"mode {mode}")
+
+
 def test_residual_score_fp32_and_bad_index(dev):
     rng = np.random.default_rng(9)
     curr = (rng.integers(-2048, 2048, (3, 64, 80, 3)) / 256.0).astype(np.float32)
