@@ -2,15 +2,16 @@
 // heads and all queries (patch_attn_prob / patch_attn_prob_layermean).
 //
 // Nothing of size N x N is materialised:
-//   stats:  for every (image, head, query) the softmax max m and sum l over all keys (two passes over
-//           the keys, so that every term exp(s - m) uses the final max, as a row softmax does);
+//   stats:  for every (image, head, query) the softmax max m and sum l over all keys, in one pass over
+//           the keys with a running max;
 //   colsum: dense mode, for every (image, 128-query block, 128-key block) the column sums over its
 //           queries of the head-mean probabilities, then the query blocks added in order; log-sum-exp
 //           mode, one pass per (256-key block, head group, image) from the row LSE (the stats launch's,
 //           or the attention's own), then the head groups added in order.
 //
 // Rounding modes (the two paths of attention.py:241-253 and triton_kernels/attention_pscore.py):
-//   kDense: s = bf16(bf16(q.k) * scale), p = bf16(exp(s - m) / l) (torch softmax of a bf16 tensor),
+//   kDense: s = bf16(bf16(q.k) * scale), p = bf16(exp(s - m) / l) (torch softmax of a bf16 tensor;
+//           formed as exp2 of one exponent that holds the max and the sum),
 //           head mean hm = bf16(sum_h p * fl(1/H)), score = bf16(sum_q hm * fl(1/N));
 //   kLse:   s = (q.k) in fp32, lse = m + log(l), p = exp2(s * (scale log2e) - lse * log2e) in fp32,
 //           score = bf16(sum_{q,h} p * fl(1/(H N))) -- the fused kernel's key-side sum from the row
@@ -20,6 +21,7 @@
 // lane pair and the sum over queries is a register sum plus one exchange.
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 
 #include "common.hpp"
 
@@ -43,41 +45,64 @@ __device__ __forceinline__ void round2_bf16(float& a, float& b) {
   b = __uint_as_float(p & 0xffff0000u);
 }
 
-// The scores of one 32 x 32 MFMA block in place: dense s = bf16(bf16(q.k) * scale), log-sum-exp mode
-// s = (q.k) * scale.
-template <int MODE>
+static constexpr float kLog2e = 1.4426950408889634f;
+
+// How a kernel forms its scores from the fp32 products a = q.k (scale > 0 for kDenseP2):
+//   kDense     s = bf16(bf16(a) * scale)
+//   kDenseP2   the same for a power-of-two scale, whose second rounding changes nothing: the kernel keeps
+//              v = bf16(a) and the scale moves into the exponent's factor
+//   kLse       s = a * scale
+// In all of them exp(s - m) = exp2(v * kf - m * kf) with v and m in the kernel's own units and kf =
+// score_factor: one FMA and one v_exp_f32 per score.
+static constexpr int kDenseP2 = 2;
+
+__host__ __device__ __forceinline__ float score_factor(int form, float scale) {
+  return form == kDenseP2 ? scale * kLog2e : kLog2e;
+}
+
+// The scores of one 32 x 32 MFMA block in place, in the kernel's units.
+template <int FORM>
 __device__ __forceinline__ void block_scores(f32x16_t& acc, float scale) {
 #pragma unroll
   for (int v = 0; v < 16; v += 2) {
     float a = acc[v], c = acc[v + 1];
-    if (MODE == kDense) {
-      round2_bf16(a, c);
-      a *= scale;
-      c *= scale;
-      round2_bf16(a, c);
-    } else {
+    if (FORM != kLse) round2_bf16(a, c);
+    if (FORM != kDenseP2) {
       a *= scale;
       c *= scale;
     }
+    if (FORM == kDense) round2_bf16(a, c);
     acc[v] = a;
     acc[v + 1] = c;
   }
 }
 
+// Work item of workgroup `bid` among `n`: dispatch places workgroup i on XCD i % 8, so XCD x takes the
+// contiguous band of items [x q + min(x, r), ...) (q = n / 8, r = n % 8) and the workgroups that share an
+// image's Q and K share an L2.
+__device__ __forceinline__ int xcd_band(int bid, int n) {
+  const int x = bid & 7, q = n >> 3, r = n & 7;
+  return x * q + min(x, r) + (bid >> 3);
+}
+
 // Row statistics: workgroup = (256 queries = 8 waves x 32, head, image). Key tiles of 64 (two 32-key
 // MFMA blocks) are staged once in LDS for all waves, double-buffered through registers (16-byte chunks
-// XOR-swizzled by row); S^T = K . Q^T puts a query's scores in one lane pair (lanes l, l ^ 32). Two
-// passes over the keys, the max and then the sum of exp(s - max) with the final max, as a row softmax
-// computes them. Waves whose queries lie past N still stage tiles and meet every barrier.
+// XOR-swizzled by row); S^T = K . Q^T puts a query's scores in one lane pair (lanes l, l ^ 32). One pass:
+// each lane keeps the running max of its half of the keys and the sum of exp(s - max), rescaled per tile
+// (the max is exact in any order; a tile's terms are summed apart and then added, which rounds less than
+// one long chain); the two lanes of a query merge at the end. Bound by the VALU (one exponential per
+// score): two passes over the keys with expf before, 266 -> 101 us at 16 images x 16 heads x 1029^2.
+// Output: kLse the row log-sum-exp (natural log), dense the row's exponent offset m kf + log2(l), so that
+// a probability is exp2(v kf - offset). Waves whose queries lie past N still stage tiles and meet every
+// barrier.
 static constexpr int kStWaves = 8;
 static constexpr int kStKeys = 64;
 
-template <int DH, int MODE>
+template <int DH, int FORM>
 __global__ __launch_bounds__(kStWaves * 64) void pattn_stats_kernel(const uint16_t* __restrict__ q, int64_t qrs,
                                                                     const uint16_t* __restrict__ kv, int64_t kvb,
                                                                     int64_t kvn, int64_t kvh, int N, int H,
-                                                                    float scale, float* __restrict__ m_out,
-                                                                    float* __restrict__ l_out) {
+                                                                    float scale, float* __restrict__ row_out) {
   constexpr int KS = DH / 16;
   constexpr int CPR = DH / 8;
   constexpr int CHUNKS = kStKeys * CPR;
@@ -85,10 +110,14 @@ __global__ __launch_bounds__(kStWaves * 64) void pattn_stats_kernel(const uint16
   constexpr int IT = CHUNKS / NT;
   static_assert(CHUNKS % NT == 0, "whole chunks per thread");
   __shared__ __align__(16) unsigned char kt[2][kStKeys * DH * 2];
-  const int b = blockIdx.z, h = blockIdx.y;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int nqb = (N + 32 * kStWaves - 1) / (32 * kStWaves);
+  const int item = xcd_band((int)blockIdx.x, (int)gridDim.x);
+  const int qb_ = item % nqb, pair = item / nqb;
+  const int h = pair % H, b = pair / H;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, g = lane >> 5;
-  const int q0 = (blockIdx.x * kStWaves + wave) * 32;
+  const int q0 = (qb_ * kStWaves + wave) * 32;
   const bool active = q0 < N;
   const uint16_t* qb = q + (int64_t)b * N * qrs + (int64_t)h * DH;
   const uint16_t* kb = kv + (int64_t)b * kvb + (int64_t)h * kvh;
@@ -96,54 +125,30 @@ __global__ __launch_bounds__(kStWaves * 64) void pattn_stats_kernel(const uint16
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) qf[ks] = frag16(qb, qrs, q0 + l32, N, ks * 16 + 8 * g);
   const int ntiles = (N + kStKeys - 1) / kStKeys;
+  const float kf = score_factor(FORM, scale);
 
-  uint4 rk[IT];
-  auto load = [&](int t) {
+  u32x4_t rk[IT];
+  auto load = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
       const int c = tid + i * NT;
       const int r = c / CPR, ch = c - r * CPR;
       const int key = t * kStKeys + r;
-      rk[i] = make_uint4(0, 0, 0, 0);
-      if (key < N) rk[i] = *reinterpret_cast<const uint4*>(kb + (int64_t)key * kvn + ch * 8);
+      rk[i] = u32x4_t{0, 0, 0, 0};
+      if (key < N) rk[i] = *reinterpret_cast<const u32x4_t*>(kb + (int64_t)key * kvn + ch * 8);
     }
   };
-  auto store = [&](int buf) {
+  auto store = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
       const int c = tid + i * NT;
       const int r = c / CPR, ch = c - r * CPR;
-      *reinterpret_cast<uint4*>(&kt[buf][r * DH * 2 + ((ch ^ (r & (CPR - 1))) << 4)]) = rk[i];
-    }
-  };
-  auto scores = [&](int buf, f32x16_t (&acc)[2]) {
-#pragma unroll
-    for (int kb2 = 0; kb2 < 2; ++kb2) {
-      const int r = kb2 * 32 + l32;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[kb2][v] = 0.0f;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int ch = 2 * ks + g;
-        const bf16x8_t kf =
-            as_bf16x8(*reinterpret_cast<const uint4*>(&kt[buf][r * DH * 2 + ((ch ^ (r & (CPR - 1))) << 4)]));
-        acc[kb2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], acc[kb2], 0, 0, 0);
-      }
-      block_scores<MODE>(acc[kb2], scale);
-    }
-  };
-  // Keys past N exist only in the last tile: there the scores of those keys become -inf.
-  auto mask_tail = [&](int t, f32x16_t (&acc)[2]) {
-    if ((t + 1) * kStKeys > N) {
-#pragma unroll
-      for (int kb2 = 0; kb2 < 2; ++kb2)
-#pragma unroll
-        for (int v = 0; v < 16; ++v)
-          if (t * kStKeys + kb2 * 32 + 8 * (v >> 2) + 4 * g + (v & 3) >= N) acc[kb2][v] = -INFINITY;
+      *reinterpret_cast<u32x4_t*>(&kt[buf][r * DH * 2 + ((ch ^ (r & (CPR - 1))) << 4)]) = rk[i];
     }
   };
 
-  float m = -INFINITY;
+  // Finite start: a lane whose keys all lie past N keeps it, with an empty sum.
+  float m = -3.0e38f, l = 0.0f;
   load(0);
   store(0);
   __syncthreads();
@@ -152,62 +157,77 @@ __global__ __launch_bounds__(kStWaves * 64) void pattn_stats_kernel(const uint16
     if (t + 1 < ntiles) load(t + 1);
     if (active) {
       f32x16_t acc[2];
-      scores(buf, acc);
-      mask_tail(t, acc);
+#pragma unroll
+      for (int kb2 = 0; kb2 < 2; ++kb2) {
+        const int r = kb2 * 32 + l32;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[kb2][v] = 0.0f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          const int ch = 2 * ks + g;
+          const bf16x8_t kfr =
+              as_bf16x8(*reinterpret_cast<const uint4*>(&kt[buf][r * DH * 2 + ((ch ^ (r & (CPR - 1))) << 4)]));
+          acc[kb2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kfr, qf[ks], acc[kb2], 0, 0, 0);
+        }
+        block_scores<FORM>(acc[kb2], scale);
+      }
+      // Keys past N exist only in the last tile: there the scores of those keys become -inf.
+      if ((t + 1) * kStKeys > N) {
+#pragma unroll
+        for (int kb2 = 0; kb2 < 2; ++kb2)
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            if (t * kStKeys + kb2 * 32 + 8 * (v >> 2) + 4 * g + (v & 3) >= N) acc[kb2][v] = -INFINITY;
+      }
+      float mx[4];
+#pragma unroll
+      for (int c4 = 0; c4 < 4; ++c4) {
+        mx[c4] = acc[c4 >> 1][8 * (c4 & 1)];
+#pragma unroll
+        for (int v = 1; v < 8; ++v) mx[c4] = fmaxf(mx[c4], acc[c4 >> 1][8 * (c4 & 1) + v]);
+      }
+      const float m_new = fmaxf(fmaxf(m, fmaxf(mx[0], mx[1])), fmaxf(mx[2], mx[3]));
+      const float alpha = __builtin_amdgcn_exp2f((m - m_new) * kf);
+      const float off = m_new * kf;
+      float ts[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int kb2 = 0; kb2 < 2; ++kb2)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) m = fmaxf(m, acc[kb2][v]);
+        for (int v = 0; v < 16; ++v) ts[v & 3] += __builtin_amdgcn_exp2f(fmaf(acc[kb2][v], kf, -off));
+      l = fmaf(l, alpha, (ts[0] + ts[1]) + (ts[2] + ts[3]));
+      m = m_new;
     }
     if (t + 1 < ntiles) store(buf ^ 1);
     __syncthreads();
   }
-  m = fmaxf(m, __shfl_xor(m, 32, 64));
-  float l = 0.0f;
-  load(0);
-  store(0);
-  __syncthreads();
-  for (int t = 0; t < ntiles; ++t) {
-    const int buf = t & 1;
-    if (t + 1 < ntiles) load(t + 1);
-    if (active) {
-      f32x16_t acc[2];
-      scores(buf, acc);
-      mask_tail(t, acc);
-#pragma unroll
-      for (int kb2 = 0; kb2 < 2; ++kb2)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) l += expf(acc[kb2][v] - m);
-    }
-    if (t + 1 < ntiles) store(buf ^ 1);
-    __syncthreads();
-  }
-  l += __shfl_xor(l, 32, 64);
+  const float m2 = __shfl_xor(m, 32, 64), l2 = __shfl_xor(l, 32, 64);
+  const float mt = fmaxf(m, m2);
+  l = l * __builtin_amdgcn_exp2f((m - mt) * kf) + l2 * __builtin_amdgcn_exp2f((m2 - mt) * kf);
   const int qi = q0 + l32;
-  if (active && g == 0 && qi < N) {
-    const int64_t o = ((int64_t)b * H + h) * N + qi;
-    m_out[o] = MODE == kDense ? m : m + logf(l);  // kLse keeps the row log-sum-exp in m_out
-    l_out[o] = l;
-  }
+  if (active && g == 0 && qi < N)
+    row_out[((int64_t)b * H + h) * N + qi] = FORM == kLse ? mt + logf(l) : fmaf(mt, kf, log2f(l));
 }
 
 // Dense key-side score: workgroup = (128-query block, 128-key block, image), 8 waves; wave w takes
 // queries 32 (w % 4) .. + 31 and keys 64 (w / 4) .. + 63 of the tile (two 32-key MFMA blocks, S = Q . K^T
 // so a key's column sits in one lane pair). For every head the Q and K tiles (128 x DH each, swizzled
-// 16-byte chunks) and the 128 queries' row max and sum are staged once in LDS, double-buffered through
-// registers; p = bf16(exp(s - m) / l) (the quotient by one correction step from the reciprocal,
-// q0 = e r, q = fma(fma(-q0, l, e), r, q0), the correctly rounded quotient for normal results) is
-// summed over heads per (query, key) in registers. After the last head each (query, key) takes
-// bf16(sum * fl(1/H)); the tile's column sums over its queries (four query waves added in order in
-// LDS) go to part[b][query block][key], and pattn_dense_reduce_kernel adds the query blocks in order.
+// 16-byte chunks) and the 128 queries' exponent offsets (pattn_stats_kernel) are staged once in LDS,
+// double-buffered through registers; p = bf16(exp2(v kf - offset)) is summed over heads per (query, key)
+// in registers. After the last head each (query, key) takes bf16(sum * fl(1/H)); the tile's column sums
+// over its queries (four query waves added in order in LDS) go to part[b][query block][key], and
+// pattn_dense_reduce_kernel adds the query blocks in order. Waves wholly past N compute nothing
+// (N = 1029 is 8 tiles and 5 rows). Bound by the VALU (one exponential and two to three bf16
+// roundings per score and head): with expf and a divided quotient before, 344 -> 123 us at 16 images x 16
+// heads x 1029^2.
 static constexpr int kDnTile = 128;
 
-template <int DH>
-__global__ __launch_bounds__(512) void pattn_colsum_kernel(const uint16_t* __restrict__ q, int64_t qrs,
+// Two workgroups per CU at DH = 64 (LDS 66 KB each, so the registers are held to 128); one at DH = 128.
+// OFF: the type of a lane's element offset from its tile's first row (32 bits while 128 rows span less).
+template <int DH, int FORM, typename OFF>
+__global__ __launch_bounds__(512, DH == 64 ? 4 : 2) void pattn_colsum_kernel(const uint16_t* __restrict__ q, int64_t qrs,
                                                            const uint16_t* __restrict__ kv, int64_t kvb, int64_t kvn,
                                                            int64_t kvh, int N, int H, float scale,
-                                                           const float* __restrict__ m_in,
-                                                           const float* __restrict__ l_in,
+                                                           const float* __restrict__ row_in,
                                                            float* __restrict__ part) {
   constexpr int KS = DH / 16;
   constexpr int CPR = DH / 8;
@@ -218,54 +238,48 @@ __global__ __launch_bounds__(512) void pattn_colsum_kernel(const uint16_t* __res
   constexpr int IT = CHUNKS / NT;
   static_assert(CHUNKS % NT == 0, "whole chunks per thread");
   __shared__ __align__(16) unsigned char tiles[2][2 * TILEB];
-  __shared__ __align__(16) float st[2][3][kDnTile];  // row max, row sum, 1 / row sum
+  __shared__ __align__(16) float st[2][kDnTile];  // row offsets
   __shared__ float colp[4][kDnTile];
-  const int b = blockIdx.z;
-  const int qt0 = blockIdx.y * kDnTile, kt0 = blockIdx.x * kDnTile;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int nb = (N + kDnTile - 1) / kDnTile;  // query blocks = key blocks
+  const int item = xcd_band((int)blockIdx.x, (int)gridDim.x);
+  const int kblk = item % nb, qblk = item / nb % nb, b = item / (nb * nb);
+  const int qt0 = qblk * kDnTile, kt0 = kblk * kDnTile;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, g = lane >> 5;
   const int wq = 32 * (wave & 3), wk = 64 * (wave >> 2);
-  const uint16_t* qimg = q + (int64_t)b * N * qrs;
-  const uint16_t* kimg = kv + (int64_t)b * kvb;
+  const bool active = qt0 + wq < N && kt0 + wk < N;
+  const float kf = score_factor(FORM, scale);
 
-  uint4 rq[IT];
-  float rs = 0.0f;
-  auto load = [&](int h) {
+  // Rows past N repeat row N - 1: their scores reach no stored column and no counted query. Offsets are
+  // relative to the tile's first row, the head's base pointers uniform.
+  const uint16_t* qbase = q + ((int64_t)b * N + qt0) * qrs;
+  const uint16_t* kbase = kv + (int64_t)b * kvb + (int64_t)kt0 * kvn;
+  OFF off_[IT];
 #pragma unroll
-    for (int i = 0; i < IT; ++i) {
-      const int c = tid + i * NT;
-      const int isk = c >= kDnTile * CPR;
-      const int cc = c - isk * kDnTile * CPR;
-      const int r = cc / CPR, ch = cc - r * CPR;
-      rq[i] = make_uint4(0, 0, 0, 0);
-      if (isk) {
-        if (kt0 + r < N)
-          rq[i] = *reinterpret_cast<const uint4*>(kimg + (int64_t)(kt0 + r) * kvn + (int64_t)h * kvh + ch * 8);
-      } else if (qt0 + r < N) {
-        rq[i] = *reinterpret_cast<const uint4*>(qimg + (int64_t)(qt0 + r) * qrs + (int64_t)h * DH + ch * 8);
-      }
-    }
-    if (tid < 2 * kDnTile) {
-      const int r = tid & (kDnTile - 1);
-      const float* src = tid < kDnTile ? m_in : l_in;
-      rs = qt0 + r < N ? src[((int64_t)b * H + h) * N + qt0 + r] : (tid < kDnTile ? 0.0f : 1.0f);
-    }
+  for (int i = 0; i < IT; ++i) {
+    const int c = tid + (i % (IT / 2)) * NT;
+    const int r = c / CPR, ch = c - r * CPR;
+    off_[i] = i < IT / 2 ? (OFF)min(r, N - 1 - qt0) * (OFF)qrs + (OFF)(ch * 8)
+                         : (OFF)min(r, N - 1 - kt0) * (OFF)kvn + (OFF)(ch * 8);
+  }
+  u32x4_t rq[IT];
+  float rs = INFINITY;
+  auto load = [&](int h) __attribute__((always_inline)) {
+    const uint16_t* qh = qbase + (int64_t)h * DH;
+    const uint16_t* kh = kbase + (int64_t)h * kvh;
+#pragma unroll
+    for (int i = 0; i < IT; ++i) rq[i] = *reinterpret_cast<const u32x4_t*>((i < IT / 2 ? qh : kh) + off_[i]);
+    if (tid < kDnTile && qt0 + tid < N) rs = row_in[((int64_t)b * H + h) * N + qt0 + tid];
   };
-  auto store = [&](int buf) {
+  auto store = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
-      const int c = tid + i * NT;
-      const int isk = c >= kDnTile * CPR;
-      const int cc = c - isk * kDnTile * CPR;
-      const int r = cc / CPR, ch = cc - r * CPR;
-      *reinterpret_cast<uint4*>(&tiles[buf][isk * TILEB + r * ROWB + ((ch ^ (r & (CPR - 1))) << 4)]) = rq[i];
+      const int c = tid + (i % (IT / 2)) * NT;
+      const int r = c / CPR, ch = c - r * CPR;
+      *reinterpret_cast<u32x4_t*>(&tiles[buf][(i < IT / 2 ? 0 : TILEB) + r * ROWB + ((ch ^ (r & (CPR - 1))) << 4)]) = rq[i];
     }
-    if (tid < kDnTile) {
-      st[buf][0][tid] = rs;
-    } else if (tid < 2 * kDnTile) {
-      st[buf][1][tid - kDnTile] = rs;
-      st[buf][2][tid - kDnTile] = 1.0f / rs;
-    }
+    if (tid < kDnTile) st[buf][tid] = rs;
   };
 
   float hs[2][16];
@@ -280,59 +294,41 @@ __global__ __launch_bounds__(512) void pattn_colsum_kernel(const uint16_t* __res
   for (int h = 0; h < H; ++h) {
     const int buf = h & 1;
     if (h + 1 < H) load(h + 1);
-    const unsigned char* qs = tiles[buf];
-    const unsigned char* ks = tiles[buf] + TILEB;
-    f32x16_t acc[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[j][v] = 0.0f;
-#pragma unroll
-    for (int kstep = 0; kstep < KS; ++kstep) {
-      const int ch = 2 * kstep + g;
+    if (active) {
+      const unsigned char* qs = tiles[buf];
+      const unsigned char* ks = tiles[buf] + TILEB;
+      bf16x8_t qf[KS];
       const int rq_ = wq + l32;
-      const bf16x8_t qf = as_bf16x8(*reinterpret_cast<const uint4*>(qs + rq_ * ROWB + ((ch ^ (rq_ & (CPR - 1))) << 4)));
+#pragma unroll
+      for (int kstep = 0; kstep < KS; ++kstep)
+        qf[kstep] = as_bf16x8(
+            *reinterpret_cast<const uint4*>(qs + rq_ * ROWB + (((2 * kstep + g) ^ (rq_ & (CPR - 1))) << 4)));
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
+        __builtin_amdgcn_sched_barrier(0);  // one block's scores in registers at a time
+        f32x16_t acc;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
         const int rk_ = wk + 32 * j + l32;
-        const bf16x8_t kf =
-            as_bf16x8(*reinterpret_cast<const uint4*>(ks + rk_ * ROWB + ((ch ^ (rk_ & (CPR - 1))) << 4)));
-        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf, kf, acc[j], 0, 0, 0);
-      }
-    }
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const int r0 = wq + 8 * a + 4 * g;
-      const float4 m4 = *reinterpret_cast<const float4*>(&st[buf][0][r0]);
-      const float4 l4 = *reinterpret_cast<const float4*>(&st[buf][1][r0]);
-      const float4 i4 = *reinterpret_cast<const float4*>(&st[buf][2][r0]);
-      const float mm[4] = {m4.x, m4.y, m4.z, m4.w};
-      const float ll[4] = {l4.x, l4.y, l4.z, l4.w};
-      const float ii[4] = {i4.x, i4.y, i4.z, i4.w};
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        float sv[4];
-#pragma unroll
-        for (int e = 0; e < 4; e += 2) {
-          float x0 = acc[j][4 * a + e], x1 = acc[j][4 * a + e + 1];
-          round2_bf16(x0, x1);
-          x0 *= scale;
-          x1 *= scale;
-          round2_bf16(x0, x1);
-          sv[e] = x0;
-          sv[e + 1] = x1;
+        for (int kstep = 0; kstep < KS; ++kstep) {
+          const bf16x8_t kfr = as_bf16x8(
+              *reinterpret_cast<const uint4*>(ks + rk_ * ROWB + (((2 * kstep + g) ^ (rk_ & (CPR - 1))) << 4)));
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf[kstep], kfr, acc, 0, 0, 0);
         }
-        float pv[4];
+        block_scores<FORM>(acc, scale);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float ex = expf(sv[e] - mm[e]);
-          const float q0 = ex * ii[e];
-          pv[e] = fmaf(fmaf(-q0, ll[e], ex), ii[e], q0);
+        for (int a = 0; a < 4; ++a) {
+          const float4 o4 = *reinterpret_cast<const float4*>(&st[buf][wq + 8 * a + 4 * g]);
+          const float off[4] = {o4.x, o4.y, o4.z, o4.w};
+          float pv[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) pv[e] = __builtin_amdgcn_exp2f(fmaf(acc[4 * a + e], kf, -off[e]));
+          round2_bf16(pv[0], pv[1]);
+          round2_bf16(pv[2], pv[3]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) hs[j][4 * a + e] += pv[e];
         }
-        round2_bf16(pv[0], pv[1]);
-        round2_bf16(pv[2], pv[3]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) hs[j][4 * a + e] += pv[e];
       }
     }
     if (h + 1 < H) store(buf ^ 1);
@@ -357,7 +353,7 @@ __global__ __launch_bounds__(512) void pattn_colsum_kernel(const uint16_t* __res
   __syncthreads();
   if (tid < kDnTile && kt0 + tid < N) {
     const float t = ((colp[0][tid] + colp[1][tid]) + colp[2][tid]) + colp[3][tid];
-    part[((int64_t)b * gridDim.y + blockIdx.y) * N + kt0 + tid] = t;
+    part[((int64_t)b * nb + qblk) * N + kt0 + tid] = t;
   }
 }
 
@@ -394,11 +390,11 @@ __global__ __launch_bounds__(kLseWaves * 64) void pattn_colsum_lse_kernel(
   constexpr int CHUNKS = 32 * CPR;     // chunks per query tile
   constexpr int NT = kLseWaves * 64;
   constexpr int IT = (CHUNKS + NT - 1) / NT;
-  constexpr float kLog2e = 1.4426950408889634f;
   __shared__ __align__(16) unsigned char qs[2][32 * DH * 2];
   __shared__ __align__(16) float ls[2][32];
   const int b = blockIdx.z, grp = blockIdx.y;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, g = lane >> 5;
   const int key = blockIdx.x * kLseKeys + wave * 32 + l32;
   const int nqb = (N + 31) / 32;
@@ -408,28 +404,28 @@ __global__ __launch_bounds__(kLseWaves * 64) void pattn_colsum_lse_kernel(
   const uint16_t* qimg = q + (int64_t)b * N * qrs;
   const float* limg = lse + (int64_t)b * H * N;
 
-  uint4 rq[IT];
+  u32x4_t rq[IT];
   float rl = INFINITY;
-  auto load = [&](int st) {
+  auto load = [&](int st) __attribute__((always_inline)) {
     const int h = h0 + st / nqb, q0 = (st % nqb) * 32;
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
       const int c = tid + i * NT;
-      rq[i] = make_uint4(0, 0, 0, 0);
+      rq[i] = u32x4_t{0, 0, 0, 0};
       if (c < CHUNKS) {
         const int r = c / CPR, ch = c - r * CPR;
-        if (q0 + r < N) rq[i] = *reinterpret_cast<const uint4*>(qimg + (int64_t)(q0 + r) * qrs + (int64_t)h * DH + ch * 8);
+        if (q0 + r < N) rq[i] = *reinterpret_cast<const u32x4_t*>(qimg + (int64_t)(q0 + r) * qrs + (int64_t)h * DH + ch * 8);
       }
     }
     if (tid < 32) rl = q0 + tid < N ? limg[(int64_t)h * N + q0 + tid] * kLog2e : INFINITY;
   };
-  auto store = [&](int buf) {
+  auto store = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
       const int c = tid + i * NT;
       if (c < CHUNKS) {
         const int r = c / CPR, ch = c - r * CPR;
-        *reinterpret_cast<uint4*>(&qs[buf][r * DH * 2 + ((ch ^ (r & (CPR - 1))) << 4)]) = rq[i];
+        *reinterpret_cast<u32x4_t*>(&qs[buf][r * DH * 2 + ((ch ^ (r & (CPR - 1))) << 4)]) = rq[i];
       }
     }
     if (tid < 32) ls[buf][tid] = rl;
@@ -506,7 +502,6 @@ template <int DH>
 void launch_colsum_lse(const uint16_t* q, int64_t qrs, const uint16_t* kv, int64_t kvb, int64_t kvn, int64_t kvh,
                        int B, int N, int H, float scale, const float* lse, float* part, uint16_t* out, int64_t osb,
                        hipStream_t st) {
-  constexpr float kLog2e = 1.4426950408889634f;
   const int hpg = lse_heads_per_group(B, N, H);
   const int groups = (H + hpg - 1) / hpg;
   const dim3 g1((unsigned)cdiv(N, kLseKeys), (unsigned)groups, (unsigned)B);
@@ -517,25 +512,38 @@ void launch_colsum_lse(const uint16_t* q, int64_t qrs, const uint16_t* kv, int64
                                                                   1.0f / (float)((int64_t)H * N), out, osb);
 }
 
-template <int DH, int MODE>
+// FORM kLse, kDense or kDenseP2 (the dense mode with a positive power-of-two scale, e.g. 64^-0.5 = 1/8).
+template <int DH, int FORM>
 void launch_pattn(const uint16_t* q, int64_t qrs, const uint16_t* kv, int64_t kvb, int64_t kvn, int64_t kvh, int B,
                   int N, int H, float scale, float* ws, uint16_t* out, int64_t osb, hipStream_t st) {
-  float* m = ws;
-  float* l = ws + (int64_t)B * H * N;
-  const dim3 g1((unsigned)cdiv(N, 32 * kStWaves), (unsigned)H, (unsigned)B);
-  pattn_stats_kernel<DH, MODE><<<g1, kStWaves * 64, 0, st>>>(q, qrs, kv, kvb, kvn, kvh, N, H, scale, m, l);
-  if constexpr (MODE == kLse) {
-    // m holds the row log-sum-exp; l (no longer read) takes the partial column sums.
-    launch_colsum_lse<DH>(q, qrs, kv, kvb, kvn, kvh, B, N, H, scale, m, l, out, osb, st);
+  float* row = ws;  // the row log-sum-exp, or the dense mode's exponent offset
+  const unsigned g1 = (unsigned)(cdiv(N, 32 * kStWaves) * H * B);
+  pattn_stats_kernel<DH, FORM><<<g1, kStWaves * 64, 0, st>>>(q, qrs, kv, kvb, kvn, kvh, N, H, scale, row);
+  if constexpr (FORM == kLse) {
+    launch_colsum_lse<DH>(q, qrs, kv, kvb, kvn, kvh, B, N, H, scale, row, ws + (int64_t)B * H * N, out, osb, st);
   } else {
     // Partial column sums per 128-query block after the statistics.
     float* part = ws + 2 * (int64_t)B * H * N;
     const int nqb = (int)cdiv(N, kDnTile);
-    const dim3 g2((unsigned)cdiv(N, kDnTile), (unsigned)nqb, (unsigned)B);
-    pattn_colsum_kernel<DH><<<g2, 512, 0, st>>>(q, qrs, kv, kvb, kvn, kvh, N, H, scale, m, l, part);
+    const unsigned g2 = (unsigned)(nqb * nqb * B);
+    if (std::max(std::abs(qrs), std::abs(kvn)) < ((int64_t)1 << 24))
+      pattn_colsum_kernel<DH, FORM, uint32_t>
+          <<<g2, 512, 0, st>>>(q, qrs, kv, kvb, kvn, kvh, N, H, scale, row, part);
+    else
+      pattn_colsum_kernel<DH, FORM, int64_t><<<g2, 512, 0, st>>>(q, qrs, kv, kvb, kvn, kvh, N, H, scale, row, part);
     const int64_t n = (int64_t)B * N;
     pattn_dense_reduce_kernel<<<(unsigned)cdiv(n, 256), 256, 0, st>>>(part, B, N, nqb, out, osb);
   }
+}
+
+template <int DH>
+void launch_pattn_mode(const uint16_t* q, int64_t qrs, const uint16_t* kv, int64_t kvb, int64_t kvn, int64_t kvh, int B,
+                       int N, int H, float scale, int mode, float* ws, uint16_t* out, int64_t osb, hipStream_t st) {
+  int e = 0;
+  const bool pow2 = scale > 0.0f && std::isfinite(scale) && std::frexp(scale, &e) == 0.5f && std::abs(e) < 64;
+  if (mode == kLse) launch_pattn<DH, kLse>(q, qrs, kv, kvb, kvn, kvh, B, N, H, scale, ws, out, osb, st);
+  else if (pow2) launch_pattn<DH, kDenseP2>(q, qrs, kv, kvb, kvn, kvh, B, N, H, scale, ws, out, osb, st);
+  else launch_pattn<DH, kDense>(q, qrs, kv, kvb, kvn, kvh, B, N, H, scale, ws, out, osb, st);
 }
 
 }  // namespace oudjat
@@ -564,16 +572,17 @@ extern "C" int oudjat_patch_attention_prob(const uint16_t* q, int64_t q_row_stri
   OUDJAT_REQUIRE(aligned(q, 16) && aligned(kv, 16) && q_row_stride % 8 == 0 && kv_stride_b % 8 == 0 &&
                      kv_stride_n % 8 == 0 && kv_stride_h % 8 == 0,
                  OUDJAT_ERR_UNSUPPORTED_LAYOUT, "patch_attention_prob: 16-byte aligned rows required");
-  OUDJAT_REQUIRE(N < (1 << 24) && H < 65536 && B < 65536, OUDJAT_ERR_TOO_LARGE, "patch_attention_prob: too large");
+  OUDJAT_REQUIRE(N < (1 << 24) && H < 65536 && B < 65536 && B * H * cdiv(N, 32 * kStWaves) < ((int64_t)1 << 31) &&
+                     (mode == kLse || B * cdiv(N, kDnTile) * cdiv(N, kDnTile) < ((int64_t)1 << 31)),
+                 OUDJAT_ERR_TOO_LARGE, "patch_attention_prob: too large");
   const hipStream_t st = as_stream(stream);
   const int b = (int)B, n = (int)N, h = (int)H;
-  if (Dh == 64) {
-    if (mode == kDense) launch_pattn<64, kDense>(q, q_row_stride, kv, kv_stride_b, kv_stride_n, kv_stride_h, b, n, h, scale, workspace, out, out_stride_b, st);
-    else launch_pattn<64, kLse>(q, q_row_stride, kv, kv_stride_b, kv_stride_n, kv_stride_h, b, n, h, scale, workspace, out, out_stride_b, st);
-  } else {
-    if (mode == kDense) launch_pattn<128, kDense>(q, q_row_stride, kv, kv_stride_b, kv_stride_n, kv_stride_h, b, n, h, scale, workspace, out, out_stride_b, st);
-    else launch_pattn<128, kLse>(q, q_row_stride, kv, kv_stride_b, kv_stride_n, kv_stride_h, b, n, h, scale, workspace, out, out_stride_b, st);
-  }
+  if (Dh == 64)
+    launch_pattn_mode<64>(q, q_row_stride, kv, kv_stride_b, kv_stride_n, kv_stride_h, b, n, h, scale, mode, workspace,
+                          out, out_stride_b, st);
+  else
+    launch_pattn_mode<128>(q, q_row_stride, kv, kv_stride_b, kv_stride_n, kv_stride_h, b, n, h, scale, mode, workspace,
+                           out, out_stride_b, st);
   return check_launch("patch_attention_prob");
 }
 

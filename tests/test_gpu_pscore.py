@@ -171,6 +171,31 @@ def test_patch_attention_prob_vs_oracle(dev, B, H, N, D, mode):
     assert u.max() <= 1.0 and float((u > 0).mean()) <= 0.02
 
 
+@pytest.mark.parametrize("B,H,N,D,scale,stride", [
+    (1, 2, 1, 64, 0.125, 0),          # one query, one key
+    (1, 3, 33, 64, 0.125, 0),         # a second wave with one query; keys of one lane half only in part
+    (9, 2, 129, 64, 0.1, 0),          # one row past a 128-tile, a scale that is no power of two, B % 8 != 0
+    (2, 4, 160, 128, 0.125, 0),       # the power-of-two form at Dh = 128; half a key block past the tile
+    (1, 2, 257, 128, 128 ** -0.5, 0),
+    (1, 2, 3, 64, 0.125, (1 << 24) + 8),  # query rows further apart than 32-bit tile offsets take
+])
+def test_dense_score_tile_edges(dev, B, H, N, D, scale, stride):
+    """The dense score where tiles, waves and lane halves end, in both forms of its scores (power-of-two
+    scale or not), against the exact evaluation: within one bf16 step (see above)."""
+    print(f"dense score edges B={B} H={H} N={N} D={D} scale={scale} stride={stride}", flush=True)
+    q, kv, qd, kvd = _qkv(B, H, N, D, 3 + N, dev)
+    qp = qd.reshape(B * N, H, D)
+    if stride:
+        wide = torch.empty_strided((B * N, H, D), (stride, D, 1), device=dev, dtype=qp.dtype)
+        wide.copy_(qp)
+        qp = wide
+    got = K.patch_attention_prob(qp, kvd, scale, K.PATTN_DENSE)
+    qh = np.ascontiguousarray(q.float().numpy().transpose(0, 2, 1, 3))
+    ref = torch.from_numpy(PS.patch_attn_prob(qh, kv[:, :, 0].float().numpy(), scale)).to(torch.bfloat16)
+    u = _bf16_ulps(got, ref)
+    assert u.max() <= 1.0 and float((u > 0).mean()) <= max(0.02, 2.0 / got.numel()), (u.max(), float((u > 0).mean()))
+
+
 def test_patch_attention_prob_vit7b_mass(dev):
     """ViT-7B at 1024 px (N = 4101 > 4096: the dense path even for the layer-mean kind): every query's
     probabilities sum to one, so the key scores of an image sum to one up to the bf16 roundings."""
