@@ -10,11 +10,8 @@
 //     fused QKV projection.
 //   * gemm_bf16_r16_kernel: 144- and 288-row tiles on 16x16x32 MFMAs with optional split K inside
 //     the workgroup; the N = C projections.
-//   * gemm_bf16_pipe_kernel: direct-to-LDS loads (global_load_lds, no staging registers), K tiles of
-//     32 in four LDS stages issued three tiles ahead, fragments read one K tile ahead of their
-//     MFMAs. 256 x 256 tiles with 8 waves; used when one round of tiles fills the GPU.
-//   * gemm_bf16_dma_kernel: direct-to-LDS loads, K tiles of 64, two stages. 128 x 128 tiles with 4
-//     waves, two workgroups per CU; used for the other grids.
+//   * gemm_bf16_dma_kernel: direct-to-LDS loads, K tiles of 64; 64- to 128-wide tiles with 4 waves,
+//     several workgroups per CU.
 //   * gemm_bf16_kernel: register-staged loads with 16-byte-aligned fallbacks (any N % 64 == 0, any
 //     output alignment).
 // Common to all:
@@ -653,12 +650,15 @@ __device__ __forceinline__ void load_gelu_table(unsigned char* dst) {
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
-// LDS bytes of the direct-to-LDS kernel before the GELU table: two K stages or the epilogue tile.
-__host__ __device__ constexpr int dma_lut_offset(int bm, int bn) {
-  return 2 * (bm + bn) * 128 > bm * (bn + 8) * 2 ? 2 * (bm + bn) * 128 : bm * (bn + 8) * 2;
-}
+// K stages: two, where the other workgroups of the CU cover a load's latency; four for the 128 x 32 tiles,
+// whose grids leave one workgroup or none per CU (the loads of three K tiles then overlap: ViT-S at
+// B = 1, 103 x 384 x 384, 5.8 -> 5.3 us).
+__host__ __device__ constexpr int dma_stages(int bn) { return bn == 32 ? 4 : 2; }
 
-__device__ __forceinline__ void wait_vm_all() { __builtin_amdgcn_s_waitcnt(0); }
+// LDS bytes of the direct-to-LDS kernel before the GELU table: the K stages or the epilogue tile.
+__host__ __device__ constexpr int dma_lut_offset(int bm, int bn) {
+  return dma_stages(bn) * (bm + bn) * 128 > bm * (bn + 8) * 2 ? dma_stages(bn) * (bm + bn) * 128 : bm * (bn + 8) * 2;
+}
 
 template <int BM, int BN, int WGM, int WGN, int EPI>
 __global__ __launch_bounds__(WGM * WGN * 64) void gemm_bf16_dma_kernel(const uint16_t* __restrict__ A, int M, int K,
@@ -735,12 +735,21 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_bf16_dma_kernel(const uin
   const int KT = K / kBK;
   const int frow = lane & 31;
   const int fchunk = lane >> 5;
-  issue(0, 0);
+  constexpr int NST = dma_stages(BN);
+  constexpr int NL = AG + BG;  // this wave's loads of a K tile
+#pragma unroll
+  for (int s = 0; s < NST - 1; ++s)
+    if (s < KT) issue(s, s);
   for (int kt = 0; kt < KT; ++kt) {
-    wait_vm_all();      // this wave's loads of step kt have landed
-    __syncthreads();    // ... and every wave's; every wave is also done reading step kt-1's stage
-    if (kt + 1 < KT) issue((kt + 1) & 1, kt + 1);
-    const unsigned char* a = smem + (kt & 1) * STAGE;
+    // This wave's loads of step kt have landed (at most NST - 2 later tiles are in flight), then every
+    // wave's; every wave is also done reading step kt - 1's stage, which is refilled.
+    const int ahead = min(NST - 2, KT - 1 - kt);
+    if (ahead <= 0) wait_vmcnt<0>();
+    else if (ahead == 1) wait_vmcnt<NL>();
+    else wait_vmcnt<2 * NL>();
+    block_barrier();
+    if (kt + NST - 1 < KT) issue((kt + NST - 1) % NST, kt + NST - 1);
+    const unsigned char* a = smem + (kt % NST) * STAGE;
     const unsigned char* b = a + BM * 128;
 #pragma unroll
     for (int ks = 0; ks < kBK / 16; ++ks) {
@@ -762,212 +771,6 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_bf16_dma_kernel(const uin
   __syncthreads();
   store_tile<BM, BN, FM, FN, NW, EPI>(acc, smem, reinterpret_cast<const uint16_t*>(smem + dma_lut_offset(BM, BN)), wm0,
                                       wn0, m0, n0, M, ea, C, ldc);
-}
-
-// ------------------------------------------------------------------------------------------------
-// Deep-pipelined direct-to-LDS kernel. K tiles of 32 (64-byte LDS rows), 4 LDS stages, operand
-// loads issued three K tiles ahead of the MFMAs that consume them, one workgroup per CU.
-//
-//   * Swizzle: chunk c of row r sits at 16-byte slot c ^ ((r >> 2) & 3). A wave reading one chunk
-//     of 16 consecutive rows (one quarter of a fragment read) then covers all 64 LDS banks once.
-//   * Loads: one global_load_lds_dwordx4 fills 16 consecutive 64-byte rows (lane l -> row l / 4,
-//     slot l % 4, i.e. global chunk (l % 4) ^ ((l / 16) % 4)). The (BM + BN) / 16 instructions of a
-//     K tile are dealt round-robin to the waves.
-//   * Per K tile: wait for this wave's loads of the tile (vmcnt), one s_barrier (every wave's loads
-//     landed, every wave done reading the stage about to be refilled), issue the loads of tile
-//     kt + 3 into that stage, then 2 x FM x FN MFMAs with all fragments read up front.
-// ------------------------------------------------------------------------------------------------
-
-static constexpr int kBK3 = 32;
-static constexpr int kStages = 4;
-
-__device__ __forceinline__ int swz64(int r, int c) { return r * 64 + ((c ^ ((r >> 2) & 3)) << 4); }
-
-__device__ __forceinline__ void wait_vmcnt_rt(int n) {
-  switch (n) {
-    case 0: wait_vmcnt<0>(); break;
-    case 1: wait_vmcnt<1>(); break;
-    case 2: wait_vmcnt<2>(); break;
-    case 3: wait_vmcnt<3>(); break;
-    case 4: wait_vmcnt<4>(); break;
-    case 5: wait_vmcnt<5>(); break;
-    case 6: wait_vmcnt<6>(); break;
-    case 7: wait_vmcnt<7>(); break;
-    case 8: wait_vmcnt<8>(); break;
-    case 9: wait_vmcnt<9>(); break;
-    case 10: wait_vmcnt<10>(); break;
-    case 11: wait_vmcnt<11>(); break;
-    case 12: wait_vmcnt<12>(); break;
-    case 13: wait_vmcnt<13>(); break;
-    case 14: wait_vmcnt<14>(); break;
-    case 15: wait_vmcnt<15>(); break;
-    case 16: wait_vmcnt<16>(); break;
-    case 17: wait_vmcnt<17>(); break;
-    case 18: wait_vmcnt<18>(); break;
-    case 19: wait_vmcnt<19>(); break;
-    case 20: wait_vmcnt<20>(); break;
-    case 21: wait_vmcnt<21>(); break;
-    case 22: wait_vmcnt<22>(); break;
-    case 23: wait_vmcnt<23>(); break;
-    default: wait_vmcnt<24>(); break;
-  }
-}
-
-// LDS bytes of the pipelined kernel before the GELU table: K stages or the epilogue tile.
-__host__ __device__ constexpr int pipe_lut_offset(int bm, int bn) {
-  return kStages * (bm + bn) * 64 > bm * (bn + 8) * 2 ? kStages * (bm + bn) * 64 : bm * (bn + 8) * 2;
-}
-
-template <int BM, int BN, int WGM, int WGN, int EPI>
-__global__ __launch_bounds__(WGM * WGN * 64) __attribute__((amdgpu_waves_per_eu(WGM * WGN / 4, WGM * WGN / 4)))
-void gemm_bf16_pipe_kernel(const uint16_t* __restrict__ A, int M, int K, int64_t lda, const uint16_t* __restrict__ W,
-                           int N, int64_t ldw, EpiArgs ea, uint16_t* __restrict__ C, int64_t ldc, int group_m) {
-  constexpr int NW = WGM * WGN;
-  constexpr int WM = BM / WGM, WN = BN / WGN;
-  constexpr int FM = WM / 32, FN = WN / 32;
-  constexpr int NI = (BM + BN) / 16;              // load instructions per K tile
-  constexpr int NLM = (NI + NW - 1) / NW;         // per wave, at most
-  constexpr int STAGE = (BM + BN) * 64;
-  static_assert(BM % 16 == 0 && BN % 16 == 0 && FM >= 1 && FN >= 1 && WM % 32 == 0 && WN % 32 == 0, "tile shape");
-
-  extern __shared__ __align__(16) unsigned char smem[];
-  // LDS: K stages (later the epilogue tile), then the GELU table for the GELU epilogue.
-  constexpr int kLutOff = pipe_lut_offset(BM, BN);
-  if constexpr (EPI == OUDJAT_EPI_BIAS_GELU) load_gelu_table<NW * 64>(smem + kLutOff);
-
-  const int tiles_n = (N + BN - 1) / BN;
-  const int tiles_m = (M + BM - 1) / BM;
-  const int tiles = gridDim.x;
-  const int bid = blockIdx.x;
-  const int xcd = bid % kNumXcd;
-  const int q = tiles / kNumXcd, r = tiles % kNumXcd;
-  const int tile = xcd * q + min(xcd, r) + bid / kNumXcd;
-  const int per_group = group_m * tiles_n;
-  const int grp = tile / per_group;
-  const int first_m = grp * group_m;
-  const int gsize = min(tiles_m - first_m, group_m);
-  const int in_grp = tile - grp * per_group;
-  const int tm = first_m + in_grp % gsize, tn = in_grp / gsize;
-  const int m0 = tm * BM, n0 = tn * BN;
-
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform, kept in SGPRs
-  const int wm0 = (wave / WGN) * WM;
-  const int wn0 = (wave % WGN) * WN;
-
-  // This wave's load instructions: i = wave + j * NW.
-  const int nl = (NI % NW == 0) ? NI / NW : (NI - wave + NW - 1) / NW;
-  const uint16_t* src[NLM];
-  int dst[NLM];
-  {
-    const int lrow = lane >> 2;
-    const int lchunk = (lane & 3) ^ ((lane >> 4) & 3);
-#pragma unroll
-    for (int j = 0; j < NLM; ++j) {
-      const int i = min(wave + j * NW, NI - 1);
-      dst[j] = i * 1024;
-      if (i < BM / 16) {
-        src[j] = A + (int64_t)min(m0 + i * 16 + lrow, M - 1) * lda + lchunk * 8;
-      } else {
-        src[j] = W + (int64_t)min(n0 + (i - BM / 16) * 16 + lrow, N - 1) * ldw + lchunk * 8;
-      }
-    }
-  }
-  const int KT = K / kBK3;
-  auto issue = [&](int stage, int kt) __attribute__((always_inline)) {
-    unsigned char* base = smem + stage * STAGE;
-    const int k0 = kt * kBK3;
-#pragma unroll
-    for (int j = 0; j < NLM; ++j)
-      if (j < nl)
-        __builtin_amdgcn_global_load_lds((const void*)(src[j] + k0), (lds_ptr_t)(base + dst[j]), 16, 0, 0);
-  };
-
-  f32x16_t acc[FM][FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-
-  // Fragment offsets: lane l reads row (l % 32) of each 32-row block at K chunk 2 * ks + l / 32.
-  const int sw = (lane >> 2) & 3;
-  const int a_lane = (wm0 + (lane & 31)) * 64;
-  const int b_lane = BM * 64 + (wn0 + (lane & 31)) * 64;
-  const int co0 = ((0 + (lane >> 5)) ^ sw) << 4;
-  const int co1 = ((2 + (lane >> 5)) ^ sw) << 4;
-
-  // Fragments of one K tile: [ks][block] for A and B, read one tile ahead of their MFMAs.
-  struct Frags {
-    bf16x8_t a[2][FM], b[2][FN];
-  };
-  auto read_frags = [&](Frags& f, int kt) __attribute__((always_inline)) {
-    const unsigned char* st = smem + (kt & (kStages - 1)) * STAGE;
-#pragma unroll
-    for (int i = 0; i < FM; ++i) f.a[0][i] = *reinterpret_cast<const bf16x8_t*>(st + a_lane + i * 2048 + co0);
-#pragma unroll
-    for (int j = 0; j < FN; ++j) f.b[0][j] = *reinterpret_cast<const bf16x8_t*>(st + b_lane + j * 2048 + co0);
-#pragma unroll
-    for (int i = 0; i < FM; ++i) f.a[1][i] = *reinterpret_cast<const bf16x8_t*>(st + a_lane + i * 2048 + co1);
-#pragma unroll
-    for (int j = 0; j < FN; ++j) f.b[1][j] = *reinterpret_cast<const bf16x8_t*>(st + b_lane + j * 2048 + co1);
-  };
-  // Row blocks at or past M (ragged last tile row) compute on clamped A rows and are never stored;
-  // a branch per row block would drain the prefetched fragments at every block boundary.
-  auto mfmas = [&](const Frags& f) __attribute__((always_inline)) {
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.b[ks][j], f.a[ks][i], acc[i][j], 0, 0, 0);
-  };
-  // Wait until at most `n_after` K tiles of this wave's loads are still in flight.
-  auto wait_tiles = [&](int n_after) __attribute__((always_inline)) {
-    if constexpr (NI % NW == 0) {
-      if (n_after >= 3) wait_vmcnt<3 * (NI / NW)>();
-      else if (n_after == 2) wait_vmcnt<2 * (NI / NW)>();
-      else if (n_after == 1) wait_vmcnt<NI / NW>();
-      else wait_vmcnt<0>();
-    } else {
-      wait_vmcnt_rt(n_after * nl);
-    }
-  };
-
-  // Pipeline: at the top of step kt the stages hold tiles kt+1 .. kt+3 (landed or in flight) and
-  // tile kt's fragments are already in registers, so tile kt's stage is free for tile kt+4.
-  //   wait for tile kt+1; barrier; issue tile kt+4; read tile kt+1's fragments; MFMAs of tile kt.
-#pragma unroll
-  for (int s = 0; s < kStages; ++s)
-    if (s < KT) issue(s, s);
-  wait_tiles(min(KT - 1, kStages - 1));
-  block_barrier();
-  Frags f0, f1;
-  read_frags(f0, 0);
-
-  auto step = [&](int kt, Frags& cur, Frags& nxt) __attribute__((always_inline)) {
-    if (kt + 1 < KT) {
-      wait_tiles(min(KT - 2 - kt, kStages - 2));
-      block_barrier();
-      if (kt + kStages < KT) issue(kt & (kStages - 1), kt + kStages);
-      __builtin_amdgcn_sched_barrier(0);
-      read_frags(nxt, kt + 1);
-    }
-    mfmas(cur);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  int kt = 0;
-  for (; kt + 1 < KT; kt += 2) {
-    step(kt, f0, f1);
-    step(kt + 1, f1, f0);
-  }
-  if (kt < KT) step(kt, f0, f1);
-
-  block_barrier();
-  store_tile<BM, BN, FM, FN, NW, EPI>(acc, smem, reinterpret_cast<const uint16_t*>(smem + kLutOff), wm0, wn0, m0, n0,
-                                      M, ea, C, ldc);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1142,9 +945,11 @@ __device__ __forceinline__ void r16_epilogue(f32x4_t (&acc)[FMB][FNB], unsigned 
 
 // FB: fragments read one K tile ahead (double-buffered registers); without it they are read right
 // after the barrier of their own K tile (for wave tiles whose accumulators leave no room).
+// Small tiles (up to 64 x 128) may share a CU (up to four waves a SIMD); the large ones keep all of its
+// registers.
 template <int BM, int BN, int WGM, int WGN, int KSPLIT, int BK, int NST, bool FB, int EPI>
 __global__ __launch_bounds__(WGM * WGN * KSPLIT * 64) __attribute__((amdgpu_waves_per_eu(
-    (WGM * WGN * KSPLIT + 3) / 4, (WGM * WGN * KSPLIT + 3) / 4)))
+    (WGM * WGN * KSPLIT + 3) / 4, BM * BN <= 64 * 128 ? 4 : (WGM * WGN * KSPLIT + 3) / 4)))
 void gemm_bf16_r16_kernel(const uint16_t* __restrict__ A, int M, int K, int64_t lda, const uint16_t* __restrict__ W,
                           int N, int64_t ldw, EpiArgs ea, uint16_t* __restrict__ C, int64_t ldc, int group_m) {
   using L = R16Layout<BK>;
@@ -1722,7 +1527,7 @@ typedef void (*gemm_fn)(const uint16_t*, int, int, int64_t, const uint16_t*, int
                         int64_t, int);
 
 struct GemmCfg {
-  int bm, bn, wgm, wgn, pf;  // pf: register prefetch depth; 0 = direct-to-LDS; -1 = pipelined; -2 = 16-row
+  int bm, bn, wgm, wgn, pf;  // pf: register prefetch depth; 0 = direct-to-LDS; -2 = 16-row; -3 / -4 = ping-pong
   gemm_fn fn[kNumEpi];       // by epilogue; fn[kEpiQkv] only for the direct-to-LDS families, fn[kEpiPartial]
                              // only for the 16-row-block family
   int bk, nst, ks;           // 16-row kernel: K tile depth, LDS stages, K groups
@@ -1740,12 +1545,6 @@ struct GemmCfg {
    {gemm_bf16_dma_kernel<BM, BN, WGM, WGN, 0>, gemm_bf16_dma_kernel<BM, BN, WGM, WGN, 1>,                 \
     gemm_bf16_dma_kernel<BM, BN, WGM, WGN, 2>, gemm_bf16_dma_kernel<BM, BN, WGM, WGN, 3>,                 \
     gemm_bf16_dma_kernel<BM, BN, WGM, WGN, 4>, gemm_bf16_dma_kernel<BM, BN, WGM, WGN, kEpiQkv>}}
-
-#define OUDJAT_GEMM_PIPE_CFG(BM, BN, WGM, WGN)                                                            \
-  {BM, BN, WGM, WGN, -1,                                                                                 \
-   {gemm_bf16_pipe_kernel<BM, BN, WGM, WGN, 0>, gemm_bf16_pipe_kernel<BM, BN, WGM, WGN, 1>,               \
-    gemm_bf16_pipe_kernel<BM, BN, WGM, WGN, 2>, gemm_bf16_pipe_kernel<BM, BN, WGM, WGN, 3>,               \
-    gemm_bf16_pipe_kernel<BM, BN, WGM, WGN, 4>, gemm_bf16_pipe_kernel<BM, BN, WGM, WGN, kEpiQkv>}}
 
 // pf = -2: 16-row-block kernel; wgm x wgn waves per K group, ks K groups.
 #define OUDJAT_GEMM_R16_CFG(BM, BN, WGM, WGN, KS, BK, NST, FB)                                            \
@@ -1776,49 +1575,49 @@ struct GemmCfg {
     gemm_bf16_pp_kernel<BM, BN, kEpiQkv, true>, nullptr},                                                 \
    64, 2, 1, 0}
 
+// The launch configurations, in the order of kCfgs.
+enum GemmTile {
+  kReg128x64,      // register-staged: any output alignment
+  kDma128x128,     // direct-to-LDS, two stages
+  kDma128x64,
+  kDma64x64,
+  kDma128x32,      // four stages: tiny grids with K < 1024
+  kR32x64,         // 16-row blocks, two K groups, 128-deep K tiles
+  kR64x64,
+  kR64x64Deep,     // three stages
+  kR96x64,
+  kR64x128,        // 64-deep K tiles, four stages
+  kR144x128,       // the N = C products of the ViT-L pass
+  kR128x256,       // long-K products of about one round of 128 x 256
+  kPp288x256, kPp288x192, kPp224x256, kPp192x256, kPp224x384,            // ping-pong, bf16
+  kPp8_288x256, kPp8_224x256, kPp8_192x256, kPp8_128x256,                // ping-pong, e4m3 operands
+};
+
 static const GemmCfg kCfgs[] = {
-    OUDJAT_GEMM_CFG(128, 128, 2, 2, 1),  // 0
-    OUDJAT_GEMM_CFG(128, 128, 2, 2, 2),  // 1
-    OUDJAT_GEMM_CFG(256, 128, 2, 2, 1),  // 2
-    OUDJAT_GEMM_CFG(256, 128, 2, 2, 2),  // 3
-    OUDJAT_GEMM_CFG(128, 256, 2, 2, 2),  // 4
-    OUDJAT_GEMM_CFG(256, 256, 2, 4, 2),  // 5
-    OUDJAT_GEMM_CFG(256, 128, 4, 2, 2),  // 6
-    OUDJAT_GEMM_CFG(128, 128, 2, 2, 2),  // 7 (placeholder slot)
-    OUDJAT_GEMM_CFG(128, 64, 2, 2, 2),   // 8 (N % 128 != 0)
-    OUDJAT_GEMM_DMA_CFG(256, 256, 2, 2),  // 9
-    OUDJAT_GEMM_DMA_CFG(256, 128, 2, 2),  // 10
-    OUDJAT_GEMM_DMA_CFG(128, 128, 2, 2),  // 11
-    OUDJAT_GEMM_DMA_CFG(128, 256, 2, 2),  // 12
-    OUDJAT_GEMM_DMA_CFG(256, 256, 4, 2),  // 13
-    OUDJAT_GEMM_DMA_CFG(256, 256, 2, 4),  // 14
-    OUDJAT_GEMM_PIPE_CFG(256, 256, 2, 4),  // 15
-    OUDJAT_GEMM_PIPE_CFG(256, 256, 2, 2),  // 16
-    OUDJAT_GEMM_PIPE_CFG(288, 256, 3, 4),  // 17
-    OUDJAT_GEMM_PIPE_CFG(256, 128, 2, 2),  // 18
-    OUDJAT_GEMM_PIPE_CFG(128, 128, 2, 2),  // 19
-    OUDJAT_GEMM_R16_CFG(144, 512, 1, 4, 1, 32, 3, true),   // 20
-    OUDJAT_GEMM_R16_CFG(144, 128, 1, 2, 2, 64, 4, true),   // 21
-    OUDJAT_GEMM_R16_CFG(144, 512, 1, 8, 1, 32, 3, false),  // 22: fc1-like (N % 512 == 0)
-    OUDJAT_GEMM_R16_CFG(144, 128, 1, 4, 2, 64, 4, true),   // 23: N = C GEMMs
-    OUDJAT_GEMM_R16_CFG(144, 128, 1, 4, 2, 64, 3, true),   // 24
-    OUDJAT_GEMM_R16_CFG(288, 256, 2, 4, 1, 64, 2, false),  // 25: 288 x 256, 128-byte operand rows
-    OUDJAT_GEMM_R16_CFG(288, 192, 2, 4, 1, 64, 2, false),  // 26: 288 x 192 (N = 3 C: 240 tiles)
-    OUDJAT_GEMM_PP_CFG(288, 256),  // 27: ping-pong 288 x 256
-    OUDJAT_GEMM_PP_CFG(288, 192),  // 28: ping-pong 288 x 192
-    OUDJAT_GEMM_R16_CFG(144, 128, 1, 4, 2, 128, 2, false),  // 29: N = C GEMMs with K % 128 == 0
-    OUDJAT_GEMM_PP_CFG(224, 256),  // 30: ping-pong 224 x 256 (a full round where 288 rows leave CUs idle)
-    OUDJAT_GEMM_PP_CFG(192, 256),  // 31: ping-pong 192 x 256 (two rounds or a little less)
-    OUDJAT_GEMM_DMA_CFG(128, 32, 4, 1),  // 32: tiny grids (128 x 32, four waves of 32 x 32)
-    OUDJAT_GEMM_DMA_CFG(128, 64, 2, 2),  // 33: tiny fused-QKV grids (whole 64-wide heads)
-    OUDJAT_GEMM_R16_CFG(128, 256, 2, 4, 1, 64, 3, false),  // 34: long-K products of ~one round of 128 x 256
-    OUDJAT_GEMM_PP8_CFG(288, 256),  // 35: FP8 ping-pong tiles
-    OUDJAT_GEMM_PP8_CFG(224, 256),  // 36
-    OUDJAT_GEMM_PP8_CFG(192, 256),  // 37
-    OUDJAT_GEMM_PP8_CFG(128, 256),  // 38
-    OUDJAT_GEMM_PP_CFG(224, 384),  // 39: ping-pong 224 x 384 (one round where 256-wide tiles need two)
+    OUDJAT_GEMM_CFG(128, 64, 2, 2, 2),
+    OUDJAT_GEMM_DMA_CFG(128, 128, 2, 2),
+    OUDJAT_GEMM_DMA_CFG(128, 64, 2, 2),
+    OUDJAT_GEMM_DMA_CFG(64, 64, 2, 2),
+    OUDJAT_GEMM_DMA_CFG(128, 32, 4, 1),
+    OUDJAT_GEMM_R16_CFG(32, 64, 1, 4, 2, 128, 2, false),
+    OUDJAT_GEMM_R16_CFG(64, 64, 1, 4, 2, 128, 2, false),
+    OUDJAT_GEMM_R16_CFG(64, 64, 1, 4, 2, 128, 3, false),
+    OUDJAT_GEMM_R16_CFG(96, 64, 1, 4, 2, 128, 2, false),
+    OUDJAT_GEMM_R16_CFG(64, 128, 1, 4, 2, 64, 4, true),
+    OUDJAT_GEMM_R16_CFG(144, 128, 1, 4, 2, 128, 2, false),
+    OUDJAT_GEMM_R16_CFG(128, 256, 2, 4, 1, 64, 3, false),
+    OUDJAT_GEMM_PP_CFG(288, 256),
+    OUDJAT_GEMM_PP_CFG(288, 192),
+    OUDJAT_GEMM_PP_CFG(224, 256),
+    OUDJAT_GEMM_PP_CFG(192, 256),
+    OUDJAT_GEMM_PP_CFG(224, 384),
+    OUDJAT_GEMM_PP8_CFG(288, 256),
+    OUDJAT_GEMM_PP8_CFG(224, 256),
+    OUDJAT_GEMM_PP8_CFG(192, 256),
+    OUDJAT_GEMM_PP8_CFG(128, 256),
 };
 static constexpr int kNumCfgs = sizeof(kCfgs) / sizeof(kCfgs[0]);
+static_assert(kNumCfgs == kPp8_128x256 + 1, "one entry per GemmTile");
 
 // Host side of the GELU table: entry s * kGeluSpan + d holds bf16(gelu(v)) for the bf16 input v
 // with sign s and magnitude bits kGeluLo + d, computed as 0.5 v erfc(-v / sqrt 2) in double,
@@ -1858,27 +1657,16 @@ static int ensure_gelu_table() {
 // Rows of output tiles each XCD sweeps before moving to the next tile column (L2 reuse of the W panel).
 constexpr int kGroupM = 8;
 
-// A grid of at most 32 tiles of 128 x 128 (ViT-S at B = 1: 103 selected rows) leaves most CUs idle
-// and each workgroup streams its whole K alone: 128 x 32 tiles give four times the workgroups at 5/8
-// of the operand bytes each. Measured in the ViT-S pass (kernel trace, 128 x 128 -> 128 x 32): proj
-// 384 x 384 10.5 -> 7.4 us, fc1 1536 x 384 10.0 -> 7.1 us. Long-K tiny products still split K when
-// given a workspace (choose_splitk: ViT-S fc2, K = 1536, 13.4 us in 12 slices against 15.0 us for
-// unsplit 128 x 32 tiles, whose weights then stream from HBM).
+// A grid of at most 32 tiles of 128 x 128 (ViT-S at B = 1: 103 selected rows) leaves most CUs idle. With
+// K < 1024 it runs on 128 x 32 tiles (103 x 384 x 384: 5.3 us with the weights from HBM, 8.9 on 128 x 128);
+// with a longer K it is one more small product below.
 static bool tiny_grid(int64_t M, int64_t N) { return N % 32 == 0 && cdiv(M, 128) * cdiv(N, 128) <= 32; }
 
-// aligned_io: C, resid 16-byte aligned with ldc, ldr % 8 == 0 and bias 8-byte aligned, which the
-// vector epilogues need; otherwise the register-staged kernel with 2-byte stores runs.
-static int choose_cfg(int64_t M, int64_t N, int64_t K, bool aligned_io) {
-  if (!aligned_io) return 8;
-  if (tiny_grid(M, N)) return 32;
-  // 256 x 256 pipelined tiles when their grid fills between half and all of the CUs in one round;
-  // 128 x 128 direct-to-LDS tiles otherwise (two workgroups per CU balance a ragged second round
-  // better); the register-staged kernel for N % 128 != 0.
-  if (N % 128 != 0) return 8;
+// Ping-pong and wide tiles of the grids that fill about one or two rounds of them, or many (-1: none; the
+// small tiles below take those products). N % 128 == 0.
+static int choose_large(int64_t M, int64_t N, int64_t K) {
   // 288 x 256 / 288 x 192 (ping-pong) tiles with 128-byte operand rows when they fill three quarters
-  // or more of the CUs in one round: ahead of the 256 x 256 pipelined tiles, which they beat at every
-  // such shape measured (ViT-7B w1 1656 x 8192 x 4096: 94 against 111 us; a plain 4176 x 3072 x 1024
-  // product: 28.5 against 33.3 us).
+  // or more of the CUs in one round.
   const int64_t tiles288 = cdiv(M, 288) * (N / 256);
   // 224 x 256 ping-pong tiles when they fill at least seven eighths of one round that 288 x 256 tiles
   // fill less (ViT-7B w1 / w2, 1656 x 8192 x 4096: 256 against 192 tiles, 92.7 against 103.4 us).
@@ -1886,26 +1674,26 @@ static int choose_cfg(int64_t M, int64_t N, int64_t K, bool aligned_io) {
   // Beyond two rounds of 288 x 256 tiles (the approximate pass, every token of the batch: M = B N)
   // those tiles in as many rounds as it takes, in place of 128 x 128 tiles (ViT-L approximate pass
   // 18.1 -> 16.5 ms, ViT-7B 337.7 -> 256.5 ms; 224 x 256 and 192 x 256 tiles came between).
-  if (N % 256 == 0 && tiles288 > 512) return 27;
-  if (N % 256 == 0 && tiles224 >= 224 && tiles224 <= 256 && tiles288 < tiles224) return 30;
-  if (N % 256 == 0 && tiles288 >= 192 && tiles288 <= 256) return 27;
+  if (N % 256 == 0 && tiles288 > 512) return kPp288x256;
+  if (N % 256 == 0 && tiles224 >= 224 && tiles224 <= 256 && tiles288 < tiles224) return kPp224x256;
+  if (N % 256 == 0 && tiles288 >= 192 && tiles288 <= 256) return kPp288x256;
   // One round of 224 x 384 ping-pong tiles where the 256-wide ones need more than one (ViT-7B qkv,
   // 1656 x 12288 x 4096: 256 tiles, 135.1 us, against 170.4 for 432 tiles of 192 x 256 in two uneven
   // rounds and 147.2 for hipBLASLt; 22 % fewer operand bytes per FLOP than 192 x 256).
   const int64_t tiles384 = cdiv(M, 224) * (N / 384);
-  if (N % 384 == 0 && tiles384 >= 224 && tiles384 <= 256) return 39;
+  if (N % 384 == 0 && tiles384 >= 224 && tiles384 <= 256) return kPp224x384;
   // Two rounds of 288-, 224- or 192-row ping-pong tiles 256 wide, whichever fills them most (ViT-L
   // keep 50 %, M = 8272: fc1 4096 wide, 464 tiles of 288 x 256, 62.7 us; qkv 3072 wide, 444 tiles of
   // 224 x 256, 53.7 us, where 128 x 128 tiles took 85.0 and 73.3 us; ViT-7B qkv, 1656 x 12288 x 4096:
   // 432 tiles of 192 x 256, 162.6 us, against 177.9 for a round and a half of 288 x 192 tiles and
   // 185.4 for 128 x 128 tiles; 192 x 256 also takes whole heads of Dh = 128 for the fused QKV
   // epilogue, which 192-wide tiles do not).
+  const int64_t tiles192 = cdiv(M, 192) * (N / 256);
   if (N % 256 == 0) {
-    const int64_t tiles192 = cdiv(M, 192) * (N / 256);
     int best = -1;
     int64_t best_tiles = 0;
     const int64_t cand_tiles[3] = {tiles288, tiles224, tiles192};
-    const int cand_cfg[3] = {27, 30, 31};
+    const int cand_cfg[3] = {kPp288x256, kPp224x256, kPp192x256};
     for (int c = 0; c < 3; ++c)
       if (cand_tiles[c] > 256 && cand_tiles[c] <= 512 && cand_tiles[c] > best_tiles) {
         best = cand_cfg[c];
@@ -1914,94 +1702,166 @@ static int choose_cfg(int64_t M, int64_t N, int64_t K, bool aligned_io) {
     if (best >= 0 && best_tiles > 384) return best;
   }
   const int64_t tiles288n = cdiv(M, 288) * (N / 192);
-  if (N % 192 == 0 && tiles288n >= 192 && tiles288n <= 256) return 28;
-  // Half a round or more of 256 x 256 tiles: 192 x 256 or 224 x 256 ping-pong tiles if they still fit
-  // one round (ViT-L keep 50 %, 8272 x 1024: 176 tiles of 192 x 256, proj 28.7 us and fc2 77.8 us,
-  // against 30.6 / 82.3 for 224 x 256 and 34.9 / 101.4 for the 132 pipelined 256 x 256 tiles), else
-  // those.
+  if (N % 192 == 0 && tiles288n >= 192 && tiles288n <= 256) return kPp288x192;
+  // Half a round or more of 256 x 256: 192 x 256 ping-pong tiles if they still fit one round, else
+  // 224 x 256 (ViT-L keep 50 %, 8272 x 1024: 176 tiles of 192 x 256, proj 28.7 us and fc2 77.8 us,
+  // against 30.6 / 82.3 for 224 x 256).
   const int64_t tiles256 = cdiv(M, 256) * cdiv(N, 256);
-  if (N % 256 == 0 && tiles256 >= 128 && tiles256 <= 256)
-    return cdiv(M, 192) * (N / 256) <= 256 ? 31 : (tiles224 <= 256 ? 30 : 15);
-  // 144-row tiles (one round of 128..256 workgroups) when 256 x 256 tiles do not fit one round.
-  const int64_t tm144 = cdiv(M, 144);
-  if (N % 512 == 0 && tm144 * (N / 512) >= 128 && tm144 * (N / 512) <= 256) return 22;
-  // 128-deep K tiles (half the barriers and load batches of the 64-deep ones; the two K groups still
-  // take alternate 32-deep steps, so the result is the same bit for bit) when K allows.
-  if (tm144 * (N / 128) >= 128 && tm144 * (N / 128) <= 256) return K % 128 == 0 ? 29 : 23;
-  // A short-K product of a quarter to a half round of 144 x 128 tiles runs best on 128 x 32 tiles,
-  // four to five workgroups per CU (ViT-L keep 10 % proj, 1712 x 1024 x 1024: 16.1 -> 15.1 us; ViT-B
-  // proj, 2088 x 768 x 768: 13.5 -> 12.5 us; weights from HBM, HIP graph). 128 x 128 tiles: 20.3 and
-  // 16.6 us; at a full round and more (the headline proj, 4176 rows) 128 x 32 tiles lose (27.6 against
-  // 17.6 us).
-  if (K <= 1024 && tm144 * (N / 128) >= 64 && tm144 * (N / 128) < 128) return 32;
-  // A round and a half of 288 x 192 tiles still beats 128 x 128 tiles.
-  if (N % 192 == 0 && tiles288n > 256 && tiles288n <= 400) return 28;
+  if (N % 256 == 0 && tiles256 >= 128 && tiles256 <= 256) return tiles192 <= 256 ? kPp192x256 : kPp224x256;
   // A long-K product whose 128 x 256 grid fills three quarters to all of one round (ViT-7B proj,
   // 1656 x 4096 x 4096: 208 tiles): 16-row-block 128 x 256 tiles, 8 waves of 64 x 64, three 64-deep
   // stages, in place of two rounds of 128 x 128 tiles (77.6 -> 70.8 us with the weights from HBM).
   const int64_t tiles128w = cdiv(M, 128) * (N / 256);
-  if (K >= 2048 && N % 256 == 0 && tiles128w >= 192 && tiles128w <= 256) return 34;
-  return 11;
+  if (K >= 2048 && N % 256 == 0 && tiles128w >= 192 && tiles128w <= 256) return kR128x256;
+  return -1;
 }
 
+// Products that fill less than a round of large tiles. What bounds them is how long the busiest CU streams
+// its operands (a CU pulls 40-60 KB/us whatever the tile) over a fixed cost per launch, so the tile is the
+// one whose time comes out least in
+//     us = fix[n] + (per_k[n] + fill[n] * (w / 256 - (n - 1))) * depth,   n = ceil(w / 256) rounds,
+// w = workgroups (output tiles x K slices), depth = K / slices. The figures are fits over 24 row counts
+// (64 .. 16464) x the 16 layer shapes of the four backbones (weights from HBM, activations cached), 3-9 %
+// off the single measurement; several workgroups share a CU where their LDS allows, hence one row per n.
+// Over those 384 products the choice is 1.19x faster in the geometric mean than the earlier rule (128 x 128
+// tiles for most of them) and 4 % off the fastest tile measured for each: 1152 x 768 x 3072 35.6 -> 14.7 us,
+// 800 x 768 x 768 12.0 -> 6.9, 224 x 3072 x 1024 14.3 -> 8.1, 400 x 4096 x 4096 32.4 -> 28.9.
+struct SmallTile {
+  int ci, max_n;
+  float fix[4], per_k[4], fill[4];
+};
+static const SmallTile kSmallTiles[] = {
+    {kDma128x128, 4, {4.74f, 8.02f, 10.22f, 12.78f}, {.00969f, .01331f, .02268f, .02784f}, {.00292f, .00243f, .00411f, .00256f}},
+    {kDma128x64, 4, {3.28f, 3.83f, 5.33f, 6.39f}, {.00832f, .00977f, .01315f, .02070f}, {.00222f, .00209f, .00162f, .00287f}},
+    {kDma64x64, 4, {2.79f, 2.79f, 2.93f, 3.94f}, {.00724f, .00824f, .00930f, .01135f}, {.00124f, .00134f, .00115f, .00185f}},
+    {kR32x64, 4, {2.96f, 3.87f, 4.44f, 5.14f}, {.00396f, .00439f, .00838f, .00927f}, {.00057f, .00061f, .00114f, .00159f}},
+    {kR64x64, 4, {3.26f, 4.29f, 5.29f, 6.32f}, {.00443f, .00515f, .01042f, .01076f}, {.00115f, .00178f, .00185f, .00300f}},
+    {kR64x64Deep, 2, {3.85f, 5.97f}, {.00318f, .00674f}, {.00063f, .00099f}},
+    {kR96x64, 3, {3.81f, 5.63f, 7.01f}, {.00467f, .00602f, .01181f}, {.00181f, .00215f, .00200f}},
+    {kR64x128, 2, {4.88f, 8.38f}, {.00489f, .01047f}, {.00148f, .00152f}},
+    {kR144x128, 2, {6.38f, 12.70f}, {.00694f, .01565f}, {.00410f, .00394f}},
+    {kR128x256, 2, {7.97f, 15.95f}, {.01177f, .02519f}, {.00570f, .00591f}},
+};
 
-// Split K when the output tiles leave most CUs idle: S K-slices side by side (S * tiles <= 256
-// workgroups, one round), each a whole number of K tiles. Candidates: the 144 x 128 16-row-block
-// tiles with slices at least 1024 deep, and the 288 x 256 ping-pong tiles with slices at least 4096
-// deep (measured: ViT-7B w3, 1656 x 4096 x 8192, 138 -> 128 us; with 1024- or 2048-deep slices the
-// partial stores and the reduce cost more than the halved operand stream saves: ViT-L fc2 49 ->
-// 68 us, ViT-7B proj 78 -> 90 us). Among those whose split fills at least 160 CUs, the one that
-// streams the fewest operand bytes per workgroup. Returns the configuration and S (-1 / S = 1: no
-// split). Every public epilogue: their tile forms are epilogue<EPI> element by element.
+// The modelled time of an M x N x K product in S slices on tile t (negative: it does not take the shape).
+static float small_tile_us(const SmallTile& t, int64_t M, int64_t N, int64_t K, int64_t S) {
+  const GemmCfg& c = kCfgs[t.ci];
+  const int64_t bk = c.pf == -2 ? c.bk : kBK;
+  if (N % c.bn != 0 || K % (S * bk) != 0 || (S > 1 && K / S < 2 * bk)) return -1.0f;
+  // 64-row tiles of a weight that no cache holds re-read it from HBM for every tile row (224 x 12288 x
+  // 4096: 54 us on 64 x 64 tiles, 46 on 144 x 128).
+  if (t.ci == kDma64x64 && N * K > ((int64_t)32 << 20)) return -1.0f;
+  const int64_t w = cdiv(M, c.bm) * (N / c.bn) * S, n = cdiv(w, kNumCus);
+  const float depth = (float)(K / S);
+  if (n > t.max_n)  // 128 x 128 tiles (128 x 64 where those do not divide N) take any number of rounds
+    return t.ci == kDma128x128 || (t.ci == kDma128x64 && N % 128 != 0)
+               ? (t.fix[3] + (t.per_k[3] + 0.5f * t.fill[3]) * depth) * (float)n / 4.0f
+               : -1.0f;
+  return t.fix[n - 1] + (t.per_k[n - 1] + t.fill[n - 1] * ((float)w / kNumCus - (float)(n - 1))) * depth;
+}
+
+// The fastest small tile; head_dim > 0 (the fused QKV): of those that cover whole heads.
+static int choose_small(int64_t M, int64_t N, int64_t K, int64_t head_dim, float* us_out = nullptr) {
+  int best = -1;
+  float best_us = 0.0f;
+  for (const SmallTile& t : kSmallTiles) {
+    if (head_dim > 0 && kCfgs[t.ci].bn % head_dim != 0) continue;
+    const float us = small_tile_us(t, M, N, K, 1);
+    if (us >= 0.0f && (best < 0 || us < best_us)) {
+      best = t.ci;
+      best_us = us;
+    }
+  }
+  if (us_out) *us_out = best_us;
+  return best < 0 ? kReg128x64 : best;
+}
+
+// Operands of 4 GiB and more are out of reach of the 32-bit buffer offsets of the 16-row and ping-pong
+// kernels: those products run on the direct-to-LDS tiles, which take 64-bit addresses.
+static bool far_operands(int64_t M, int64_t lda, int64_t N, int64_t ldw) {
+  const int64_t limit = (int64_t)1 << 32;
+  return M * lda * 2 >= limit || N * ldw * 2 >= limit;
+}
+static int far_cfg(int64_t N) { return N % 128 == 0 ? kDma128x128 : kDma128x64; }
+
+// aligned_io: C, resid 16-byte aligned with ldc, ldr % 8 == 0 and bias 8-byte aligned, which the
+// vector epilogues need; otherwise the register-staged kernel with 2-byte stores runs.
+static int choose_cfg(int64_t M, int64_t N, int64_t K, bool aligned_io) {
+  if (!aligned_io) return kReg128x64;
+  if (tiny_grid(M, N) && K < 1024) return kDma128x32;
+  const int large = N % 128 == 0 ? choose_large(M, N, K) : -1;
+  return large >= 0 ? large : choose_small(M, N, K, 0);
+}
+
+// Split K when the output tiles leave most CUs idle: S K-slices side by side, each a whole number of K
+// tiles, whose fp32 partial tiles a second launch sums in order (or the packed residual step, which then
+// reads them in place of the product). Every public epilogue: their tile forms are epilogue<EPI> element
+// by element. The slices' reduce costs 3 us and 0.13 us per megabyte of partials. Returns the
+// configuration and S (-1 / S = 1: no split); the choice does not depend on the epilogue.
+//   * 288 x 256 ping-pong tiles in slices at least 4096 deep (ViT-7B w3, 1656 x 4096 x 8192: 138 -> 128 us;
+//     with shallower slices the partial stores and the reduce cost more than the halved operand stream
+//     saves: ViT-L fc2 49 -> 68 us, ViT-7B proj 78 -> 90 us);
+//   * K in two to four slices at least 1024 deep of a product of 33 to 127 tiles of 144 x 128 (the fc2 of
+//     ViT-B, and of ViT-L at keep 10 %, whose reduce runs in the residual step), on the tile and slice count
+//     of least modelled time;
+//   * any other product with K >= 1024 whose split is modelled faster than its one launch (ViT-S at B = 1
+//     fc2, 103 x 384 x 1536: 13.5 us in 12 slices of 144 x 128 tiles, 8.6 in 6 of 32 x 64).
 static int choose_splitk(int64_t M, int64_t N, int64_t K, int epi, int* S_out) {
   *S_out = 1;
   if (N % 128 != 0 || epi >= kEpiQkv) return -1;
-  struct Cand { int ci, bm, bn, bk, min_slice; };
-  const Cand cands[] = {{29, 144, 128, 128, 1024}, {23, 144, 128, 64, 1024}, {27, 288, 256, 64, 4096}};
+  const int64_t t288 = N % 256 == 0 ? cdiv(M, 288) * (N / 256) : 0;
+  const int64_t t144 = cdiv(M, 144) * (N / 128);
+  int deep = 1, mid = 1;  // the slice counts the first two rules find
+  for (int S = 4; S >= 2; --S) {
+    if (deep == 1 && t288 > 0 && t288 < 128 && S * t288 <= kNumCus && S * t288 >= 160 && K % (S * 64) == 0 &&
+        K / S >= 4096)
+      deep = S;
+    if (mid == 1 && t144 > 32 && t144 < 128 && S * t144 <= kNumCus && S * t144 >= 160 && K % (S * 64) == 0 &&
+        K / S >= 1024)
+      mid = S;
+  }
+  if (deep > 1 && (mid == 1 || (288 + 256) * (K / deep) < (144 + 128) * (K / mid))) {
+    *S_out = deep;
+    return kPp288x256;
+  }
+  if (mid == 1 && (K < 1024 || choose_large(M, N, K) >= 0)) return -1;
   int best = -1, best_s = 1;
-  int64_t best_bytes = 0;
-  for (const Cand& c : cands) {
-    if (N % c.bn != 0) continue;
-    const int64_t tiles = cdiv(M, c.bm) * (N / c.bn);
-    if (tiles >= 128) continue;  // fills the GPU without a split
-    // A product of a few dozen 144 x 128 tiles at most with a long K loop (ViT-S at B = 1, fc2: 103
-    // rows, 3 tiles, K = 1536) splits deep, down to two K tiles per slice, on those tiles: its partial
-    // tiles are a few megabytes at most, while unsplit each workgroup would stream all of K alone on
-    // an idle GPU (16.2 against 23.5 us in 12 slices). With K < 1024 the second launch costs more
-    // than the split saves (ViT-S proj and fc1, K = 384: 13.7 -> 15.2 and 12.5 -> 14.5 us in 3).
-    const bool tiny = c.bm == 144 && tiles <= 32 && K >= 1024;
-    const int s_max = tiny ? 16 : 4;
-    const int64_t min_slice = tiny ? 2 * c.bk : c.min_slice;
-    const int64_t min_wgs = tiny ? 2 * tiles : 160;
-    for (int S = (int)std::min<int64_t>(s_max, 256 / std::max<int64_t>(tiles, 1)); S >= 2; --S) {
-      if (K % ((int64_t)S * c.bk) != 0 || K / S < min_slice || S * tiles < min_wgs) continue;
-      const int64_t bytes = (int64_t)(c.bm + c.bn) * (K / S);
-      if (best < 0 || bytes < best_bytes) {
-        best = c.ci;
+  float best_us = 0.0f;
+  for (const SmallTile& t : kSmallTiles) {
+    if (kCfgs[t.ci].fn[kEpiPartial] == nullptr) continue;
+    for (int S = 2; S <= 16; ++S) {
+      const float us = small_tile_us(t, M, N, K, S);
+      if (us < 0.0f) continue;
+      const float all = us + 3.0f + 0.13f * ((float)S * M * N * 4.0f * 1e-6f);
+      if (best < 0 || all < best_us) {
+        best = t.ci;
         best_s = S;
-        best_bytes = bytes;
+        best_us = all;
       }
-      break;
     }
   }
-  *S_out = best_s;
+  float one_us = 0.0f;
+  if (best >= 0 && mid == 1) {
+    choose_small(M, N, K, 0, &one_us);
+    if (best_us > 0.97f * one_us) best = -1;
+  }
+  if (best >= 0) *S_out = best_s;
   return best;
 }
 
 // Fused QKV: tiles must cover whole heads (Dh | BN; a tile may span the q / k / v boundaries).
 // 288 x 192 (ping-pong) tiles when the plain choice would leave more CUs idle in its single round.
 static int choose_qkv_cfg(int64_t M, int64_t N, int64_t K, int64_t Dh) {
-  if (tiny_grid(M, N) && 64 % Dh == 0 && N % 64 == 0) return 33;  // ViT-S at B = 1: 10.5 -> 8.2 us
   // One round of whole-head 224 x 384 tiles (ViT-7B: 179.6 -> 140.3 us per fused QKV in the pass).
   const int64_t t384 = cdiv(M, 224) * (N / 384);
-  if (N % 384 == 0 && 384 % Dh == 0 && t384 >= 224 && t384 <= 256) return 39;
-  int ci = choose_cfg(M, N, K, true);
+  if (N % 384 == 0 && 384 % Dh == 0 && t384 >= 224 && t384 <= 256) return kPp224x384;
+  int ci = choose_large(M, N, K);
   const int64_t tiles288n = cdiv(M, 288) * (N / 192);
-  if (N % 192 == 0 && tiles288n >= 192 && tiles288n <= 256 &&
+  if (ci >= 0 && N % 192 == 0 && tiles288n >= 192 && tiles288n <= 256 &&
       cdiv(M, kCfgs[ci].bm) * cdiv(N, kCfgs[ci].bn) < tiles288n)
-    ci = 28;
-  if (kCfgs[ci].pf > 0 || kCfgs[ci].bn % Dh != 0 || N % kCfgs[ci].bn != 0) ci = 11;  // 128 x 128 direct-to-LDS
-  return ci;
+    ci = kPp288x192;
+  if (ci >= 0 && kCfgs[ci].bn % Dh == 0 && N % kCfgs[ci].bn == 0) return ci;
+  return choose_small(M, N, K, Dh);
 }
 
 // FP8 products (e4m3 operands: half the operand bytes per K of bf16) on the FP8 ping-pong tiles, chosen
@@ -2011,20 +1871,20 @@ static int choose_qkv_cfg(int64_t M, int64_t N, int64_t K, int64_t Dh) {
 static int choose_cfg_fp8(int64_t M, int64_t N) {
   const int64_t t288 = cdiv(M, 288) * (N / 256), t224 = cdiv(M, 224) * (N / 256);
   const int64_t t192 = cdiv(M, 192) * (N / 256);
-  if (t224 >= 224 && t224 <= 256 && t288 < t224) return 36;
-  if (t288 >= 192 && t288 <= 256) return 35;
+  if (t224 >= 224 && t224 <= 256 && t288 < t224) return kPp8_224x256;
+  if (t288 >= 192 && t288 <= 256) return kPp8_288x256;
   int best = -1;
   int64_t best_tiles = 0;
   const int64_t cand_tiles[3] = {t288, t224, t192};
-  const int cand_cfg[3] = {35, 36, 37};
+  const int cand_cfg[3] = {kPp8_288x256, kPp8_224x256, kPp8_192x256};
   for (int c = 0; c < 3; ++c)
     if (cand_tiles[c] > 256 && cand_tiles[c] <= 512 && cand_tiles[c] > best_tiles) {
       best = cand_cfg[c];
       best_tiles = cand_tiles[c];
     }
   if (best >= 0 && best_tiles > 384) return best;
-  if (t192 >= 192 && t192 <= 256) return 37;
-  return 38;
+  if (t192 >= 192 && t192 <= 256) return kPp8_192x256;
+  return kPp8_128x256;
 }
 
 // Launches configuration `ci` with epilogue `epi` (arguments already validated).
@@ -2052,7 +1912,7 @@ static int launch_gemm(int ci, const uint16_t* A, int64_t M, int64_t K, int64_t 
     grid = tiles + warm_slots(cfg, tiles);
   }
   // K stages, or (direct-to-LDS kernels) the bf16 output tile of the epilogue if that is larger.
-  size_t lds = cfg.pf < 0 ? (size_t)kStages * (cfg.bm + cfg.bn) * 64 : (size_t)2 * (cfg.bm + cfg.bn) * 128;
+  size_t lds = (size_t)(cfg.pf == 0 ? dma_stages(cfg.bn) : 2) * (cfg.bm + cfg.bn) * 128;
   if (cfg.pf <= 0) lds = lds > (size_t)cfg.bm * (cfg.bn + 8) * 2 ? lds : (size_t)cfg.bm * (cfg.bn + 8) * 2;
   if (cfg.pf <= -2) lds = r16_lut_offset(cfg.bm, cfg.bn, cfg.wgm, cfg.wgn, cfg.ks, cfg.bk, cfg.nst);
   if (cfg.pf <= 0 && epi == OUDJAT_EPI_BIAS_GELU) lds += kGeluLut * sizeof(uint16_t);
@@ -2167,6 +2027,8 @@ static int linear_bf16_impl(const uint16_t* A, int64_t M, int64_t K, int64_t lda
     ea.acc_scale = 1.0f;
     ea.bias = nullptr;
   }
+  if (aligned_io && far_operands(M, lda, N, ldw))
+    return launch_gemm(far_cfg(N), A, M, K, lda, W, N, ldw, epi, ea, C, ldc, as_stream(stream), "linear_bf16");
   if (workspace && aligned_io && aligned(workspace, 16)) {
     int S = 1;
     const int ci = choose_splitk(M, N, K, epi, &S);
@@ -2225,7 +2087,7 @@ extern "C" int oudjat_linear_swiglu_nvfp4(const uint16_t* A, int64_t M, int64_t 
   ea.xh_ts = tensor_scale;
   // The epilogue exists on the ping-pong tiles; shapes whose choice is another family take 192 x 256.
   int ci = choose_cfg(M, N, K, true);
-  if (kCfgs[ci].fn[kEpiSwigluXh] == nullptr) ci = 31;
+  if (kCfgs[ci].fn[kEpiSwigluXh] == nullptr) ci = kPp192x256;
   return launch_gemm(ci, A, M, K, lda, W, N, ldw, kEpiSwigluXh, ea, xhat, ldc, as_stream(stream), what);
 }
 
@@ -2315,8 +2177,9 @@ static int linear_qkv_rope_kv_impl(const uint16_t* A, int64_t M, int64_t K, int6
   }
   ea.qkv = QkvArgs{(int)H, (int)Dh, sin_table, cos_table, table_stride, patch_mask, rope_idx, batch_idx, token_idx,
                    kv, kv_stride_b, kv_stride_n, q_out};
-  return launch_gemm(choose_qkv_cfg(M, N, K, Dh), A, M, K, lda, W, N, ldw, kEpiQkv, ea, nullptr, 0, as_stream(stream),
-                     "linear_qkv_rope_kv", 1, warm, warm_bytes);
+  const int ci = far_operands(M, lda, N, ldw) ? far_cfg(N) : choose_qkv_cfg(M, N, K, Dh);
+  return launch_gemm(ci, A, M, K, lda, W, N, ldw, kEpiQkv, ea, nullptr, 0, as_stream(stream), "linear_qkv_rope_kv", 1,
+                     warm, warm_bytes);
 }
 
 extern "C" int oudjat_linear_qkv_rope_kv(const uint16_t* A, int64_t M, int64_t K, int64_t lda, const uint16_t* W,
@@ -2389,8 +2252,6 @@ static int kernel_name_of(const GemmCfg& c, int epi, char* buf, int64_t buflen) 
   else if (c.pf == -2)
     n = snprintf(buf, (size_t)buflen, "oudjat::gemm_bf16_r16_kernel<%d, %d, %d, %d, %d, %d, %d, %s, %d>", c.bm, c.bn,
                  c.wgm, c.wgn, c.ks, c.bk, c.nst, c.fb ? "true" : "false", epi);
-  else if (c.pf == -1)
-    n = snprintf(buf, (size_t)buflen, "oudjat::gemm_bf16_pipe_kernel<%d, %d, %d, %d, %d>", c.bm, c.bn, c.wgm, c.wgn, epi);
   else if (c.pf == 0)
     n = snprintf(buf, (size_t)buflen, "oudjat::gemm_bf16_dma_kernel<%d, %d, %d, %d, %d>", c.bm, c.bn, c.wgm, c.wgn, epi);
   else

@@ -185,6 +185,41 @@ def test_linear_tiny_grid(dev, M, N, Kd):
     assert_bf16_close(got, F64.silu_mul(base, r), max_ulps=1, max_frac_off=1e-3, what="tiny + swiglu")
 
 
+# Products below a round of large tiles, one or two on every small tile (the kernel's name is part of the
+# case): ragged row counts, one row, widths that are no multiple of 128, depths that are no multiple of 128.
+SMALL_SHAPES = [(1, 64, 1024, "r16_kernel<32, 64, 1, 4, 2, 128, 2"), (103, 768, 1024, "r16_kernel<32, 64, 1, 4, 2, 128, 2"),
+                (1401, 384, 384, "r16_kernel<64, 64, 1, 4, 2, 128, 2"), (1001, 1088, 768, "r16_kernel<64, 64, 1, 4, 2, 128, 2"),
+                (1, 192, 1536, "r16_kernel<64, 64, 1, 4, 2, 128, 3"), (1152, 768, 3072, "r16_kernel<64, 64, 1, 4, 2, 128, 3"),
+                (705, 1536, 512, "r16_kernel<96, 64, 1, 4, 2, 128, 2"), (1153, 1088, 512, "r16_kernel<96, 64, 1, 4, 2, 128, 2"),
+                (1, 384, 1216, "r16_kernel<64, 128, 1, 4, 2, 64, 4"), (1713, 1024, 1216, "r16_kernel<64, 128, 1, 4, 2, 64, 4"),
+                (1, 320, 1216, "dma_kernel<64, 64, 2, 2"), (1153, 2304, 768, "dma_kernel<64, 64, 2, 2"),
+                (1153, 3072, 768, "dma_kernel<128, 64, 2, 2"), (9001, 192, 64, "dma_kernel<64, 64, 2, 2"),
+                (2089, 3072, 1216, "dma_kernel<128, 128, 2, 2"), (1401, 3072, 1024, "r16_kernel<144, 128, 1, 4, 2, 128, 2"),
+                (33, 768, 3072, "r16_kernel<64, 64, 1, 4, 2, 128, 2, false, 6"),   # split K on the small tiles
+                (37, 1536, 3072, "r16_kernel<64, 64, 1, 4, 2, 128, 3, false, 6"),
+                (161, 384, 4096, "r16_kernel<96, 64, 1, 4, 2, 128, 2, false, 6"),
+                (203, 4096, 3072, "r16_kernel<64, 128, 1, 4, 2, 64, 4, true, 6")]
+
+
+@pytest.mark.parametrize("M,N,Kd,kernel", SMALL_SHAPES)
+def test_linear_small_tiles(dev, M, N, Kd, kernel):
+    """Within the accumulation bound of the oracle, and every epilogue the oracle's epilogue of the same
+    bf16(acc + bias)."""
+    print(f"small tiles {M}x{N}x{Kd}", flush=True)
+    assert kernel in K.linear_kernel_name(M, N, Kd, _lib.EPI_BIAS), K.linear_kernel_name(M, N, Kd, _lib.EPI_BIAS)
+    xd, wd, bd, base = _epi_case(dev, M, N, Kd, 80)
+    g, r = _rand((N,), 84), _rand((M, N), 85)
+    got = K.linear(xd, wd, bd, epilogue=_lib.EPI_BIAS_LS, gamma=g.to(dev))
+    assert_bits_equal(got, F64.mul(base, g), "small + ls")
+    got = K.linear(xd, wd, bd, epilogue=_lib.EPI_BIAS_LS_RESID, gamma=g.to(dev), resid=r.to(dev))
+    assert_bits_equal(got, F64.fma_add(r, base, g), "small + ls + resid")
+    got = K.linear(xd, wd, bd, epilogue=_lib.EPI_BIAS_GELU)
+    assert_bf16_close(got, F64.gelu(base), max_ulps=1, max_frac_off=max(1e-3, 1.0 / base.numel()), what="small + gelu")
+    got = K.linear(xd, wd, bd, epilogue=_lib.EPI_BIAS_SILU_MUL, resid=r.to(dev))
+    assert_bf16_close(got, F64.silu_mul(base, r), max_ulps=1, max_frac_off=max(1e-3, 1.0 / base.numel()),
+                      what="small + swiglu")
+
+
 def test_linear_without_workspace_does_not_split(dev):
     """The C ABI without a workspace runs the one-launch kernel: same bound, and the workspace size
     query is 0 for a shape that fills the GPU."""
