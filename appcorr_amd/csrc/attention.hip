@@ -17,11 +17,11 @@
 // the LDS transpose read (ds_read_tr16_b64, its lane mapping described above the buffer-load
 // kernel).
 //
-// One workgroup per (image, head) covers up to 10 query waves = 320 queries (8 for Dh = 128); larger T
-// is split evenly over several workgroups. At the headline shape (T = 261: 8 full waves and a last
-// wave of 5 queries, 256 workgroups for B*H = 256, one per CU) the buffer-load kernel shares the
-// last wave's key tiles among 4 waves, so each workgroup runs 12. K/V tiles of 64 keys are double-buffered in LDS with the next tile's global loads in
-// flight during the current tile's MFMAs, so each (image, head) streams its K/V once.
+// Query waves per workgroup and workgroups per (image, head) are chosen per shape (attn_shape): 4 to 12
+// waves at Dh = 64, up to 8 at Dh = 128. At the headline shape (T = 261: 8 full waves and a last wave of 5
+// queries, 256 workgroups for B*H = 256, one per CU) the buffer-load kernel shares the last wave's key
+// tiles among 4 waves, so each workgroup runs 12. K/V tiles of 64 keys are staged in LDS with the next
+// tiles' global loads in flight during the current tile's MFMAs.
 #include <stdlib.h>
 
 #include <type_traits>
@@ -383,9 +383,9 @@ __global__ __launch_bounds__((DH == 64 ? kMaxWaves64 : kMaxWaves128) * 64) void 
 
 
 // ------------------------------------------------------------------------------------------------
-// Dh = 64, >= 8 waves: K and V tiles reach LDS by buffer loads straight from the cache (no register
-// staging), both in their natural [key][dim] rows, NST stages deep. Waves 0..7 each load 8 rows of K
-// and 8 rows of V per tile (one 1 KB instruction each); keys past N fall outside the per-(image,
+// Dh = 64: K and V tiles reach LDS by buffer loads straight from the cache (no register staging), both
+// in their natural [key][dim] rows, NST stages deep. Waves 0..7 each load 8 rows of K and 8 rows of V
+// per tile (one 1 KB instruction each; with fewer than 8 waves, waves 0..3 load two such groups); keys past N fall outside the per-(image,
 // head) descriptors and load as zeros (their scores are masked). The A operand of O^T += V^T . P^T
 // comes from V's rows through the LDS transpose read: in each 16-lane group, source lane s addresses
 // 4 dims (8 bytes) of key k0 + s / 4 at dim c0 + 4 (s % 4), and lane j receives dim c0 + j for keys
@@ -407,24 +407,19 @@ __device__ __forceinline__ int kv_slot(int row, int chunk) { return row * 128 + 
 // light_split: 0, or kLightParts when the launch has one workgroup per (image, head) whose last
 // query wave is light; that wave's work is then done by kLightParts waves (the last ones), part p
 // taking the key tiles t with t % NST == p, and merged at the end (see the light path below).
-// full_split: 1, or 2 (small T, one workgroup per (image, head)): each full query wave's work is done
-// by two waves, part p taking the tiles of stages p and p + 2, merged at the end like the light
-// parts, so that a workgroup of few query waves still puts two or three waves on every SIMD.
-// full_split is a template parameter so that without it the full waves' stage mask is a constant and
-// each tile's S^T MFMAs and the previous tile's softmax stay in one basic block (interleaved).
 // Key-part workspace of a split launch, per (image, head, part): the running max of each query
 // (kv_part_rows(T) floats, T rounded up to 4 so the rows below stay 16-byte aligned), its sum (as
 // many), then its unnormalised 64-dim output rows (T x 64).
 __host__ __device__ __forceinline__ int64_t kv_part_rows(int64_t T) { return (T + 3) & ~(int64_t)3; }
 __host__ __device__ __forceinline__ int64_t kv_part_stride(int64_t T) { return 2 * kv_part_rows(T) + 64 * T; }
 
-template <int NST, int FSPLIT, bool KVS>
-__global__ __launch_bounds__(kDmaMaxWaves * 64) void sq_attention_dma_kernel(
+// LPW: K/V row groups a loader wave takes per tile: 1 (waves 0..7 load) with at least 8 waves, else 2
+// (waves 0..3).
+template <int NST, bool KVS, int LPW>
+__global__ __launch_bounds__((LPW == 1 ? kDmaMaxWaves : 8) * 64) void sq_attention_dma_kernel(
     const uint16_t* __restrict__ q, int64_t qrs, int T, const uint16_t* __restrict__ kv, int64_t kvb, int64_t kvn,
     int64_t kvkv, int64_t kvh, int N, float scale_log2, uint16_t* __restrict__ out, int64_t ors,
     int waves_per_wg, int light_split, float* __restrict__ part_ws, int kv_parts) {
-  constexpr int full_split = FSPLIT;
-  static_assert(FSPLIT == 1 || FSPLIT == 2, "full_split");
   constexpr int DH = 64, QK_STEPS = 4, OB = 2;
   constexpr int TILEB = kKeyTile * 128;  // one K (or V) tile: 64 rows of 128 bytes
   constexpr int STAGE = 2 * TILEB;
@@ -433,35 +428,45 @@ __global__ __launch_bounds__(kDmaMaxWaves * 64) void sq_attention_dma_kernel(
 
   extern __shared__ __align__(16) unsigned char smem[];
 
-  const int b = blockIdx.z, h = blockIdx.y;
-  // KVS: one query workgroup per (image, head) and blockIdx.x = key part (contiguous tile ranges).
-  const int qblk = KVS ? 0 : (int)blockIdx.x;
+  // Workgroups that share an (image, head)'s K and V go to one XCD (ids 8 apart), so that its L2 serves all
+  // but the first: pairs are taken in groups of 8, query workgroups outermost within a group.
+  int b = blockIdx.z, h = blockIdx.y, x = blockIdx.x;
+  if (gridDim.x > 1) {
+    const int nx = (int)gridDim.x, H = (int)gridDim.y, pairs = H * (int)gridDim.z;
+    const int id = x + nx * (h + H * b);
+    const int first = id / (8 * nx) * 8, rem = id - first * nx, m = min(8, pairs - first);
+    x = rem / m;
+    const int pair = first + rem - x * m;
+    b = pair / H;
+    h = pair - b * H;
+  }
+  // KVS: x = query workgroup * kv_parts + key part (contiguous tile ranges).
+  const int kpart = KVS ? x % kv_parts : 0;
+  const int qblk = KVS ? x / kv_parts : x;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l32 = lane & 31, g = lane >> 5;
-  // Query wave of this wave, its part of a split full wave (fpart, 0 without a split) and its part of
-  // a split light wave (lpart, -1: not split). Full query waves 0 .. nfq - 1 take waves
-  // [0, nfq * full_split), the split light wave the kLightParts waves after them.
+  // Query wave of this wave and its part of a split light wave (lpart, -1: not split). Full query waves
+  // 0 .. nfq - 1 take waves 0 .. nfq - 1, the split light wave the kLightParts waves after them.
   const int nfq = light_split ? waves_per_wg - 1 : waves_per_wg;
-  const int lpart = (light_split && wave >= nfq * full_split) ? wave - nfq * full_split : -1;
-  const int fpart = lpart >= 0 ? 0 : wave % full_split;
-  const int qwave = lpart >= 0 ? waves_per_wg - 1 : wave / full_split;
-  const int q0 = (qblk * waves_per_wg + qwave) * 32;
+  const int lpart = (light_split && wave >= nfq) ? wave - nfq : -1;
+  const int qwave = lpart >= 0 ? waves_per_wg - 1 : wave;
+  const int q0 = qwave < waves_per_wg ? (qblk * waves_per_wg + qwave) * 32 : T;  // waves past them only load
   const bool active = q0 < T;
-  const bool merged = light_split || full_split > 1;  // the parts meet in LDS after the key loop
+  const bool merged = light_split;  // the light parts meet in LDS after the key loop
 
   const uint16_t* kbase = kv + (int64_t)b * kvb + (int64_t)h * kvh;
   const uint32_t bytes = (uint32_t)((int64_t)N * kvn * 2);
   const i32x4_t rsrc_k = make_buffer_rsrc(kbase, bytes);
   const i32x4_t rsrc_v = make_buffer_rsrc(kbase + kvkv, bytes);
-  const bool loader = wave < 8;
-  const int lrow = 8 * wave + (lane >> 3);                  // tile row this lane loads
+  const bool loader = wave < 8 / LPW;
+  const int lrow = 8 * wave + (lane >> 3);                  // tile row this lane loads (LPW = 2: and row + 32)
   const uint32_t tstep = (uint32_t)kKeyTile * (uint32_t)kvn * 2u;
   // Key tiles of this workgroup: [tb, tb + ntiles); tiles are numbered from tb in the loops below.
   int tb = 0, ntiles = (N + kKeyTile - 1) / kKeyTile;
   if constexpr (KVS) {
     const int per = (ntiles + kv_parts - 1) / kv_parts;
-    tb = (int)blockIdx.x * per;
+    tb = kpart * per;
     ntiles = min(per, ntiles - tb);
   }
   const uint32_t off0 = (uint32_t)lrow * (uint32_t)kvn * 2u + (uint32_t)(((lane & 7) ^ kv_swz(lrow)) << 4) +
@@ -471,15 +476,20 @@ __global__ __launch_bounds__(kDmaMaxWaves * 64) void sq_attention_dma_kernel(
       unsigned char* base = smem + stage * STAGE + wave * 1024;
       buffer_load_lds16(rsrc_k, base, off0 + (uint32_t)t * tstep);
       buffer_load_lds16(rsrc_v, base + TILEB, off0 + (uint32_t)t * tstep);
+      if constexpr (LPW == 2) {  // rows 32 further on: the same swizzle
+        const uint32_t far = off0 + (uint32_t)t * tstep + 32u * (uint32_t)kvn * 2u;
+        buffer_load_lds16(rsrc_k, base + 4096, far);
+        buffer_load_lds16(rsrc_v, base + 4096 + TILEB, far);
+      }
     }
   };
-  // At most n tiles after the one needed may still be in flight (two loads per tile per loader).
+  // At most n tiles after the one needed may still be in flight (2 LPW loads per tile per loader).
   static_assert(NST <= 5, "wait_tiles covers up to three tiles in flight");
   auto wait_tiles = [&](int n) __attribute__((always_inline)) {
     if (n <= 0) wait_vmcnt<0>();
-    else if (n == 1) wait_vmcnt<2>();
-    else if (n == 2) wait_vmcnt<4>();
-    else wait_vmcnt<6>();
+    else if (n == 1) wait_vmcnt<2 * LPW>();
+    else if (n == 2) wait_vmcnt<4 * LPW>();
+    else wait_vmcnt<6 * LPW>();
   };
 
   // Query fragments, loaded before the K/V prologue so that their latency overlaps the first tiles'
@@ -517,17 +527,15 @@ __global__ __launch_bounds__(kDmaMaxWaves * 64) void sq_attention_dma_kernel(
   using I1 = std::integral_constant<int, 1>;
   using I2 = std::integral_constant<int, 2>;
   using I3 = std::integral_constant<int, 3>;
-  // `stages`: bit s set when this wave computes the tiles held in stage s (all of them, except for
-  // the parts of a split light wave).
   // `act`: `active`, or std::true_type where the caller knows the wave is active (the full waves:
   // T - q0 > 16), so that no branch separates a tile's S^T MFMAs from the previous tile's softmax and
   // the scheduler can interleave them. The steps of the main loop never hold the last (ragged) key
   // tile, so their softmax has no masking branch either (`mask_c` false).
   using BF = std::false_type;
   using BT = std::true_type;
-  auto pipeline = [&](auto& sa, auto& sb, auto&& scores, auto&& finish, auto stages, auto act)
+  auto pipeline = [&](auto& sa, auto& sb, auto&& scores, auto&& finish, auto act)
                       __attribute__((always_inline)) {
-    if (act && (stages & 1)) scores(sa, smem);
+    if (act) scores(sa, smem);
     auto step = [&](auto stage_c, int t, auto& cur, auto& nxt, auto last_c) __attribute__((always_inline)) {
       constexpr int SG = decltype(stage_c)::value;  // stage of tile t
       constexpr bool TAIL = decltype(last_c)::value;  // the step may hold the last tile
@@ -535,9 +543,9 @@ __global__ __launch_bounds__(kDmaMaxWaves * 64) void sq_attention_dma_kernel(
         wait_tiles(min(NST - 3, ntiles - 2 - t));
         block_barrier();
         if (t + NST - 1 < ntiles) issue((SG + NST - 1) % NST, t + NST - 1);
-        if (act && ((stages >> ((SG + 1) % NST)) & 1)) scores(nxt, smem + ((SG + 1) % NST) * STAGE);
+        if (act) scores(nxt, smem + ((SG + 1) % NST) * STAGE);
       }
-      if (act && ((stages >> SG) & 1)) finish(cur, smem + SG * STAGE, t, last_c);
+      if (act) finish(cur, smem + SG * STAGE, t, last_c);
     };
     int t = 0;
     for (; t + NST < ntiles; t += NST) {
@@ -659,44 +667,16 @@ __global__ __launch_bounds__(kDmaMaxWaves * 64) void sq_attention_dma_kernel(
       }
     };
     Scores sa, sb;
-    if constexpr (FSPLIT > 1)
-      pipeline(sa, sb, scores, finish, 0x5 << fpart, BT{});
-    else
-      pipeline(sa, sb, scores, finish, std::integral_constant<int, (1 << NST) - 1>{}, BT{});
+    pipeline(sa, sb, scores, finish, BT{});
 
-    if (merged) {
-      // Every wave has passed its last tile's reads after the first barrier, so the stages are free.
-      // Full-wave parts park behind the light parts' area: m, l, o[2][16] for 64 lanes per wave.
-      constexpr int LIGHT_AREA = (kLightParts - 1) * 18 * 64;
-      constexpr int FSTRIDE = 34 * 64;
-      float* fpark = reinterpret_cast<float*>(smem) + LIGHT_AREA + qwave * FSTRIDE;
+    if (merged) {  // the barriers of the light parts' merge
       block_barrier();
-      if (full_split > 1 && fpart == 1) {
-        fpark[lane] = m_i;
-        fpark[64 + lane] = l_i;
-#pragma unroll
-        for (int d = 0; d < OB; ++d)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) fpark[(2 + 16 * d + v) * 64 + lane] = o[d][v];
-      }
       block_barrier();
-      if (full_split > 1 && fpart == 0) {
-        const float m1 = fpark[lane], l1 = fpark[64 + lane];
-        const float m = fmaxf(m_i, m1);  // part 0 holds tile 0: m is finite
-        const float a0 = __builtin_amdgcn_exp2f((m_i - m) * scale_log2);
-        const float a1 = __builtin_amdgcn_exp2f((m1 - m) * scale_log2);
-        l_i = fmaf(l1, a1, l_i * a0);
-        m_i = m;  // l_i and o are now relative to m (read by a key-part write)
-#pragma unroll
-        for (int d = 0; d < OB; ++d)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) o[d][v] = fmaf(fpark[(2 + 16 * d + v) * 64 + lane], a1, o[d][v] * a0);
-      }
     }
     const int qr = q0 + l32;
-    if (KVS && active && qr < T && fpart == 0) {
+    if (KVS && active && qr < T) {
       // This key part's unnormalised output, running max and sum (sq_attention_merge_kernel).
-      float* ws = part_ws + ((int64_t)(b * (int)gridDim.y + h) * kv_parts + (int)blockIdx.x) * kv_part_stride(T);
+      float* ws = part_ws + ((int64_t)(b * (int)gridDim.y + h) * kv_parts + kpart) * kv_part_stride(T);
       if (g == 0) {
         ws[qr] = m_i;
         ws[kv_part_rows(T) + qr] = l_i;
@@ -708,7 +688,7 @@ __global__ __launch_bounds__(kDmaMaxWaves * 64) void sq_attention_dma_kernel(
         for (int r4 = 0; r4 < 4; ++r4)
           *reinterpret_cast<f32x4_t*>(orow + d * 32 + 8 * r4 + 4 * g) =
               f32x4_t{o[d][4 * r4], o[d][4 * r4 + 1], o[d][4 * r4 + 2], o[d][4 * r4 + 3]};
-    } else if (active && qr < T && fpart == 0) {
+    } else if (active && qr < T) {
       const float inv = 1.0f / l_i;
       uint16_t* orow = out + ((int64_t)b * T + qr) * ors + (int64_t)h * DH;
 #pragma unroll
@@ -828,7 +808,6 @@ __global__ __launch_bounds__(kDmaMaxWaves * 64) void sq_attention_dma_kernel(
         }
       }
     };
-    using AllStages = std::integral_constant<int, (1 << NST) - 1>;
     if (lpart >= 0) {
       // Split light wave: part p takes keys 16 p .. 16 p + 15 of every tile, so every SIMD gets the
       // same share of the light work at every step. S^T of the slice is one 16-key block (A = K rows
@@ -888,10 +867,10 @@ __global__ __launch_bounds__(kDmaMaxWaves * 64) void sq_attention_dma_kernel(
         }
       };
       ScoresQ qa, qb;
-      pipeline(qa, qb, scores_q, finish_q, AllStages{}, active);
+      pipeline(qa, qb, scores_q, finish_q, active);
     } else {
       Scores16 sa, sb;
-      pipeline(sa, sb, scores, finish, AllStages{}, active);
+      pipeline(sa, sb, scores, finish, active);
     }
 
     if (merged) {
@@ -945,7 +924,7 @@ __global__ __launch_bounds__(kDmaMaxWaves * 64) void sq_attention_dma_kernel(
     // O^T[16 db + 4 G + v][query l16]: 4 consecutive dims per lane and block.
     const int qr = q0 + l16;
     if (KVS && active && qr < T && lpart <= 0) {
-      float* ws = part_ws + ((int64_t)(b * (int)gridDim.y + h) * kv_parts + (int)blockIdx.x) * kv_part_stride(T);
+      float* ws = part_ws + ((int64_t)(b * (int)gridDim.y + h) * kv_parts + kpart) * kv_part_stride(T);
       if (G == 0) {
         ws[qr] = m_i;
         ws[kv_part_rows(T) + qr] = l_i;
@@ -1032,61 +1011,92 @@ __global__ __launch_bounds__(256) void sq_attention_merge_kernel(const float* __
   *reinterpret_cast<bf16x4_t*>(orow + 4) = w1;
 }
 
-// Two waves per full query wave (the buffer-load kernel's full_split) when a single workgroup per
-// (image, head) would otherwise have fewer than 8 waves, as long as the split still has the 8 loader
-// waves, fits the workgroup and leaves room for the parked partials (4 full waves at most).
-static int full_split_for(int64_t n_wg, int64_t nfq, int light_parts) {
-  if (n_wg != 1 || nfq > 4) return 1;
-  const int64_t waves = 2 * nfq + light_parts;
-  return (waves >= 8 && waves <= kDmaMaxWaves && nfq + (light_parts ? 1 : 0) < 8) ? 2 : 1;
-}
-
 }  // namespace oudjat
 
 using namespace oudjat;
 
-// Launch shape of a sparse_query_attention call: query workgroups per (image, head), waves per
-// workgroup, and for the buffer-load kernel its light split, full split and key parts.
+// Launch shape of a sparse_query_attention call: query workgroups per (image, head), query waves per
+// workgroup, and for the buffer-load kernel its light split, key parts and waves.
 struct AttnShape {
   int64_t n_wg;
   int w;
   bool dma;
-  int split, nfq, fsplit, kv_parts;
+  int split, kv_parts, waves;
 };
+
+// Modelled time (us) of the buffer-load kernel: wgs workgroups of `waves` waves (w query waves, three more
+// when a light one is split) over L key tiles each, reading `streams` distinct K/V ranges; light: the last
+// query wave has 1..16 queries. Up to four waves, a wave runs alone on its SIMD and two workgroups share a
+// CU; above, one workgroup holds the CU and the SIMD with the most waves sets the pace per tile (a step at
+// every multiple of four). Fitted to sweeps over 100 shapes of 4 .. 65 tiles (below one round of workgroups
+// of up to four waves, 640 points, within 3 % rms); it only ranks the shapes of one call.
+static double attn_wg_us(int64_t wgs, int64_t streams, int w, int waves, bool light, int64_t L) {
+  if (waves <= 4) {
+    const double u = std::min(1.0, (double)streams / kNumCus), lt = light ? 0.08 : 0.0;
+    if (wgs <= kNumCus) return 3.85 + 0.15 * w + (double)L * (0.58 + 0.02 * w + 0.26 * u * u + lt);
+    if (wgs <= 2 * kNumCus) return 5.2 + (double)L * (0.92 + 0.09 * w + lt);
+    const double rounds = std::max((double)wgs / (2 * kNumCus), 1.5);  // a short second round costs half of one
+    return 5.0 + rounds * ((double)L * (0.66 + 0.14 * w + lt) + 1.0);
+  }
+  static const double tile_us[13] = {0, 0, 0, 0, 0, 1.00, 1.05, 1.10, 1.17, 1.50, 1.65, 1.85, 1.95};
+  const double t = waves == w ? tile_us[w] : (w <= 4 ? 0.84 : w == 5 ? 0.90 : 1.42);  // with a split light wave
+  const double f = std::min(1.0, (double)wgs / kNumCus);
+  const double round = (waves == w ? 6.0 : 6.2) + (double)L * t * (0.8 + 0.2 * f);
+  const int64_t full = wgs / kNumCus;
+  return round * ((double)full + (wgs % kNumCus ? (full ? 0.8 : 1.0) : 0.0));
+}
 
 static AttnShape attn_shape(int64_t B, int64_t T, int64_t H, int64_t Dh, int64_t N, bool offsets_fit) {
   AttnShape s{};
   const int64_t waves = cdiv(T, 32);
-  s.n_wg = cdiv(waves, Dh == 64 ? kMaxWaves64 : kMaxWaves128);
-  s.w = (int)cdiv(waves, s.n_wg);
-  if (s.w < kMinWaves) s.w = kMinWaves;
-  // Buffer-load kernel for Dh = 64 with >= 8 waves, counting the waves of split full and light
-  // query waves (its byte offsets must fit 31 bits); the register-staged kernel otherwise.
-  const int w = s.w;
-  const bool small_split = s.n_wg == 1 && w < 8 && full_split_for(s.n_wg, (T - (w - 1) * 32 <= 16) ? w - 1 : w,
-                                                                 (T - (w - 1) * 32 <= 16) ? kLightParts : 0) > 1;
-  s.dma = Dh == 64 && (w >= 8 || small_split) && offsets_fit;
+  // Buffer-load kernel for Dh = 64 (its byte offsets must fit 31 bits); the register-staged kernel
+  // otherwise.
+  s.dma = Dh == 64 && offsets_fit;
   s.kv_parts = 1;
-  if (!s.dma) return s;
-  // One workgroup per (image, head) whose last query wave is light (1..16 queries): that wave is
-  // split over kLightParts waves (its merge area, 3 parts of 18 x 64 floats, fits the stages).
-  const int64_t last = T - (w - 1) * 32;
-  s.split = (s.n_wg == 1 && last >= 1 && last <= 16 && w - 1 + kLightParts <= kDmaMaxWaves) ? kLightParts : 0;
-  s.nfq = s.split ? w - 1 : w;
-  s.fsplit = full_split_for(s.n_wg, s.nfq, s.split);
-  // Key parts: with one workgroup per (image, head) and fewer than half as many (image, head) pairs
-  // as CUs, the key tiles are dealt to up to kMaxKvParts workgroups per pair in contiguous ranges
-  // (as many as one round of workgroups on the CUs holds), and a merge launch combines them.
-  const int64_t pairs = B * H;
-  const int64_t ntiles = cdiv(N, kKeyTile);
-  if (s.n_wg == 1 && 2 * pairs <= kNumCus) {
-    int64_t parts = std::min<int64_t>(std::min<int64_t>(kNumCus / pairs, ntiles), kMaxKvParts);
-    const int64_t per = cdiv(ntiles, parts);
-    parts = cdiv(ntiles, per);
-    // Worth it only when each workgroup is spared at least kMinTilesSaved key tiles (~1 us each),
-    // against the merge launch (~3-5 us).
-    if (parts >= 2 && ntiles - per >= kMinTilesSaved) s.kv_parts = (int)parts;
+  if (!s.dma) {
+    s.n_wg = cdiv(waves, Dh == 64 ? kMaxWaves64 : kMaxWaves128);
+    s.w = (int)std::max<int64_t>(cdiv(waves, s.n_wg), kMinWaves);
+    return s;
   }
+  // Query waves per workgroup: the shape of least modelled time among 1 to 4 (the finest fill of the CUs) and
+  // 5 to 12 waves (up to three on every SIMD); one workgroup per (image, head) may split its light last wave
+  // (1..16 queries) over kLightParts waves (the merge area, 3 parts of 18 x 64 floats, fits the stages). Key
+  // parts: the key tiles of each query workgroup dealt to 2 .. kMaxKvParts workgroups in contiguous ranges,
+  // whose fp32 rows a merge launch combines (2 us and their bytes); always for few pairs of up to ten waves
+  // and many tiles, else where it is modelled faster.
+  // Measured (HIP graph, before -> after; B x heads, queries of keys): 16 x 16, 1029 of 1029 132 -> 110 us
+  // (four workgroups of nine waves -> three of eleven); 16 x 16, 330 of 1029 65.5 -> 38.8 (two of six -> one of
+  // eleven); 3 x 12, 384 of 764 21.2 -> 12.1 (two of six, register-staged -> six of two); 1 x 16, 1500 of 4101
+  // 96 -> 50; 16 x 16, 107 of 1029 25.0 -> 19.9 (two waves per full query wave -> one); 2 x 6, 200 of 1000
+  // 26.2 -> 10.0 (four key parts); 1 x 6, 103 of 201 8.3 -> 6.0 (one of four -> four of one).
+  const int64_t pairs = B * H, L = cdiv(N, kKeyTile);
+  const int64_t few = std::min<int64_t>(std::min<int64_t>(kNumCus / std::max<int64_t>(pairs, 1), L), kMaxKvParts);
+  const bool must_split = waves <= 10 && 2 * pairs <= kNumCus && few >= 2 && L - cdiv(L, few) >= kMinTilesSaved;
+  double best = -1.0;
+  auto consider = [&](int64_t n, bool light) {
+    const int w = (int)cdiv(waves, n);
+    if (n < 1 || w > kDmaMaxWaves) return;
+    const int64_t last = T - (int64_t)(w - 1) * 32;  // queries of the last wave (n == 1)
+    const int split = light ? kLightParts : 0;
+    if (light && (n > 1 || last > 16 || w < 4 || w - 1 + kLightParts > kDmaMaxWaves)) return;
+    const int all = std::max(split ? w - 1 + kLightParts : w, kMinWaves);
+    for (int64_t p = must_split ? 2 : 1; p <= std::min<int64_t>(L, kMaxKvParts); ++p) {
+      const int64_t per = cdiv(L, p);
+      if (cdiv(L, per) != p) continue;
+      double us = attn_wg_us(pairs * n * p, pairs * p, w, all, n == 1 && last <= 16, per);
+      if (p > 1) us += 2.0 + (double)pairs * T * p * (64 + 2) * 4 * 2 / 3e6;
+      if (best >= 0.0 && us >= best) continue;
+      best = us;
+      s.n_wg = n;
+      s.split = split;
+      s.waves = all;
+      s.w = w;
+      s.kv_parts = (int)p;
+    }
+  };
+  for (int64_t w = 1; w <= kMinWaves; ++w) consider(cdiv(waves, w), false);
+  for (int64_t n = cdiv(waves, kDmaMaxWaves); n <= cdiv(waves, 5) && n <= cdiv(waves, kDmaMaxWaves) + 4; ++n) consider(n, false);
+  consider(1, true);
   return s;
 }
 
@@ -1114,7 +1124,8 @@ static int sparse_query_attention_impl(const uint16_t* q, int64_t qrs, int64_t B
   OUDJAT_REQUIRE(N < ((int64_t)1 << 30) && T < ((int64_t)1 << 30), OUDJAT_ERR_TOO_LARGE,
                  "sparse_query_attention: N or T too large");
   const float scale_log2 = scale * 1.4426950408889634f;
-  const AttnShape s = attn_shape(B, T, H, Dh, N, N * kvn * 2 < ((int64_t)1 << 31));
+  // The row log-sum-exp comes from the register-staged kernel.
+  const AttnShape s = attn_shape(B, T, H, Dh, N, !lse && N * kvn * 2 < ((int64_t)1 << 31));
   const int w = s.w;
   dim3 grid((unsigned)s.n_wg, (unsigned)H, (unsigned)B);
   hipStream_t st = as_stream(stream);
@@ -1138,20 +1149,20 @@ static int sparse_query_attention_impl(const uint16_t* q, int64_t qrs, int64_t B
     const size_t lds_dma = (size_t)kAttnStages * 2 * kKeyTile * 128;
     static_assert((size_t)kAttnStages * 2 * kKeyTile * 128 <= 64 * 1024, "needs no larger-LDS attribute");
     static_assert((kLightParts - 1) * 18 * 64 * 4 <= kAttnStages * 2 * kKeyTile * 128, "merge area");
-    static_assert(((kLightParts - 1) * 18 + 4 * 34) * 64 * 4 <= kAttnStages * 2 * kKeyTile * 128,
-                  "merge area of the light parts and of four split full waves");
-    const int threads = (s.nfq * s.fsplit + (s.split ? kLightParts : 0)) * 64;
+    const int threads = s.waves * 64;
     const int split = s.split;
     const bool kvs = s.kv_parts > 1 && workspace && aligned(workspace, 16) &&
                      attn_workspace_elems(B, T, H, s.kv_parts) <= workspace_elems;
-    if (kvs) {
-      dim3 pgrid((unsigned)s.kv_parts, (unsigned)H, (unsigned)B);
-      if (s.fsplit > 1)
-        sq_attention_dma_kernel<kAttnStages, 2, true><<<pgrid, threads, lds_dma, st>>>(
-            q, qrs, (int)T, kv, kvb, kvn, kvkv, kvh, (int)N, scale_log2, out, ors, w, split, workspace, s.kv_parts);
+    auto launch_kv = [&](auto kvs_c, dim3 g, float* ws, int parts) {
+      if (s.waves >= 8)
+        sq_attention_dma_kernel<kAttnStages, decltype(kvs_c)::value, 1><<<g, threads, lds_dma, st>>>(
+            q, qrs, (int)T, kv, kvb, kvn, kvkv, kvh, (int)N, scale_log2, out, ors, w, split, ws, parts);
       else
-        sq_attention_dma_kernel<kAttnStages, 1, true><<<pgrid, threads, lds_dma, st>>>(
-            q, qrs, (int)T, kv, kvb, kvn, kvkv, kvh, (int)N, scale_log2, out, ors, w, split, workspace, s.kv_parts);
+        sq_attention_dma_kernel<kAttnStages, decltype(kvs_c)::value, 2><<<g, threads, lds_dma, st>>>(
+            q, qrs, (int)T, kv, kvb, kvn, kvkv, kvh, (int)N, scale_log2, out, ors, w, split, ws, parts);
+    };
+    if (kvs) {
+      launch_kv(std::true_type{}, dim3((unsigned)(s.n_wg * s.kv_parts), (unsigned)H, (unsigned)B), workspace, s.kv_parts);
       const int rc = check_launch("sparse_query_attention");
       if (rc != OUDJAT_OK) return rc;
       const unsigned mgrid = (unsigned)cdiv(B * T * H * 8, 256);
@@ -1173,14 +1184,7 @@ static int sparse_query_attention_impl(const uint16_t* q, int64_t qrs, int64_t B
       }
       return check_launch("sparse_query_attention (merge)");
     }
-    if (s.fsplit > 1)
-      sq_attention_dma_kernel<kAttnStages, 2, false><<<grid, threads, lds_dma, st>>>(q, qrs, (int)T, kv, kvb, kvn, kvkv,
-                                                                                      kvh, (int)N, scale_log2, out, ors,
-                                                                                      w, split, nullptr, 1);
-    else
-      sq_attention_dma_kernel<kAttnStages, 1, false><<<grid, threads, lds_dma, st>>>(q, qrs, (int)T, kv, kvb, kvn, kvkv,
-                                                                                      kvh, (int)N, scale_log2, out, ors,
-                                                                                      w, split, nullptr, 1);
+    launch_kv(std::false_type{}, grid, nullptr, 1);
     return check_launch("sparse_query_attention");
   }
   // Two stages of one K and one V tile (64 keys x Dh bf16 each): 32 KB at Dh = 64, 64 KB at

@@ -506,6 +506,26 @@ def test_attention_key_split(dev, B, T, N, H, scale_up):
     assert_bits_equal(short.cpu(), plain.cpu(), "workspace too small: unsplit kernel")
 
 
+@pytest.mark.parametrize("B,T,N,H", [(1, 1, 1, 1), (1, 103, 201, 6), (1, 200, 261, 7), (3, 384, 764, 12), (2, 200, 1000, 6),
+                                     (1, 1500, 1101, 5), (16, 330, 193, 16), (16, 384, 129, 16), (16, 33, 65, 16),
+                                     (5, 64, 1029, 9), (16, 107, 1029, 16), (3, 385, 600, 3), (16, 517, 128, 16)])
+def test_attention_launch_shapes(dev, B, T, N, H):
+    """Dh = 64: one to twelve query waves per workgroup (with idle loader waves, two K/V row groups per
+    loader below eight waves), several query workgroups per (image, head) with and without key parts,
+    pair counts off a multiple of eight in the workgroup numbering, key counts one past a tile; against
+    the float64 reference, and repeated launches are bit-identical."""
+    D = 64
+    print(f"attention launch shape {B},{T},{N},{H}", flush=True)
+    q = _rand((B * T, H, D), 46)
+    kv = _rand((B, N, 2, H, D), 47)
+    qd, kvd = q.to(dev), kv.to(dev)
+    got = K.sparse_query_attention(qd, kvd, T, D ** -0.5)
+    assert_bits_equal(K.sparse_query_attention(qd, kvd, T, D ** -0.5).cpu(), got.cpu(), "repeat launch")
+    qb = q.reshape(B, T, H, D).transpose(1, 2)
+    o64 = F64.sdpa(qb, kv[:, :, 0].transpose(1, 2), kv[:, :, 1].transpose(1, 2), D ** -0.5)
+    _check_attention(got.cpu(), qb, kv, D ** -0.5, o64.transpose(1, 2).reshape(B * T, H * D), f"shape {B},{T},{N},{H}")
+
+
 @pytest.mark.parametrize("B,T,N,H,scale_up", [(4, 414, 4101, 32, 1.0), (1, 7, 64, 2, 1.0), (2, 257, 65, 3, 1.0),
                                                (1, 300, 300, 4, 8.0), (2, 512, 1029, 2, 1.0), (1, 33, 129, 1, 1.0)])
 def test_attention_dh128_shapes(dev, B, T, N, H, scale_up):
