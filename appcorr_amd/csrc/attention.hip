@@ -17,13 +17,14 @@
 // the LDS transpose read (ds_read_tr16_b64, its lane mapping described above the buffer-load
 // kernel).
 //
-// Query waves per workgroup and workgroups per (image, head) are chosen per shape (attn_shape): 4 to 12
-// waves at Dh = 64, up to 8 at Dh = 128. At the headline shape (T = 261: 8 full waves and a last wave of 5
+// Query waves per workgroup and workgroups per (image, head) are chosen per shape (attn_shape): 1 to 12
+// waves at Dh = 64, 4 to 8 at Dh = 128. At the headline shape (T = 261: 8 full waves and a last wave of 5
 // queries, 256 workgroups for B*H = 256, one per CU) the buffer-load kernel shares the last wave's key
 // tiles among 4 waves, so each workgroup runs 12. K/V tiles of 64 keys are staged in LDS with the next
 // tiles' global loads in flight during the current tile's MFMAs.
 #include <stdlib.h>
 
+#include <atomic>
 #include <type_traits>
 
 #include "common.hpp"
@@ -89,6 +90,14 @@ __device__ __forceinline__ float prob_row_sum(const bf16x8_t (&pf)[4]) {
     r[j] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(pf[j], pf[j], 6, 7), ones, r[j], false);
   }
   return xor32_sum((r[0] + r[1]) + (r[2] + r[3]));
+}
+
+// Slot of 16-byte chunk c in key row r of a tile: c ^ row_swz(r), so that 16 keys at one chunk (a K fragment
+// read) cover all banks. Dh = 128: also the 4 keys x 4 chunks that half a wave's V transpose read takes
+// (four consecutive keys differ in the chunk index above the 4 chunks).
+template <int DH>
+__device__ __forceinline__ int row_swz(int row) {
+  return DH == 128 ? ((row & 3) << 2) | ((row >> 2) & 3) : row & 7;
 }
 
 // MINW: fewest waves a launch of this instance uses (sizes the per-thread share of a K/V tile);
@@ -193,7 +202,7 @@ __global__ __launch_bounds__((DH == 64 ? kMaxWaves64 : kMaxWaves128) * 64) void 
       const int c = tid + i * nthreads;
       if (c < ITEMS) {
         const int kk = c / CPR, kc = c - kk * CPR;
-        const int slot = kk * KROWB + ((kc ^ (kk & (CPR - 1))) << 4);
+        const int slot = kk * KROWB + ((kc ^ row_swz<DH>(kk)) << 4);
         *reinterpret_cast<u32x4_t*>(ks + slot) = r.k[i];
         *reinterpret_cast<u32x4_t*>(vs + slot) = r.v[i];
       }
@@ -212,7 +221,7 @@ __global__ __launch_bounds__((DH == 64 ? kMaxWaves64 : kMaxWaves128) * 64) void 
 #pragma unroll
       for (int run = 0; run < 2; ++run) {
         const int key = 4 * g + (sl >> 2) + 8 * run;
-        voff[d][run] = KSTAGE + key * KROWB + (((dcol >> 3) ^ (key & (CPR - 1))) << 4) + ((dcol >> 2) & 1) * 8;
+        voff[d][run] = KSTAGE + key * KROWB + (((dcol >> 3) ^ row_swz<DH>(key)) << 4) + ((dcol >> 2) & 1) * 8;
       }
     }
   }
@@ -234,7 +243,7 @@ __global__ __launch_bounds__((DH == 64 ? kMaxWaves64 : kMaxWaves128) * 64) void 
         for (int kstep = 0; kstep < QK_STEPS; ++kstep) {
           const int ch = kstep * 2 + g;
           kf[kb][kstep] =
-              as_bf16x8(*reinterpret_cast<const uint4*>(ks + key * KROWB + ((ch ^ (key & (CPR - 1))) << 4)));
+              as_bf16x8(*reinterpret_cast<const uint4*>(ks + key * KROWB + ((ch ^ row_swz<DH>(key)) << 4)));
         }
       }
 #pragma unroll
@@ -383,15 +392,19 @@ __global__ __launch_bounds__((DH == 64 ? kMaxWaves64 : kMaxWaves128) * 64) void 
 
 
 // ------------------------------------------------------------------------------------------------
-// Dh = 64: K and V tiles reach LDS by buffer loads straight from the cache (no register staging), both
-// in their natural [key][dim] rows, NST stages deep. Waves 0..7 each load 8 rows of K and 8 rows of V
-// per tile (one 1 KB instruction each; with fewer than 8 waves, waves 0..3 load two such groups); keys past N fall outside the per-(image,
-// head) descriptors and load as zeros (their scores are masked). The A operand of O^T += V^T . P^T
+// K and V tiles reach LDS by buffer loads straight from the cache (no register staging), both in their
+// natural [key][dim] rows, NST stages deep. Each loader wave takes 1 KB row groups of K and of V (8 rows at
+// Dh = 64, 4 at Dh = 128), LPW of each per tile; keys past N fall outside the per-(image, head) descriptors
+// and load as zeros (their scores are masked). The A operand of O^T += V^T . P^T
 // comes from V's rows through the LDS transpose read: in each 16-lane group, source lane s addresses
 // 4 dims (8 bytes) of key k0 + s / 4 at dim c0 + 4 (s % 4), and lane j receives dim c0 + j for keys
-// k0 .. k0 + 3. Rows are 128 bytes; 16-byte chunk c of key row r sits in slot c ^ kv_swz(r) (below).
+// k0 .. k0 + 3. 16-byte chunk c of key row r sits in slot c ^ tile_swz(r) (below).
 // The arithmetic (MFMA order, softmax, P rounding) is that of sq_attention_kernel, so both give
 // bit-identical outputs.
+// Dh = 128, measured against the register-staged kernel (two stages, a barrier with nothing issued across
+// it, two-way bank conflicts of the V reads): 4 x 32 heads, 4101 of 4101 1343 -> 1100 us, 414 of 4101 150 ->
+// 128. The matrix cores are busy half of the cycles there and the VALU (softmax) half, and the clock falls
+// from 1.9 to 1.75 GHz as they overlap more.
 // ------------------------------------------------------------------------------------------------
 
 // Slot of 16-byte chunk `chunk` in 128-byte key row `row`: chunk ^ sw(row), sw a permutation of the
@@ -403,6 +416,15 @@ __device__ __forceinline__ int kv_swz(int row) {
   return m ^ ((m & 1) << 2);
 }
 __device__ __forceinline__ int kv_slot(int row, int chunk) { return row * 128 + ((chunk ^ kv_swz(row)) << 4); }
+// The same for 256-byte rows (Dh = 128).
+template <int DH>
+__device__ __forceinline__ int tile_swz(int row) {
+  return DH == 128 ? row_swz<128>(row) : kv_swz(row);
+}
+template <int DH>
+__device__ __forceinline__ int tile_slot(int row, int chunk) {
+  return row * DH * 2 + ((chunk ^ tile_swz<DH>(row)) << 4);
+}
 
 // light_split: 0, or kLightParts when the launch has one workgroup per (image, head) whose last
 // query wave is light; that wave's work is then done by kLightParts waves (the last ones), part p
@@ -413,15 +435,20 @@ __device__ __forceinline__ int kv_slot(int row, int chunk) { return row * 128 + 
 __host__ __device__ __forceinline__ int64_t kv_part_rows(int64_t T) { return (T + 3) & ~(int64_t)3; }
 __host__ __device__ __forceinline__ int64_t kv_part_stride(int64_t T) { return 2 * kv_part_rows(T) + 64 * T; }
 
-// LPW: K/V row groups a loader wave takes per tile: 1 (waves 0..7 load) with at least 8 waves, else 2
-// (waves 0..3).
-template <int NST, bool KVS, int LPW>
-__global__ __launch_bounds__((LPW == 1 ? kDmaMaxWaves : 8) * 64) void sq_attention_dma_kernel(
+// LW: loader waves, 8 (waves 0..7) in workgroups of at least 8 waves, else 4.
+// Dh = 128 has no light waves and no key parts; F8OUT as in sq_attention_kernel.
+template <int DH, int NST, bool KVS, int LW, bool F8OUT>
+__global__ __launch_bounds__((DH == 64 && LW == 8 ? kDmaMaxWaves : 8) * 64) void sq_attention_dma_kernel(
     const uint16_t* __restrict__ q, int64_t qrs, int T, const uint16_t* __restrict__ kv, int64_t kvb, int64_t kvn,
     int64_t kvkv, int64_t kvh, int N, float scale_log2, uint16_t* __restrict__ out, int64_t ors,
-    int waves_per_wg, int light_split, float* __restrict__ part_ws, int kv_parts) {
-  constexpr int DH = 64, QK_STEPS = 4, OB = 2;
-  constexpr int TILEB = kKeyTile * 128;  // one K (or V) tile: 64 rows of 128 bytes
+    int waves_per_wg, int light_split, float* __restrict__ part_ws, int kv_parts, uint8_t* __restrict__ out8,
+    const float* __restrict__ f8s) {
+  static_assert(DH == 64 || (DH == 128 && !KVS), "key parts are Dh = 64 only");
+  constexpr int QK_STEPS = DH / 16, OB = DH / 32;
+  constexpr int ROWB = 2 * DH, CPR = DH / 8;   // bytes and 16-byte chunks of a key row
+  constexpr int TILEB = kKeyTile * ROWB;       // one K (or V) tile
+  constexpr int RPI = 1024 / ROWB;             // rows of one load instruction
+  constexpr int LPW = kKeyTile / (RPI * LW);   // row groups (K and V each) a loader wave takes per tile
   constexpr int STAGE = 2 * TILEB;
   static_assert(NST >= 2, "stages");
   typedef short i16x4_t __attribute__((ext_vector_type(4)));
@@ -459,8 +486,9 @@ __global__ __launch_bounds__((LPW == 1 ? kDmaMaxWaves : 8) * 64) void sq_attenti
   const uint32_t bytes = (uint32_t)((int64_t)N * kvn * 2);
   const i32x4_t rsrc_k = make_buffer_rsrc(kbase, bytes);
   const i32x4_t rsrc_v = make_buffer_rsrc(kbase + kvkv, bytes);
-  const bool loader = wave < 8 / LPW;
-  const int lrow = 8 * wave + (lane >> 3);                  // tile row this lane loads (LPW = 2: and row + 32)
+  const bool loader = wave < LW;
+  const int lrow = RPI * wave + lane / CPR;  // tile row this lane loads, and rows RPI LW further on (same swizzle)
+  static_assert(RPI * LW % 16 == 0, "the swizzle repeats every 16 rows");
   const uint32_t tstep = (uint32_t)kKeyTile * (uint32_t)kvn * 2u;
   // Key tiles of this workgroup: [tb, tb + ntiles); tiles are numbered from tb in the loops below.
   int tb = 0, ntiles = (N + kKeyTile - 1) / kKeyTile;
@@ -469,17 +497,16 @@ __global__ __launch_bounds__((LPW == 1 ? kDmaMaxWaves : 8) * 64) void sq_attenti
     tb = kpart * per;
     ntiles = min(per, ntiles - tb);
   }
-  const uint32_t off0 = (uint32_t)lrow * (uint32_t)kvn * 2u + (uint32_t)(((lane & 7) ^ kv_swz(lrow)) << 4) +
+  const uint32_t off0 = (uint32_t)lrow * (uint32_t)kvn * 2u + (uint32_t)(((lane % CPR) ^ tile_swz<DH>(lrow)) << 4) +
                         (uint32_t)tb * tstep;
   auto issue = [&](int stage, int t) __attribute__((always_inline)) {
     if (loader) {
       unsigned char* base = smem + stage * STAGE + wave * 1024;
-      buffer_load_lds16(rsrc_k, base, off0 + (uint32_t)t * tstep);
-      buffer_load_lds16(rsrc_v, base + TILEB, off0 + (uint32_t)t * tstep);
-      if constexpr (LPW == 2) {  // rows 32 further on: the same swizzle
-        const uint32_t far = off0 + (uint32_t)t * tstep + 32u * (uint32_t)kvn * 2u;
-        buffer_load_lds16(rsrc_k, base + 4096, far);
-        buffer_load_lds16(rsrc_v, base + 4096 + TILEB, far);
+#pragma unroll
+      for (int i = 0; i < LPW; ++i) {
+        const uint32_t off = off0 + (uint32_t)t * tstep + (uint32_t)(i * RPI * LW) * (uint32_t)kvn * 2u;
+        buffer_load_lds16(rsrc_k, base + i * LW * 1024, off);
+        buffer_load_lds16(rsrc_v, base + i * LW * 1024 + TILEB, off);
       }
     }
   };
@@ -496,7 +523,7 @@ __global__ __launch_bounds__((LPW == 1 ? kDmaMaxWaves : 8) * 64) void sq_attenti
   // (the prologue's vmcnt waits then cover them as older loads). Full wave (T - q0 > 16): query
   // q0 + lane % 32, dims 16 ks + 8 (lane / 32) .. + 7; light wave: query q0 + lane % 16, dims
   // 32 ks + 8 (lane / 16) .. + 7, ks < 2.
-  const bool full_wave = T - q0 > 16;
+  const bool full_wave = DH == 128 ? active : T - q0 > 16;
   uint4 qraw[QK_STEPS];
   {
     const int qr = q0 + (full_wave ? l32 : (lane & 15));
@@ -577,7 +604,7 @@ __global__ __launch_bounds__((LPW == 1 ? kDmaMaxWaves : 8) * 64) void sq_attenti
     // address are compile-time offsets.
     int koff[QK_STEPS];
 #pragma unroll
-    for (int kstep = 0; kstep < QK_STEPS; ++kstep) koff[kstep] = kv_slot(l32, kstep * 2 + g);
+    for (int kstep = 0; kstep < QK_STEPS; ++kstep) koff[kstep] = tile_slot<DH>(l32, kstep * 2 + g);
     int voff[OB][2];
     {
       const int sl = lane & 15, hh = (lane >> 4) & 1;
@@ -585,8 +612,8 @@ __global__ __launch_bounds__((LPW == 1 ? kDmaMaxWaves : 8) * 64) void sq_attenti
       for (int db = 0; db < OB; ++db) {
         const int dcol = 32 * db + 16 * hh + 4 * (sl & 3);  // first of the 4 dims this lane addresses
         const int k1 = 4 * g + (sl >> 2);                   // key of k-step 0 (first run)
-        voff[db][0] = TILEB + kv_slot(k1, dcol >> 3) + ((dcol >> 2) & 1) * 8;
-        voff[db][1] = TILEB + kv_slot(k1 + 8, dcol >> 3) + ((dcol >> 2) & 1) * 8;
+        voff[db][0] = TILEB + tile_slot<DH>(k1, dcol >> 3) + ((dcol >> 2) & 1) * 8;
+        voff[db][1] = TILEB + tile_slot<DH>(k1 + 8, dcol >> 3) + ((dcol >> 2) & 1) * 8;
       }
     }
 
@@ -600,7 +627,7 @@ __global__ __launch_bounds__((LPW == 1 ? kDmaMaxWaves : 8) * 64) void sq_attenti
         bf16x8_t kf[QK_STEPS];
 #pragma unroll
         for (int kstep = 0; kstep < QK_STEPS; ++kstep)
-          kf[kstep] = as_bf16x8(*reinterpret_cast<const uint4*>(st + koff[kstep] + kb * 32 * 128));
+          kf[kstep] = as_bf16x8(*reinterpret_cast<const uint4*>(st + koff[kstep] + kb * 32 * ROWB));
         const f32x16_t zero = {};
         sc.s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[0], qf[0], zero, 0, 0, 0);
 #pragma unroll
@@ -657,9 +684,9 @@ __global__ __launch_bounds__((LPW == 1 ? kDmaMaxWaves : 8) * 64) void sq_attenti
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) i16x4_t*)(st + voff[db][0] + j * 16 * 128));
+              (__attribute__((address_space(3))) i16x4_t*)(st + voff[db][0] + j * 16 * ROWB));
           const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) i16x4_t*)(st + voff[db][1] + j * 16 * 128));
+              (__attribute__((address_space(3))) i16x4_t*)(st + voff[db][1] + j * 16 * ROWB));
           typedef short i16x8_t __attribute__((ext_vector_type(8)));
           const i16x8_t both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
           o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, both), pf[j], o[db], 0, 0, 0);
@@ -688,6 +715,19 @@ __global__ __launch_bounds__((LPW == 1 ? kDmaMaxWaves : 8) * 64) void sq_attenti
         for (int r4 = 0; r4 < 4; ++r4)
           *reinterpret_cast<f32x4_t*>(orow + d * 32 + 8 * r4 + 4 * g) =
               f32x4_t{o[d][4 * r4], o[d][4 * r4 + 1], o[d][4 * r4 + 2], o[d][4 * r4 + 3]};
+    } else if (F8OUT && active && qr < T) {
+      const float inv = 1.0f / l_i;
+      const float s8 = *f8s;
+      uint8_t* orow = out8 + ((int64_t)b * T + qr) * ors + (int64_t)h * DH;
+#pragma unroll
+      for (int d = 0; d < OB; ++d)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+          uint32_t w = 0;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w |= fp8_act_code(round_bf16(o[d][4 * r4 + e] * inv), s8) << (8 * e);
+          *reinterpret_cast<uint32_t*>(orow + d * 32 + 8 * r4 + 4 * g) = w;
+        }
     } else if (active && qr < T) {
       const float inv = 1.0f / l_i;
       uint16_t* orow = out + ((int64_t)b * T + qr) * ors + (int64_t)h * DH;
@@ -702,6 +742,10 @@ __global__ __launch_bounds__((LPW == 1 ? kDmaMaxWaves : 8) * 64) void sq_attenti
           *reinterpret_cast<bf16x4_t*>(orow + d * 32 + 8 * r4 + 4 * g) = w;
         }
     }
+  } else if constexpr (DH == 128) {  // an idle wave: loads and barriers only
+    int sa = 0, sb = 0;
+    auto none = [](auto&&...) {};
+    pipeline(sa, sb, none, none, BF{});
   } else {
     // ---- Light wave (<= 16 queries left, e.g. the 5 of T = 261 after 8 full waves): 16 queries on
     // v_mfma_f32_16x16x32_bf16, half the MFMA and softmax work of a full wave. 8 full waves and one
@@ -1049,13 +1093,29 @@ static double attn_wg_us(int64_t wgs, int64_t streams, int w, int waves, bool li
 static AttnShape attn_shape(int64_t B, int64_t T, int64_t H, int64_t Dh, int64_t N, bool offsets_fit) {
   AttnShape s{};
   const int64_t waves = cdiv(T, 32);
-  // Buffer-load kernel for Dh = 64 (its byte offsets must fit 31 bits); the register-staged kernel
-  // otherwise.
-  s.dma = Dh == 64 && offsets_fit;
+  // Buffer-load kernel when its byte offsets fit 31 bits; the register-staged kernel otherwise.
+  s.dma = offsets_fit;
   s.kv_parts = 1;
   if (!s.dma) {
     s.n_wg = cdiv(waves, Dh == 64 ? kMaxWaves64 : kMaxWaves128);
     s.w = (int)std::max<int64_t>(cdiv(waves, s.n_wg), kMinWaves);
+    return s;
+  }
+  if (Dh == 128) {
+    // One workgroup per CU (128 KB of LDS). A key tile takes about 1.2 us with one wave per SIMD and 1.7 to
+    // 1.9 with two (five to eight waves), measured over 17 .. 65 tiles; the fewest rounds of those wins.
+    // 1 x 32 heads, 200 queries of 1029 keys: two workgroups of four waves 25.4 us, one of seven 33.1;
+    // 3 x 32, 700 of 1029: five of five 65.6, three of eight 71.5.
+    double best = -1.0;
+    for (int w = kMinWaves; w <= kMaxWaves128; ++w) {
+      const int64_t n = cdiv(waves, w);
+      const double us = (double)cdiv(B * H * n, kNumCus) * (w == kMinWaves ? 1.2 : 1.7 + 0.05 * (w - 5));
+      if (best >= 0.0 && us >= best) continue;
+      best = us;
+      s.n_wg = n;
+      s.w = (int)std::max<int64_t>(cdiv(waves, n), kMinWaves);
+    }
+    s.waves = s.w;
     return s;
   }
   // Query waves per workgroup: the shape of least modelled time among 1 to 4 (the finest fill of the CUs) and
@@ -1106,6 +1166,36 @@ static int64_t attn_workspace_elems(int64_t B, int64_t T, int64_t H, int kv_part
   return kv_parts > 1 ? B * H * kv_parts * kv_part_stride(T) : 0;
 }
 
+// Dh = 128 on the buffer-load kernel: four stages of K and V tiles are 128 KB of LDS.
+template <bool F8OUT>
+static int launch_attention128(const AttnShape& s, const uint16_t* q, int64_t qrs, int64_t B, int64_t T, int64_t H,
+                               const uint16_t* kv, int64_t kvb, int64_t kvn, int64_t kvkv, int64_t kvh, int64_t N,
+                               float scale_log2, uint16_t* out, int64_t ors, uint8_t* out8, const float* f8s,
+                               const char* what, oudjat_stream_t stream) {
+  constexpr int lds = kAttnStages * 2 * kKeyTile * 256;
+  static std::atomic<uint8_t> attr_set[64] = {};
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return set_error(OUDJAT_ERR_HIP, "%s: hipGetDevice: %s", what, hipGetErrorString(e));
+  if (!attr_set[dev & 63].load(std::memory_order_acquire)) {
+    for (const void* fn : {(const void*)sq_attention_dma_kernel<128, kAttnStages, false, 8, F8OUT>,
+                           (const void*)sq_attention_dma_kernel<128, kAttnStages, false, 4, F8OUT>}) {
+      e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+      if (e != hipSuccess) return set_error(OUDJAT_ERR_HIP, "%s: hipFuncSetAttribute: %s", what, hipGetErrorString(e));
+    }
+    attr_set[dev & 63].store(1, std::memory_order_release);
+  }
+  const dim3 grid((unsigned)s.n_wg, (unsigned)H, (unsigned)B);
+  hipStream_t st = as_stream(stream);
+  if (s.w >= 8)
+    sq_attention_dma_kernel<128, kAttnStages, false, 8, F8OUT><<<grid, s.w * 64, lds, st>>>(
+        q, qrs, (int)T, kv, kvb, kvn, kvkv, kvh, (int)N, scale_log2, out, ors, s.w, 0, nullptr, 1, out8, f8s);
+  else
+    sq_attention_dma_kernel<128, kAttnStages, false, 4, F8OUT><<<grid, s.w * 64, lds, st>>>(
+        q, qrs, (int)T, kv, kvb, kvn, kvkv, kvh, (int)N, scale_log2, out, ors, s.w, 0, nullptr, 1, out8, f8s);
+  return check_launch(what);
+}
+
 static int sparse_query_attention_impl(const uint16_t* q, int64_t qrs, int64_t B, int64_t T, int64_t H, int64_t Dh,
                                        const uint16_t* kv, int64_t kvb, int64_t kvn, int64_t kvkv, int64_t kvh,
                                        int64_t N, float scale, uint16_t* out, int64_t ors, float* workspace,
@@ -1130,8 +1220,8 @@ static int sparse_query_attention_impl(const uint16_t* q, int64_t qrs, int64_t B
   dim3 grid((unsigned)s.n_wg, (unsigned)H, (unsigned)B);
   hipStream_t st = as_stream(stream);
   if (lse) {
-    // The register-staged kernel with the row log-sum-exp (at Dh = 128 the kernel every call runs;
-    // at Dh = 64 its output equals the buffer-load kernel's on every row of a full query wave).
+    // The register-staged kernel with the row log-sum-exp (its output equals the buffer-load kernel's, at
+    // Dh = 64 on every row of a full query wave).
     OUDJAT_REQUIRE(aligned(lse, 4), OUDJAT_ERR_UNSUPPORTED_LAYOUT, "sparse_query_attention: lse alignment");
     const size_t lds = 2 * 2 * (size_t)kKeyTile * Dh * 2;
     if (Dh == 128)
@@ -1145,6 +1235,9 @@ static int sparse_query_attention_impl(const uint16_t* q, int64_t qrs, int64_t B
           q, qrs, (int)T, kv, kvb, kvn, kvkv, kvh, (int)N, scale_log2, out, ors, w, lse);
     return check_launch("sparse_query_attention (lse)");
   }
+  if (s.dma && Dh == 128)
+    return launch_attention128<false>(s, q, qrs, B, T, H, kv, kvb, kvn, kvkv, kvh, N, scale_log2, out, ors, nullptr,
+                                      nullptr, "sparse_query_attention", stream);
   if (s.dma) {
     const size_t lds_dma = (size_t)kAttnStages * 2 * kKeyTile * 128;
     static_assert((size_t)kAttnStages * 2 * kKeyTile * 128 <= 64 * 1024, "needs no larger-LDS attribute");
@@ -1155,11 +1248,11 @@ static int sparse_query_attention_impl(const uint16_t* q, int64_t qrs, int64_t B
                      attn_workspace_elems(B, T, H, s.kv_parts) <= workspace_elems;
     auto launch_kv = [&](auto kvs_c, dim3 g, float* ws, int parts) {
       if (s.waves >= 8)
-        sq_attention_dma_kernel<kAttnStages, decltype(kvs_c)::value, 1><<<g, threads, lds_dma, st>>>(
-            q, qrs, (int)T, kv, kvb, kvn, kvkv, kvh, (int)N, scale_log2, out, ors, w, split, ws, parts);
+        sq_attention_dma_kernel<64, kAttnStages, decltype(kvs_c)::value, 8, false><<<g, threads, lds_dma, st>>>(
+            q, qrs, (int)T, kv, kvb, kvn, kvkv, kvh, (int)N, scale_log2, out, ors, w, split, ws, parts, nullptr, nullptr);
       else
-        sq_attention_dma_kernel<kAttnStages, decltype(kvs_c)::value, 2><<<g, threads, lds_dma, st>>>(
-            q, qrs, (int)T, kv, kvb, kvn, kvkv, kvh, (int)N, scale_log2, out, ors, w, split, ws, parts);
+        sq_attention_dma_kernel<64, kAttnStages, decltype(kvs_c)::value, 4, false><<<g, threads, lds_dma, st>>>(
+            q, qrs, (int)T, kv, kvb, kvn, kvkv, kvh, (int)N, scale_log2, out, ors, w, split, ws, parts, nullptr, nullptr);
     };
     if (kvs) {
       launch_kv(std::true_type{}, dim3((unsigned)(s.n_wg * s.kv_parts), (unsigned)H, (unsigned)B), workspace, s.kv_parts);
@@ -1249,12 +1342,15 @@ extern "C" int oudjat_sparse_query_attention_fp8(const uint16_t* q, int64_t qrs,
                  "4-byte aligned output rows required");
   OUDJAT_REQUIRE(B <= 65535 && H <= 65535 && N < ((int64_t)1 << 30) && T < ((int64_t)1 << 30), OUDJAT_ERR_TOO_LARGE,
                  "sparse_query_attention_fp8: too large");
-  const AttnShape s = attn_shape(B, T, H, Dh, N, true);
+  const AttnShape s = attn_shape(B, T, H, Dh, N, N * kvn * 2 < ((int64_t)1 << 31));
+  const float scale_log2 = scale * 1.4426950408889634f;
+  if (s.dma)
+    return launch_attention128<true>(s, q, qrs, B, T, H, kv, kvb, kvn, kvkv, kvh, N, scale_log2, nullptr, ors, out,
+                                     act_inv_scale, "sparse_query_attention_fp8", stream);
   dim3 grid((unsigned)s.n_wg, (unsigned)H, (unsigned)B);
   const size_t lds = 2 * 2 * (size_t)kKeyTile * Dh * 2;
   sq_attention_kernel<128, kMinWaves, false, false, true><<<grid, s.w * 64, lds, as_stream(stream)>>>(
-      q, qrs, (int)T, kv, kvb, kvn, kvkv, kvh, (int)N, scale * 1.4426950408889634f, nullptr, ors, s.w, nullptr, out,
-      act_inv_scale);
+      q, qrs, (int)T, kv, kvb, kvn, kvkv, kvh, (int)N, scale_log2, nullptr, ors, s.w, nullptr, out, act_inv_scale);
   return check_launch("sparse_query_attention_fp8");
 }
 

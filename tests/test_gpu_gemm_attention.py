@@ -526,6 +526,28 @@ def test_attention_launch_shapes(dev, B, T, N, H):
     _check_attention(got.cpu(), qb, kv, D ** -0.5, o64.transpose(1, 2).reshape(B * T, H * D), f"shape {B},{T},{N},{H}")
 
 
+@pytest.mark.parametrize("B,T,N,H,pad", [(1, 200, 261, 7, 0), (2, 257, 65, 3, 8), (1, 128, 64, 9, 0), (3, 700, 129, 5, 0),
+                                         (16, 257, 193, 16, 0), (1, 1, 1, 1, 0), (1, 40, 130, 1, 1 << 23)])
+def test_attention_dh128_buffer_loads(dev, B, T, N, H, pad):
+    """Dh = 128: four and eight loader waves, one to 256 pairs, one key past a tile, padded key rows; the
+    last case's key rows lie past the 31-bit byte offsets (the register-staged kernel). The output equals
+    the register-staged kernel's (the log-sum-exp entry) bit for bit, and that one is within the bound of
+    the float64 reference."""
+    D = 128
+    print(f"attention dh128 {B},{T},{N},{H} pad {pad}", flush=True)
+    q = _rand((B * T, H, D), 48).to(dev)
+    store = torch.empty((B, N, 2 * H * D + pad), device=dev, dtype=torch.bfloat16)
+    kv = store[:, :, : 2 * H * D].unflatten(2, (2, H, D))
+    kv.copy_(_rand((B, N, 2, H, D), 49).to(dev))
+    got = K.sparse_query_attention(q, kv, T, D ** -0.5)
+    staged = K.sparse_query_attention(q, kv, T, D ** -0.5, lse=torch.empty((B, H, T), device=dev))
+    assert_bits_equal(got.cpu(), staged.cpu(), "register-staged kernel")
+    qb = q.cpu().reshape(B, T, H, D).transpose(1, 2)
+    kvc = kv.cpu()
+    o64 = F64.sdpa(qb, kvc[:, :, 0].transpose(1, 2), kvc[:, :, 1].transpose(1, 2), D ** -0.5)
+    _check_attention(got.cpu(), qb, kvc, D ** -0.5, o64.transpose(1, 2).reshape(B * T, H * D), f"dh128 {B},{T},{N},{H}")
+
+
 @pytest.mark.parametrize("B,T,N,H,scale_up", [(4, 414, 4101, 32, 1.0), (1, 7, 64, 2, 1.0), (2, 257, 65, 3, 1.0),
                                                (1, 300, 300, 4, 8.0), (2, 512, 1029, 2, 1.0), (1, 33, 129, 1, 1.0)])
 def test_attention_dh128_shapes(dev, B, T, N, H, scale_up):
