@@ -39,6 +39,11 @@ EPI_RAW_BF16 = 16  # flag: round the accumulator to bf16 before the scale and bi
 
 QUERY_PROB_NOALLOC_MAX = 1 << 20  # OUDJAT_QUERY_PROB_NOALLOC_MAX: fp32 elements of the no-alloc scratch array
 
+FUSION_SERVER = 0
+FUSION_ADD = 1
+FUSION_MULTIPLY = 2
+FUSION_MOBILE = 3
+FUSION_GEO_MEAN = 4
 IMPORTANCE_L2 = 0
 IMPORTANCE_ENERGY = 1
 IMPORTANCE_RMS = 2
@@ -71,6 +76,10 @@ SIGNATURES: dict[str, list] = {
     "oudjat_selftest": [_p],
     "oudjat_patch_importance": [_p, _i64, _i64, _i64, _i32, _p, _p],
     "oudjat_topk_plan": [_p, _i64, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _p],
+    "oudjat_plan_scores": [_p, _i64, _i64, _f32, _p, _i64, _i64, _i64, _f32, _i32, _p, _i64, _i64, _i64, _i64, _p, _p,
+                           _p, _p],
+    "oudjat_topk_plan_scores": [_p, _i64, _i64, _f32, _p, _i64, _i64, _i64, _f32, _i32, _p, _i64, _i64, _i64, _i64, _p,
+                                _p, _p, _i64, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p],
     "oudjat_threshold_keep": [_p, _i64, _i64, _i64, _f32, _p, _p, _p],
     "oudjat_patch_attention_prob": [_p, _i64, _i64, _i64, _i64, _i64, _p, _i64, _i64, _i64, _f32, _i32, _p, _p, _i64,
                                     _p],

@@ -584,11 +584,16 @@ class SelfAttentionBlock(nn.Module):
         for k, t in zip(keys, torch._foreach_add(prev, vals)):
             cache_feature[k] = t
 
-    @annotate("build_packed_query_state")
-    def _build_query_plan(self, x: Tensor, dindice: Tensor, rope, cache_feature: Dict, tag: str, kw: dict,
-                          num_pretokens: int) -> PartialTokenQueryPlan:
+    @staticmethod
+    def _keep_count(kw: dict, Pn: int) -> int:
+        ratio = float(kw["token_keep_ratio"])
+        return Pn if ratio >= 1.0 else min(int(Pn * ratio), Pn)
+
+    def _elementwise_scores(self, x: Tensor, dindice_patches: Tensor, cache_feature: Dict, tag: str, kw: dict,
+                            num_pretokens: int):
+        """(server, mobile or None, combined) candidate scores with torch's own gathers and elementwise steps:
+        score types and layouts the plan kernels do not read (_candidate_scores)."""
         B, N, _ = x.shape
-        dindice_patches = dindice[:, num_pretokens:]
         mobile = None
         if kw["mobile_pscore"] != "none" and kw["mobile_pscore_weight"] != 0.0:
             mobile = self._resolve_mobile_patch_scores(kw["mobile_pscore"], kw["mobile_pscore_hint"], dindice_patches,
@@ -606,23 +611,65 @@ class SelfAttentionBlock(nn.Module):
         else:
             combined = self._combine_patch_scores(server, kw["server_pscore_weight"], mobile,
                                                   kw["mobile_pscore_weight"], kw["pscore_fusion"])
+        return server, mobile, combined
+
+    def _candidate_scores(self, B: int, N: int, cache_feature: Dict, tag: str, kw: dict, dind: Tensor,
+                          num_pretokens: int) -> "K.CandidateScores | None":
+        """The same scores as the plan kernels' source, or None where they do not apply: scores that are not
+        fp32 rows on dindice's device, a hint of a width that the elementwise path refuses, no candidates."""
+        hint, fusion, hint_off = None, _lib.FUSION_SERVER, 0
+        if (kw["mobile_pscore"] in self._MOBILE_HINT_PSCORE_ALIASES and kw["mobile_pscore_weight"] != 0.0
+                and kw["mobile_pscore_hint"] is not None):
+            hint = kw["mobile_pscore_hint"]
+            if hint.dim() != 2 or hint.shape[0] != B or hint.shape[1] not in (N - num_pretokens, N):
+                return None
+            hint_off = num_pretokens if hint.shape[1] == N - num_pretokens else 0
+            fusion = {"multiply": _lib.FUSION_MULTIPLY, "geo_mean": _lib.FUSION_GEO_MEAN}.get(kw["pscore_fusion"],
+                                                                                             _lib.FUSION_ADD)
+            if kw["server_pscore_weight"] == 0.0 and kw["mobile_pscore_weight"] == 1.0 and fusion == _lib.FUSION_ADD:
+                fusion = _lib.FUSION_MOBILE  # 0 * 0 + 1 * mobile is mobile itself
+        elif kw["mobile_pscore"] != "none" and kw["mobile_pscore_weight"] != 0.0 and \
+                kw["mobile_pscore"] not in self._MOBILE_HINT_PSCORE_ALIASES:
+            return None
+        server = None
+        if kw["server_pscore_weight"] != 0.0:
+            server = self._resolve_server_token_scores(cache_feature, tag, kw["server_pscore"])
+        if dind.dtype != torch.long or dind.dim() != 2 or dind.shape[1] <= num_pretokens or not (
+                dind.is_cuda and K.CandidateScores.takes(server, B, dind.device)
+                and K.CandidateScores.takes(hint, B, dind.device)):
+            return None
+        return K.CandidateScores(server, kw["server_pscore_weight"], hint, hint_off, kw["mobile_pscore_weight"], fusion)
+
+    @annotate("build_packed_query_state")
+    def _build_query_plan(self, x: Tensor, dindice: Tensor, rope, cache_feature: Dict, tag: str, kw: dict,
+                          num_pretokens: int) -> PartialTokenQueryPlan:
+        B, N, _ = x.shape
+        dindice_patches = dindice[:, num_pretokens:]
+        Pn = dindice_patches.shape[1]
+        thres = kw["token_keep_thres"]
         cvm = kw.get("candidate_valid_mask")
+        dind = dindice.contiguous()
+        valid = tp = None
+        src = self._candidate_scores(B, N, cache_feature, tag, kw, dind, num_pretokens)
+        if src is not None and thres is None and cvm is None:   # scores and top-k plan in one launch
+            tp, valid, server, mobile, combined = K.topk_plan_scores(src, self._keep_count(kw, Pn), dind, num_pretokens,
+                                                                     N)
+        elif src is not None:
+            server, mobile, combined = K.plan_scores(src, dind, num_pretokens)
+        else:
+            server, mobile, combined = self._elementwise_scores(x, dindice_patches, cache_feature, tag, kw,
+                                                                num_pretokens)
         if cvm is not None:
             combined = combined.masked_fill(~cvm.to(combined.device), float("-inf"))
-        Pn = dindice_patches.shape[1]
         scores = combined.to(torch.float32).contiguous()
-        thres = kw["token_keep_thres"]
         all_valid = True
-        if thres is None:                                       # top-k (block.py:377-394, 397-490)
-            ratio = float(kw["token_keep_ratio"])
-            k = Pn if ratio >= 1.0 else min(int(Pn * ratio), Pn)
-            tp = K.topk_plan(scores, k, dindice.contiguous(), num_pretokens, N)
-            valid = None
+        if tp is not None:
+            pass
+        elif thres is None:                                     # top-k (block.py:377-394, 397-490)
+            tp = K.topk_plan(scores, self._keep_count(kw, Pn), dind, num_pretokens, N)
         elif kw["token_keep_cap"] > 0:                          # fixed width, sync-free (block.py:492-560)
             width = max(0, min(int(kw["token_keep_cap"]), Pn))
-            tp = K.threshold_plan(scores, thres, dindice.contiguous(), num_pretokens, width, padded=False,
-                                  num_tokens=N)
-            valid = None
+            tp = K.threshold_plan(scores, thres, dind, num_pretokens, width, padded=False, num_tokens=N)
         else:                                                   # padded (block.py:562-621)
             # The width is the largest kept count, read back to the host as the reference's .item()
             # does (block.py:570); rows past an image's count are not queries.
@@ -632,17 +679,19 @@ class SelfAttentionBlock(nn.Module):
             if num_pretokens == 0 and width > 0 and int(counts_h.min()) == 0:
                 raise NotImplementedError("padded threshold plan with num_pretokens == 0: an image that keeps no "
                                           "candidate has no row to stand in for its padding; set token_keep_cap")
-            tp = K.threshold_plan(scores, thres, dindice.contiguous(), num_pretokens, width, padded=True,
-                                  num_tokens=N)
+            tp = K.threshold_plan(scores, thres, dind, num_pretokens, width, padded=True, num_tokens=N)
             valid = tp.query_valid
             all_valid = bool(B <= 1 or valid.numel() == 0 or bool((counts_h == width).all()))
         T = tp.update_indice.shape[1]
+        # slots 0 .. T - 1: the first image's rows of a top-k plan (a threshold plan may repeat rows)
+        slots = (tp.active_pos_idx[:T] if thres is None and B > 0
+                 else torch.arange(T, device=x.device, dtype=torch.long))
         if valid is None:
             valid = torch.ones((B, T), device=x.device, dtype=torch.bool)
         qs = PackedQueryState(
             active_batch_idx=tp.active_batch_idx, active_pos_idx=tp.active_pos_idx,
             active_token_idx=tp.active_token_idx, query_valid_mask=valid,
-            active_query_pos_padded=torch.arange(T, device=x.device, dtype=torch.long).unsqueeze(0).expand(B, -1),
+            active_query_pos_padded=slots.unsqueeze(0).expand(B, -1),
             active_query_mask=valid, all_valid=all_valid, active_patch_mask=tp.active_patch_mask,
             active_rope_idx=tp.active_rope_idx, row_slot=tp.row_slot)
         keep = tp.keep_mask

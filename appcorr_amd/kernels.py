@@ -402,22 +402,82 @@ def topk_plan(scores: torch.Tensor, k: int, dindice: torch.Tensor, num_pretokens
     _require(dindice.shape[0] == B and dindice.shape[1] == num_pretokens + Pn, "topk_plan: dindice shape mismatch")
     k = int(k)
     _require(0 <= k <= Pn, f"topk_plan: k={k} outside [0, {Pn}]")
-    T = num_pretokens + k
-    dev = scores.device
-    upd = torch.empty((B, T), device=dev, dtype=torch.long)
-    abat = torch.empty((B * T,), device=dev, dtype=torch.long)
-    apos = torch.empty_like(abat)
-    atok = torch.empty_like(abat)
-    pmask = torch.empty((B * T,), device=dev, dtype=torch.bool)
-    ridx = torch.empty_like(abat)
-    keep = torch.empty((B, Pn), device=dev, dtype=torch.bool)
-    slot = None
-    if num_tokens is not None:
-        slot = torch.empty((B, int(num_tokens)), device=dev, dtype=torch.int32)
+    tp = _empty_topk_plan(B, Pn, num_pretokens + k, num_tokens, scores.device)
     _launch("topk_plan", scores, "oudjat_topk_plan", _ptr(scores), B, Pn, scores.stride(0), k, _ptr(dindice), dindice.stride(0),
-         num_pretokens, 0 if num_tokens is None else int(num_tokens), _ptr(upd), _ptr(abat), _ptr(apos), _ptr(atok),
-         _ptr(pmask), _ptr(ridx), _ptr(keep), _ptr(slot), _stream(scores))
-    return TopkPlan(upd, abat, apos, atok, pmask, ridx, keep, slot)
+         num_pretokens, 0 if num_tokens is None else int(num_tokens), _ptr(tp.update_indice), _ptr(tp.active_batch_idx),
+         _ptr(tp.active_pos_idx), _ptr(tp.active_token_idx), _ptr(tp.active_patch_mask), _ptr(tp.active_rope_idx),
+         _ptr(tp.keep_mask), _ptr(tp.row_slot), _stream(scores))
+    return tp
+
+
+def _empty_topk_plan(B: int, Pn: int, T: int, num_tokens: int | None, dev: torch.device) -> TopkPlan:
+    abat = torch.empty((B * T,), device=dev, dtype=torch.long)
+    return TopkPlan(
+        update_indice=torch.empty((B, T), device=dev, dtype=torch.long), active_batch_idx=abat,
+        active_pos_idx=torch.empty_like(abat), active_token_idx=torch.empty_like(abat),
+        active_patch_mask=torch.empty((B * T,), device=dev, dtype=torch.bool), active_rope_idx=torch.empty_like(abat),
+        keep_mask=torch.empty((B, Pn), device=dev, dtype=torch.bool),
+        row_slot=None if num_tokens is None else torch.empty((B, int(num_tokens)), device=dev, dtype=torch.int32))
+
+
+@dataclass
+class CandidateScores:
+    """Where the candidates' scores come from (oudjat_plan_scores): the per-token server score [B, n] and the
+    client's hint [B, n] (either may be None; hint column t - hint_offset is token t), their weights and the
+    fusion."""
+    server: torch.Tensor | None
+    server_weight: float
+    hint: torch.Tensor | None
+    hint_offset: int
+    mobile_weight: float
+    fusion: int
+
+    @staticmethod
+    def takes(t: torch.Tensor | None, B: int, dev: torch.device) -> bool:
+        """A score tensor the kernels read: fp32 [>= B, n] on `dev`, contiguous rows, not empty."""
+        return t is None or (t.dtype == torch.float32 and t.dim() == 2 and t.shape[0] >= B and t.numel() > 0
+                             and t.device == dev and (t.shape[1] == 1 or t.stride(1) == 1))
+
+    def _args(self, dindice: torch.Tensor, num_pretokens: int):
+        B, Pn = dindice.shape[0], dindice.shape[1] - num_pretokens
+        _require_cuda(dindice)
+        _require(self.takes(self.server, B, dindice.device) and self.takes(self.hint, B, dindice.device),
+                 "plan scores: server and hint must be fp32 [B, n] with contiguous rows on dindice's device")
+        _require(dindice.dtype == torch.long and dindice.dim() == 2 and dindice.stride(1) == 1 and Pn > 0 and B > 0,
+                 "plan scores: dindice must be [B, pre + P] int64 with contiguous rows, P > 0")
+        dev = dindice.device
+        server = torch.empty((B, Pn), device=dev, dtype=torch.float32)
+        mobile = None if self.hint is None else torch.empty_like(server)
+        combined = mobile if self.fusion == _lib.FUSION_MOBILE else torch.empty_like(server)
+        sv, ht = self.server, self.hint
+        args = (_ptr(sv), 0 if sv is None else sv.stride(0), 0 if sv is None else sv.shape[1], self.server_weight,
+                _ptr(ht), 0 if ht is None else ht.stride(0), 0 if ht is None else ht.shape[1], self.hint_offset,
+                self.mobile_weight, self.fusion, _ptr(dindice), dindice.stride(0), num_pretokens, B, Pn, _ptr(server),
+                _ptr(mobile), None if combined is mobile else _ptr(combined))
+        return args, server, mobile, combined
+
+
+def plan_scores(src: CandidateScores, dindice: torch.Tensor, num_pretokens: int):
+    """The candidates' (server, mobile or None, combined) scores [B, P] in one launch (block.py:638-687):
+    bit for bit the gathers and elementwise steps. With FUSION_MOBILE combined is mobile."""
+    args, server, mobile, combined = src._args(dindice, num_pretokens)
+    _launch("plan_scores", dindice, "oudjat_plan_scores", *args, _stream(dindice))
+    return server, mobile, combined
+
+
+def topk_plan_scores(src: CandidateScores, k: int, dindice: torch.Tensor, num_pretokens: int, num_tokens: int):
+    """plan_scores and topk_plan of the combined scores in one launch: (plan, query_valid [B, T] all True,
+    server, mobile, combined)."""
+    args, server, mobile, combined = src._args(dindice, num_pretokens)
+    B, Pn = combined.shape
+    k = int(k)
+    _require(0 <= k <= Pn, f"topk_plan: k={k} outside [0, {Pn}]")
+    tp = _empty_topk_plan(B, Pn, num_pretokens + k, num_tokens, dindice.device)
+    valid = torch.empty((B, num_pretokens + k), device=dindice.device, dtype=torch.bool)
+    _launch("topk_plan", dindice, "oudjat_topk_plan_scores", *args, k, int(num_tokens), _ptr(tp.update_indice),
+            _ptr(tp.active_batch_idx), _ptr(tp.active_pos_idx), _ptr(tp.active_token_idx), _ptr(tp.active_patch_mask),
+            _ptr(tp.active_rope_idx), _ptr(tp.keep_mask), _ptr(tp.row_slot), _ptr(valid), _stream(dindice))
+    return tp, valid, server, mobile, combined
 
 
 @dataclass

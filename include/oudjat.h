@@ -142,6 +142,37 @@ int oudjat_topk_plan(const float* scores, int64_t B, int64_t P, int64_t score_st
                      uint8_t* active_patch_mask, int64_t* active_rope_idx, uint8_t* keep_mask,
                      int32_t* row_slot, oudjat_stream_t stream);
 
+/* Rows 2+3 -- candidate scores from the cached server score and the client's hint,
+ * _resolve_server_token_scores / _resolve_mobile_patch_scores / _combine_patch_scores
+ * (appcorr/models/dinov3/layers/block.py:638-687, 862-940): candidate p of image b is token t =
+ * dindice[b, num_pre + p]; server_sel = server[b, t] (0 when server is NULL), mobile_sel =
+ * hint[b, t - hint_offset] (NULL only with OUDJAT_FUSION_SERVER); combined by `fusion`, every operation
+ * rounded to fp32 by itself. A token outside a score row scores NaN. server [B, server_n], hint
+ * [B, hint_n] fp32 (row strides *_stride_b); server_sel, mobile_sel, combined [B, P] fp32, each may be NULL. */
+enum {
+  OUDJAT_FUSION_SERVER = 0,   /* server_w * server_sel */
+  OUDJAT_FUSION_ADD = 1,      /* server_w * server_sel + mobile_w * mobile_sel */
+  OUDJAT_FUSION_MULTIPLY = 2, /* (server_w * server_sel) * (mobile_w * mobile_sel) */
+  OUDJAT_FUSION_MOBILE = 3,   /* mobile_sel */
+  OUDJAT_FUSION_GEO_MEAN = 4  /* sqrt(max(OUDJAT_FUSION_MULTIPLY, 0)), NaN kept */
+};
+int oudjat_plan_scores(const float* server, int64_t server_stride_b, int64_t server_n, float server_w,
+                       const float* hint, int64_t hint_stride_b, int64_t hint_n, int64_t hint_offset,
+                       float mobile_w, int fusion, const int64_t* dindice, int64_t dindice_stride_b,
+                       int64_t num_pre, int64_t B, int64_t P, float* server_sel, float* mobile_sel,
+                       float* combined, oudjat_stream_t stream);
+
+/* oudjat_plan_scores and oudjat_topk_plan of its combined scores in one launch; query_valid [B, T]
+ * (1 byte) is set to 1. Limits as oudjat_topk_plan. */
+int oudjat_topk_plan_scores(const float* server, int64_t server_stride_b, int64_t server_n, float server_w,
+                            const float* hint, int64_t hint_stride_b, int64_t hint_n, int64_t hint_offset,
+                            float mobile_w, int fusion, const int64_t* dindice, int64_t dindice_stride_b,
+                            int64_t num_pre, int64_t B, int64_t P, float* server_sel, float* mobile_sel,
+                            float* combined, int64_t k, int64_t num_tokens, int64_t* update_indice,
+                            int64_t* active_batch_idx, int64_t* active_pos_idx, int64_t* active_token_idx,
+                            uint8_t* active_patch_mask, int64_t* active_rope_idx, uint8_t* keep_mask,
+                            int32_t* row_slot, uint8_t* query_valid, oudjat_stream_t stream);
+
 /* Threshold selection (next-rank row f3) -- the kept mask and per-image kept count of
  * _select_patch_keep_mask's threshold branch (appcorr/models/dinov3/layers/block.py:374-376):
  * keep_mask[b, p] = scores[b, p] >= thres, compared in fp32 as torch compares an fp32 tensor with a

@@ -112,3 +112,60 @@ def test_plan_stats_masked_and_special_values(dev):
     s3[1, np.flatnonzero(keep[1])[:2]] = -np.inf  # only kept -inf: kept mass -inf
     _check_stats(dev, s3, keep)
     _check_stats(dev, np.zeros((2, 0), dtype=np.float32), np.zeros((2, 0), dtype=bool))
+
+
+@pytest.mark.parametrize("B,P,gh,k,fusion,server,hint", [
+    (2, 64, 100, 16, "SERVER", "fp", None), (16, 1024, 1024, 256, "GEO_MEAN", "fp", "patches"),
+    (3, 759, 759, 379, "ADD", "fp", "tokens"), (1, 1, 5, 1, "MULTIPLY", "fp", "patches"),
+    (4, 1025, 4096, 0, "MOBILE", None, "patches"), (2, 3000, 3000, 3000, "ADD", None, "tokens"),
+    (2, 300, 300, 75, "GEO_MEAN", "wide", "patches")])
+def test_plan_scores_equal_elementwise_steps(dev, B, P, gh, k, fusion, server, hint):
+    """The candidate scores formed by the plan kernels equal torch's gathers and elementwise steps bit for bit
+    (negative scores, infinities, NaN, -0, products that would contract to a fused multiply-add, strided score
+    rows), and the fused top-k plan equals topk_plan of those scores; query_valid is all ones."""
+    from appcorr_amd import _lib
+    rng = np.random.default_rng(B * P + k)
+    npre, N = 5, gh + 5
+    cand = np.stack([np.sort(rng.permutation(gh)[:P]) + npre for _ in range(B)])
+    dind = torch.from_numpy(np.concatenate([np.broadcast_to(np.arange(npre), (B, npre)), cand], 1).astype(np.int64)).to(dev)
+
+    def rows(n):
+        v = (rng.standard_normal((B, n)) * 10.0 ** rng.integers(-3, 3, (B, n))).astype(np.float32)
+        special = np.array([np.inf, -np.inf, np.nan, -0.0, 0.0, 3e38, 1e-45], np.float32)
+        at = rng.permutation(v.size)[: v.size // 16]
+        v.ravel()[at] = special[rng.integers(0, special.size, at.size)]
+        return torch.from_numpy(v).to(dev)
+
+    sv = None if server is None else rows(N) if server == "fp" else rows(3 * N)[:, N: 2 * N]
+    off = 0 if hint == "tokens" else npre
+    ht = None if hint is None else rows(N - off)
+    ws, wm = (0.0 if sv is None else 0.7), (1.0 if fusion == "MOBILE" else 1.3)
+    src = K.CandidateScores(sv, ws, ht, off, wm, getattr(_lib, "FUSION_" + fusion))
+    idx = dind[:, npre:]
+    s_ref = torch.zeros((B, P), device=dev) if sv is None else sv.gather(1, idx)
+    m_ref = None if ht is None else ht.gather(1, idx - off)
+    c_ref = ws * s_ref
+    if fusion == "MOBILE":
+        c_ref = m_ref
+    elif fusion != "SERVER":
+        term = wm * m_ref
+        c_ref = c_ref + term if fusion == "ADD" else c_ref * term
+        if fusion == "GEO_MEAN":
+            c_ref = torch.sqrt(torch.clamp(c_ref, min=0.0))
+
+    def same(a, b, what):
+        a, b = a.cpu().numpy(), b.cpu().numpy()
+        nan = np.isnan(b)
+        assert (np.isnan(a) == nan).all() and (a[~nan] == b[~nan]).all(), what
+
+    tp, valid, *fused = K.topk_plan_scores(src, k, dind, npre, N)
+    for got in (K.plan_scores(src, dind, npre), fused):
+        for g, r, what in zip(got, (s_ref, m_ref, c_ref), ("server", "mobile", "combined")):
+            assert (g is None) == (r is None), what
+            if r is not None:
+                same(g, r, what)
+    ref = K.topk_plan(c_ref.contiguous(), k, dind, npre, N)
+    for name in ("update_indice", "active_batch_idx", "active_pos_idx", "active_token_idx", "active_patch_mask",
+                 "active_rope_idx", "keep_mask", "row_slot"):
+        assert torch.equal(getattr(tp, name), getattr(ref, name)), name
+    assert bool(valid.all()) and valid.shape == (B, npre + k)
