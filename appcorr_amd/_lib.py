@@ -97,6 +97,7 @@ SIGNATURES: dict[str, list] = {
     "oudjat_rope_active_inplace": [_p, _i64, _i64, _p, _i64, _i64, _p, _p, _i64, _p, _p, _i64, _i64, _i64, _p],
     "oudjat_qkv_rope_kv_scatter": [_p, _i64, _i64, _i64, _p, _p, _i64, _p, _p, _p, _p, _p, _i64, _i64, _p, _p],
     "oudjat_layernorm_rows": [_p, _i64, _i64, _i64, _p, _p, _f32, _p, _i64, _p],
+    "oudjat_add_layernorm_rows": [_p, _p, _i64, _i64, _p, _p, _f32, _p, _p, _p, _i64, _p],
     "oudjat_layernorm_rows_prefetch": [_p, _i64, _i64, _i64, _p, _p, _f32, _p, _i64, _p, _i64, _p],
     "oudjat_linear_bf16": [_p, _i64, _i64, _i64, _p, _i64, _i64, _p, _i32, _p, _p, _i64, _p, _i64, _f32, _p, _i64,
                            _p],

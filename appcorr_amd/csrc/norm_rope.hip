@@ -121,14 +121,19 @@ __device__ __forceinline__ void layernorm_row(const float (&v)[CH][8], int lane,
 // the region sits in the last-level cache when the kernels after this one read it: the weights of a
 // linear that follows, whose first-touch misses would otherwise go to HBM. The words are folded into
 // a register that an empty asm statement consumes (nothing is stored); the output is the same bits.
-template <int CH, int NWR, bool PF = false>
+// ADD: the row is bf16(x + add), which also goes to `sum` (both contiguous): the approximate block's
+// attention residual with its norm2, whose rows are then not read back (16464 rows of 1024: residual 16.0
+// and norm 14.8 us apart, 23.5 together; 16404 of 4096: 73.5 and 47.4, 97).
+template <int CH, int NWR, bool PF = false, bool ADD = false>
 __global__ __launch_bounds__(kNormThreads) void layernorm_kernel(const uint16_t* __restrict__ x, int64_t rows, int C,
                                                                int64_t xs, const uint16_t* __restrict__ w,
                                                                const uint16_t* __restrict__ bias, float eps,
                                                                uint16_t* __restrict__ out, int64_t os,
                                                                const float* __restrict__ xh_ts,
                                                                const uint32_t* __restrict__ pf = nullptr,
-                                                               int64_t pf_lines = 0) {
+                                                               int64_t pf_lines = 0,
+                                                               const uint16_t* __restrict__ add = nullptr,
+                                                               uint16_t* __restrict__ sum = nullptr) {
   __shared__ float red[2 * kNormRowsPerWg];
   const int wave = threadIdx.x >> 6, slot = wave / NWR, part = wave % NWR;
   const int64_t row = (int64_t)blockIdx.x * (kNormRowsPerWg / NWR) + slot;
@@ -138,15 +143,17 @@ __global__ __launch_bounds__(kNormThreads) void layernorm_kernel(const uint16_t*
   const int chunks = (C >> 3) / NWR;  // this wave's part of the row
   const int c0 = part * chunks * 8;   // its first column
   // Every load of the lane is issued before the first use (one memory round trip per wave).
-  uint4 raw[CH];
+  uint4 raw[CH], rad[CH];
 #pragma unroll
-  for (int j = 0; j < CH; ++j) raw[j] = make_uint4(0u, 0u, 0u, 0u);
+  for (int j = 0; j < CH; ++j) raw[j] = rad[j] = make_uint4(0u, 0u, 0u, 0u);
   if (live) {
     const uint4* xv = reinterpret_cast<const uint4*>(x + row * xs + c0);
+    const uint4* dv = reinterpret_cast<const uint4*>(ADD ? add + row * C + c0 : nullptr);
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
       const int c = lane + 64 * j;
       if (c < chunks) raw[j] = xv[c];
+      if (ADD && c < chunks) rad[j] = dv[c];
     }
   }
   uint32_t touched = 0;
@@ -155,7 +162,19 @@ __global__ __launch_bounds__(kNormThreads) void layernorm_kernel(const uint16_t*
   if (NWR > 1 || live) {
     float v[CH][8];
 #pragma unroll
-    for (int j = 0; j < CH; ++j) unpack8(raw[j], v[j]);
+    for (int j = 0; j < CH; ++j) {
+      unpack8(raw[j], v[j]);
+      if constexpr (ADD) {
+        float f[8];
+        unpack8(rad[j], f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[j][e] += f[e];
+        const uint4 o = pack8(v[j]);
+        const int c = lane + 64 * j;
+        if (live && c < chunks) reinterpret_cast<uint4*>(sum + row * C + c0)[c] = o;
+        unpack8(o, v[j]);
+      }
+    }
     layernorm_row<CH, NWR>(v, lane, chunks, C, w + c0, bias + c0, eps, out + (live ? row : 0) * os + c0, xh_ts, red,
                            slot, part, live);
   }
@@ -490,7 +509,7 @@ static void row_dispatch(int64_t C, F&& f) {
 static int layernorm_launch(const uint16_t* x, int64_t rows, int64_t C, int64_t xs, const uint16_t* w,
                             const uint16_t* b, float eps, const float* xh_ts, uint16_t* out, int64_t os,
                             oudjat_stream_t stream, const char* what, const void* pf = nullptr,
-                            int64_t pf_bytes = 0) {
+                            int64_t pf_bytes = 0, const uint16_t* add = nullptr, uint16_t* sum = nullptr) {
   OUDJAT_REQUIRE(rows >= 0 && C > 0, OUDJAT_ERR_INVALID_ARGUMENT, "%s: bad size", what);
   OUDJAT_REQUIRE(pf_bytes >= 0 && (pf_bytes == 0 || pf), OUDJAT_ERR_INVALID_ARGUMENT,
                  "%s: prefetch region of %lld bytes without a pointer", what, (long long)pf_bytes);
@@ -507,14 +526,16 @@ static int layernorm_launch(const uint16_t* x, int64_t rows, int64_t C, int64_t 
   hipStream_t st = as_stream(stream);
   const int64_t pf_lines = pf_bytes / 128;  // whole lines; a partial last line is left to the reader
   const uint32_t* p = static_cast<const uint32_t*>(pf);
-  auto go = [&](auto pf_c) {
+  auto go = [&](auto pf_c, auto add_c) {
     row_dispatch(C, [&](auto ch, auto nwr) {
-      layernorm_kernel<decltype(ch)::value, decltype(nwr)::value, decltype(pf_c)::value>
-          <<<grid, kNormThreads, 0, st>>>(x, rows, (int)C, xs, w, b, eps, out, os, xh_ts, p, pf_lines);
+      layernorm_kernel<decltype(ch)::value, decltype(nwr)::value, decltype(pf_c)::value, decltype(add_c)::value>
+          <<<grid, kNormThreads, 0, st>>>(x, rows, (int)C, xs, w, b, eps, out, os, xh_ts, p, pf_lines, add, sum);
     });
   };
-  if (pf_lines > 0) go(std::true_type{});
-  else go(std::false_type{});
+  if (add && pf_lines > 0) go(std::true_type{}, std::true_type{});
+  else if (add) go(std::false_type{}, std::true_type{});
+  else if (pf_lines > 0) go(std::true_type{}, std::false_type{});
+  else go(std::false_type{}, std::false_type{});
   return check_launch(what);
 }
 
@@ -529,6 +550,16 @@ extern "C" int oudjat_layernorm_rows_prefetch(const uint16_t* x, int64_t rows, i
                                               oudjat_stream_t stream) {
   return layernorm_launch(x, rows, C, xs, w, b, eps, nullptr, out, os, stream, "layernorm_rows_prefetch", prefetch,
                           prefetch_bytes);
+}
+
+extern "C" int oudjat_add_layernorm_rows(const uint16_t* x, const uint16_t* add, int64_t rows, int64_t C,
+                                         const uint16_t* w, const uint16_t* b, float eps, uint16_t* sum, uint16_t* out,
+                                         const void* prefetch, int64_t prefetch_bytes, oudjat_stream_t stream) {
+  OUDJAT_REQUIRE(rows == 0 || (add && sum), OUDJAT_ERR_INVALID_ARGUMENT, "add_layernorm_rows: null pointer");
+  OUDJAT_REQUIRE(aligned(add, 16) && aligned(sum, 16), OUDJAT_ERR_UNSUPPORTED_LAYOUT,
+                 "add_layernorm_rows: 16-byte aligned rows required");
+  return layernorm_launch(x, rows, C, C, w, b, eps, nullptr, out, C, stream, "add_layernorm_rows", prefetch,
+                          prefetch_bytes, add, sum);
 }
 
 extern "C" int oudjat_layernorm_rows_nvfp4(const uint16_t* x, int64_t rows, int64_t C, int64_t xs, const uint16_t* w,

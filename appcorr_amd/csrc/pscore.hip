@@ -36,7 +36,8 @@ __device__ __forceinline__ double group_sum_f64(double v, int width) {
   return v;
 }
 
-// Block-wide reductions over kPsThreads threads; `red` holds one slot per wave.
+// Block-wide reductions over NT threads; `red` holds one slot per wave.
+template <int NT = kPsThreads>
 __device__ __forceinline__ float block_max(float v, float* red) {
   v = wave_max(v);
   const int w = threadIdx.x >> 6;
@@ -45,9 +46,10 @@ __device__ __forceinline__ float block_max(float v, float* red) {
   __syncthreads();
   float m = red[0];
 #pragma unroll
-  for (int i = 1; i < kPsThreads / 64; ++i) m = fmaxf(m, red[i]);
+  for (int i = 1; i < NT / 64; ++i) m = fmaxf(m, red[i]);
   return m;
 }
+template <int NT = kPsThreads>
 __device__ __forceinline__ double block_sum_f64(double v, double* red) {
   v = wave_sum_f64(v);
   const int w = threadIdx.x >> 6;
@@ -56,7 +58,7 @@ __device__ __forceinline__ double block_sum_f64(double v, double* red) {
   __syncthreads();
   double s = 0.0;
 #pragma unroll
-  for (int i = 0; i < kPsThreads / 64; ++i) s += red[i];  // fixed order
+  for (int i = 0; i < NT / 64; ++i) s += red[i];  // fixed order
   return s;
 }
 
@@ -72,19 +74,22 @@ __device__ __forceinline__ double dot8_f64(const float* a, const uint4& kv) {
 
 // One workgroup per (head h, image b): p[n] = bf16(e_n / sum e), e_n = exp(s_n - max s),
 // s_n = bf16(bf16(q . k_n) * scale), written as fp32 to ws[(b * H + h) * N + n].
-// L = Dh / 8 lanes share one key row (16 bytes each).
+// L = Dh / 8 lanes share one key row (16 bytes each). B * H workgroups are a round of the CUs at most, so
+// each takes 16 waves: with four, the keys streamed at 1.3 to 1.6 TB/s (16 images x 16 heads x 1029 keys of
+// Dh = 64 took 21 us, 4 x 32 x 4101 of Dh = 128 107).
+constexpr int kQpThreads = 1024;
 template <int L>
-__global__ void __launch_bounds__(kPsThreads) query_prob_kernel(const uint16_t* __restrict__ q, int64_t q_sb,
+__global__ void __launch_bounds__(kQpThreads) query_prob_kernel(const uint16_t* __restrict__ q, int64_t q_sb,
                                                                 int64_t q_sh, const uint16_t* __restrict__ k,
                                                                 int64_t k_sb, int64_t k_sn, int64_t k_sh, int N,
                                                                 int H, float scale, float* __restrict__ ws) {
   __shared__ float srow[kPsMaxKeys];
-  __shared__ float red_f[kPsThreads / 64];
-  __shared__ double red_d[kPsThreads / 64];
+  __shared__ float red_f[kQpThreads / 64];
+  __shared__ double red_d[kQpThreads / 64];
   const int h = blockIdx.x, b = blockIdx.y;
   const int lane_in_key = threadIdx.x % L;
   const int key_slot = threadIdx.x / L;
-  constexpr int kKeysPerIter = kPsThreads / L;
+  constexpr int kKeysPerIter = kQpThreads / L;
 
   float qa[8];
   unpack8(*reinterpret_cast<const uint4*>(q + b * q_sb + h * q_sh + lane_in_key * 8), qa);
@@ -109,29 +114,40 @@ __global__ void __launch_bounds__(kPsThreads) query_prob_kernel(const uint16_t* 
   }
   __syncthreads();
   float m = -INFINITY;
-  for (int n = threadIdx.x; n < N; n += kPsThreads) m = fmaxf(m, srow[n]);
-  m = block_max(m, red_f);
+  for (int n = threadIdx.x; n < N; n += kQpThreads) m = fmaxf(m, srow[n]);
+  m = block_max<kQpThreads>(m, red_f);
   double part = 0.0;
-  for (int n = threadIdx.x; n < N; n += kPsThreads) {
+  for (int n = threadIdx.x; n < N; n += kQpThreads) {
     const float e = (float)exp((double)(srow[n] - m));
     srow[n] = e;
     part += (double)e;
   }
-  const float tot = (float)block_sum_f64(part, red_d);
+  const float tot = (float)block_sum_f64<kQpThreads>(part, red_d);
   float* out = ws + ((int64_t)b * H + h) * N;
-  for (int n = threadIdx.x; n < N; n += kPsThreads) out[n] = round_bf16(div_rn(srow[n], tot));
+  for (int n = threadIdx.x; n < N; n += kQpThreads) out[n] = round_bf16(div_rn(srow[n], tot));
 }
 
 // out[b, n] = bf16(fl(sum_h p[b, h, n]) * factor), summed exactly in float64.
-__global__ void __launch_bounds__(kPsThreads) head_mean_kernel(const float* __restrict__ ws, int B, int H, int N,
+// One wave per workgroup (B * N / 64 of them) and eight heads' loads in flight: one load at a time from
+// B * N / 256 workgroups took 6.2 us at 16 x 1029 x 16 heads.
+constexpr int kHmThreads = 64;
+__global__ void __launch_bounds__(kHmThreads) head_mean_kernel(const float* __restrict__ ws, int B, int H, int N,
                                                                float factor, void* __restrict__ out,
                                                                int64_t out_sb, int out_bf16) {
-  const int64_t i = (int64_t)blockIdx.x * kPsThreads + threadIdx.x;
+  const int64_t i = (int64_t)blockIdx.x * kHmThreads + threadIdx.x;
   if (i >= (int64_t)B * N) return;
   const int b = (int)(i / N), n = (int)(i % N);
   const float* p = ws + (int64_t)b * H * N + n;
   double s = 0.0;
-  for (int h = 0; h < H; ++h) s += (double)p[(int64_t)h * N];
+  int h = 0;
+  for (; h + 8 <= H; h += 8) {
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = p[(int64_t)(h + u) * N];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s += (double)v[u];
+  }
+  for (; h < H; ++h) s += (double)p[(int64_t)h * N];
   const uint32_t bits = f32_to_bf16((float)s * factor);
   if (out_bf16)
     reinterpret_cast<uint16_t*>(out)[b * out_sb + n] = (uint16_t)bits;
@@ -249,15 +265,15 @@ extern "C" int oudjat_query_attention_prob(const uint16_t* q, int64_t q_stride_b
   hipStream_t s = as_stream(stream);
   const dim3 grid((unsigned)H, (unsigned)B);
   if (Dh == 64)
-    query_prob_kernel<8><<<grid, kPsThreads, 0, s>>>(q, q_stride_b, q_stride_h, k, k_stride_b, k_stride_n,
+    query_prob_kernel<8><<<grid, kQpThreads, 0, s>>>(q, q_stride_b, q_stride_h, k, k_stride_b, k_stride_n,
                                                      k_stride_h, (int)N, (int)H, scale, workspace);
   else
-    query_prob_kernel<16><<<grid, kPsThreads, 0, s>>>(q, q_stride_b, q_stride_h, k, k_stride_b, k_stride_n,
+    query_prob_kernel<16><<<grid, kQpThreads, 0, s>>>(q, q_stride_b, q_stride_h, k, k_stride_b, k_stride_n,
                                                       k_stride_h, (int)N, (int)H, scale, workspace);
   int st = check_launch("query_attention_prob");
   if (st != OUDJAT_OK) return st;
   const float factor = 1.0f / (float)H;
-  head_mean_kernel<<<(unsigned)cdiv(B * N, kPsThreads), kPsThreads, 0, s>>>(workspace, (int)B, (int)H, (int)N,
+  head_mean_kernel<<<(unsigned)cdiv(B * N, kHmThreads), kHmThreads, 0, s>>>(workspace, (int)B, (int)H, (int)N,
                                                                            factor, out, out_stride_b, out_bf16);
   return check_launch("query_attention_prob(head mean)");
 }

@@ -418,10 +418,9 @@ class SelfAttentionBlock(nn.Module):
         g1 = self._gamma(self.ls1, x2)
         inc = K.linear(attn, self.attn.proj.weight, self.attn.proj.bias, epilogue=_lib.EPI_BIAS_LS, gamma=g1,
                        site="proj")
-        ones = self._gamma(nn.Identity(), x2)
-        x_attn = K.fused_layerscale_add(x2, inc, ones)                       # x + ls1(attn)
-        mlp = self._mlp_scaled(K.layer_norm(x_attn, self.norm2.weight, self.norm2.bias, self.norm2.eps,
-                                            prefetch=self._mlp_prefetch()))
+        x_attn, xn2 = K.add_layer_norm(x2, inc, self.norm2.weight, self.norm2.bias, self.norm2.eps,  # x + ls1(attn)
+                                       prefetch=self._mlp_prefetch())
+        mlp = self._mlp_scaled(xn2)
         bos, out = K.residual_pair(inc, x_attn, mlp)  # block.py:336-347: inc + mlp cached, x_attn + mlp out
         cache_feature[f"{tag}_blocks_out_sum"] = bos.view(B, N, C)
         out = out.view(B, N, C)

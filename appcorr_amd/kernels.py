@@ -677,6 +677,24 @@ def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, eps: f
     return out
 
 
+def add_layer_norm(x: torch.Tensor, add: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, eps: float = 1e-5,
+                   prefetch: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor]:
+    """(bf16(x + add), layer_norm of it) of two contiguous bf16 tensors of one shape, in one launch and with the
+    bits of the two; prefetch as layer_norm's."""
+    _require_cuda(x, add, weight, bias, prefetch)
+    _require(x.dtype == add.dtype == weight.dtype == bias.dtype == torch.bfloat16, "add_layer_norm: bf16 only")
+    _require(x.shape == add.shape and x.is_contiguous() and add.is_contiguous(),
+             "add_layer_norm: contiguous tensors of one shape required")
+    _require(prefetch is None or (prefetch.is_contiguous() and prefetch.device == x.device),
+             "add_layer_norm: prefetch must be a contiguous tensor on the rows' device")
+    C = x.shape[-1]
+    total, out = torch.empty_like(x), torch.empty_like(x)
+    _launch("layernorm", x, "oudjat_add_layernorm_rows", _ptr(x), _ptr(add), x.numel() // max(C, 1), C,
+            _ptr(weight.contiguous()), _ptr(bias.contiguous()), float(eps), _ptr(total), _ptr(out), _ptr(prefetch),
+            0 if prefetch is None else prefetch.numel() * prefetch.element_size(), _stream(x))
+    return total, out
+
+
 def residual_pair(inc: torch.Tensor, x_attn: torch.Tensor, mlp: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """(bf16(inc + mlp), bf16(x_attn + mlp)) of three same-shape bf16 tensors with contiguous rows, in one
     launch: the approximate block's cached blocks_out_sum and its output (block.py:336-347)."""

@@ -319,6 +319,14 @@ int oudjat_layernorm_rows_prefetch(const uint16_t* x, int64_t rows, int64_t C, i
                                    int64_t out_row_stride, const void* prefetch, int64_t prefetch_bytes,
                                    oudjat_stream_t stream);
 
+/* Row 5 -- the approximate block's attention residual with norm2 (block.py:330-341) in one launch:
+ * sum = bf16(x + add) and out = oudjat_layernorm_rows_prefetch(sum), the bits of the two launches.
+ * x, add, sum, out: contiguous [rows, C]; sum may not alias x or add. */
+int oudjat_add_layernorm_rows(const uint16_t* x, const uint16_t* add, int64_t rows, int64_t C,
+                              const uint16_t* weight, const uint16_t* bias, float eps, uint16_t* sum,
+                              uint16_t* out, const void* prefetch, int64_t prefetch_bytes,
+                              oudjat_stream_t stream);
+
 /* Rows 6, 11, 12, 13 -- C[M, N] = epilogue(A[M, K] . W[N, K]^T) on bf16 MFMA with fp32 accumulate.
  * Replaces the qkv / proj / fc1 / fc2 nn.Linear calls (attention.py:415,532; ffn_layers.py:43-49)
  * and the LayerScale / residual ops folded into their epilogues (block.py:1129-1141); the SwiGLU

@@ -142,3 +142,17 @@ def test_patch_importance(dev):
                       (2, (d.double() ** 2).mean(-1).sqrt())):
         got = K.patch_importance(d.to(dev), mode).cpu().double()
         torch.testing.assert_close(got, ref, rtol=2e-6, atol=0)
+
+
+@pytest.mark.parametrize("rows,C,prefetch", [(1, 8, False), (5, 384, True), (203, 1024, False), (17, 1032, True),
+                                             (33, 4096, True), (2, 8192, False), (0, 1024, False)])
+def test_add_layer_norm_equals_the_two_launches(dev, rows, C, prefetch):
+    """One row to a ragged last workgroup, one to four waves a row, with and without a prefetched region: the
+    sum and its LayerNorm carry the bits of the separate launches."""
+    x, a = _rand_bf16((rows, C), 21).to(dev), _rand_bf16((rows, C), 22).to(dev)
+    w, b = _rand_bf16((C,), 23).to(dev), _rand_bf16((C,), 24).to(dev)
+    region = _rand_bf16((100, 512), 25).to(dev) if prefetch else None
+    total, ln = K.add_layer_norm(x, a, w, b, 1e-5, prefetch=region)
+    ref = K.fused_layerscale_add(x, a, torch.ones_like(w))
+    assert_bits_equal(total.cpu(), ref.cpu(), "sum")
+    assert_bits_equal(ln.cpu(), K.layer_norm(ref, w, b, 1e-5).cpu(), "layer norm")
