@@ -75,8 +75,8 @@ __device__ __forceinline__ double dot8_f64(const float* a, const uint4& kv) {
 // One workgroup per (head h, image b): p[n] = bf16(e_n / sum e), e_n = exp(s_n - max s),
 // s_n = bf16(bf16(q . k_n) * scale), written as fp32 to ws[(b * H + h) * N + n].
 // L = Dh / 8 lanes share one key row (16 bytes each). B * H workgroups are a round of the CUs at most, so
-// each takes 16 waves: with four, the keys streamed at 1.3 to 1.6 TB/s (16 images x 16 heads x 1029 keys of
-// Dh = 64 took 21 us, 4 x 32 x 4101 of Dh = 128 107).
+// each takes 16 waves: with four, too few loads were in flight (4 x 32 heads x 4101 keys of Dh = 128: 107 ->
+// 51 us; 16 x 16 x 1029 of Dh = 64, where the float64 dot products weigh as much as the loads, 21 -> 20).
 constexpr int kQpThreads = 1024;
 template <int L>
 __global__ void __launch_bounds__(kQpThreads) query_prob_kernel(const uint16_t* __restrict__ q, int64_t q_sb,
@@ -129,7 +129,7 @@ __global__ void __launch_bounds__(kQpThreads) query_prob_kernel(const uint16_t* 
 
 // out[b, n] = bf16(fl(sum_h p[b, h, n]) * factor), summed exactly in float64.
 // One wave per workgroup (B * N / 64 of them) and eight heads' loads in flight: one load at a time from
-// B * N / 256 workgroups took 6.2 us at 16 x 1029 x 16 heads.
+// B * N / 256 workgroups took 6.2 us at 16 x 1029 x 16 heads (now 4.8) and 11 at 4 x 4101 x 32 (4.6).
 constexpr int kHmThreads = 64;
 __global__ void __launch_bounds__(kHmThreads) head_mean_kernel(const float* __restrict__ ws, int B, int H, int N,
                                                                float factor, void* __restrict__ out,
