@@ -147,8 +147,9 @@ __global__ __launch_bounds__(kStWaves * 64) void pattn_stats_kernel(const uint16
     }
   };
 
-  // Finite start: a lane whose keys all lie past N keeps it, with an empty sum.
-  float m = -3.0e38f, l = 0.0f;
+  // A lane whose keys so far all lie past N (N <= 4: the whole half g = 1) has m = -inf and an empty sum; its
+  // exponents are then taken from 0, never from the difference of two infinities.
+  float m = -INFINITY, l = 0.0f;
   load(0);
   store(0);
   __syncthreads();
@@ -187,8 +188,9 @@ __global__ __launch_bounds__(kStWaves * 64) void pattn_stats_kernel(const uint16
         for (int v = 1; v < 8; ++v) mx[c4] = fmaxf(mx[c4], acc[c4 >> 1][8 * (c4 & 1) + v]);
       }
       const float m_new = fmaxf(fmaxf(m, fmaxf(mx[0], mx[1])), fmaxf(mx[2], mx[3]));
-      const float alpha = __builtin_amdgcn_exp2f((m - m_new) * kf);
-      const float off = m_new * kf;
+      const float ref = m_new == -INFINITY ? 0.0f : m_new;
+      const float alpha = __builtin_amdgcn_exp2f((m - ref) * kf);
+      const float off = ref * kf;
       float ts[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int kb2 = 0; kb2 < 2; ++kb2)

@@ -196,6 +196,24 @@ def test_dense_score_tile_edges(dev, B, H, N, D, scale, stride):
     assert u.max() <= 1.0 and float((u > 0).mean()) <= max(0.02, 2.0 / got.numel()), (u.max(), float((u > 0).mean()))
 
 
+@pytest.mark.parametrize("mode", [K.PATTN_DENSE, K.PATTN_LSE])
+@pytest.mark.parametrize("N,D,scale", [(1, 64, 0.1), (3, 64, 1.0), (4, 64, 64 ** -0.5), (1, 128, 128 ** -0.5),
+                                       (3, 128, 0.1), (4, 128, 128 ** -0.5), (5, 64, 0.1)])
+def test_patch_score_of_a_few_keys(dev, N, D, scale, mode):
+    """N <= 4: one lane of every query's pair holds no key at all. Every form of the scores (power-of-two
+    scale, below and at 1, and not), within one bf16 step of the exact evaluation."""
+    print(f"patch score of {N} keys D={D} scale={scale} mode={mode}", flush=True)
+    B, H = 2, 3
+    q, kv, qd, kvd = _qkv(B, H, N, D, 40 + N, dev)
+    got = K.patch_attention_prob(qd.reshape(B * N, H, D), kvd, scale, mode)
+    qh = np.ascontiguousarray(q.float().numpy().transpose(0, 2, 1, 3))
+    fn = PS.patch_attn_prob if mode == K.PATTN_DENSE else PS.patch_attn_prob_fused
+    ref = torch.from_numpy(fn(qh, kv[:, :, 0].float().numpy(), scale)).to(torch.bfloat16)
+    assert bool(torch.isfinite(got).all()), got
+    u = _bf16_ulps(got, ref)
+    assert u.max() <= 1.0, u.max()
+
+
 def test_patch_attention_prob_vit7b_mass(dev):
     """ViT-7B at 1024 px (N = 4101 > 4096: the dense path even for the layer-mean kind): every query's
     probabilities sum to one, so the key scores of an image sum to one up to the bf16 roundings."""
