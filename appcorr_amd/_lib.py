@@ -125,6 +125,7 @@ SIGNATURES: dict[str, list] = {
     "oudjat_sparse_query_attention_ws": [_p, _i64, _i64, _i64, _i64, _i64, _p, _i64, _i64, _i64, _i64, _i64, _f32,
                                          _p, _i64, _p, _i64, _p],
     "oudjat_sparse_query_attention_workspace_elems": [_i64, _i64, _i64, _i64, _i64],
+    "oudjat_sparse_query_attention_shape": [_i64, _i64, _i64, _i64, _i64, _i64, _p],
     "oudjat_sparse_query_attention_fp8": [_p, _i64, _i64, _i64, _i64, _i64, _p, _i64, _i64, _i64, _i64, _i64, _f32,
                                           _p, _p, _i64, _p],
     "oudjat_sparse_query_attention_lse": [_p, _i64, _i64, _i64, _i64, _i64, _p, _i64, _i64, _i64, _i64, _i64, _f32,

@@ -1090,11 +1090,18 @@ static double attn_wg_us(int64_t wgs, int64_t streams, int w, int waves, bool li
   return round * ((double)full + (wgs % kNumCus ? (full ? 0.8 : 1.0) : 0.0));
 }
 
-static AttnShape attn_shape(int64_t B, int64_t T, int64_t H, int64_t Dh, int64_t N, bool offsets_fit) {
+// The buffer-load kernel reads the keys of a pair through a descriptor of N * kvn elements from its first key:
+// it covers the N rows of Dh elements only where they lie forwards and do not overlap (a key row broadcast
+// over N has kvn = 0 and an empty descriptor), and its byte offsets must fit 31 bits.
+static bool buffer_rows_fit(int64_t N, int64_t kvn, int64_t Dh) {
+  return kvn >= Dh && N * kvn * 2 < ((int64_t)1 << 31);
+}
+
+// rows_fit: buffer_rows_fit of the call's keys (and no row log-sum-exp is asked for).
+static AttnShape attn_shape(int64_t B, int64_t T, int64_t H, int64_t Dh, int64_t N, bool rows_fit) {
   AttnShape s{};
   const int64_t waves = cdiv(T, 32);
-  // Buffer-load kernel when its byte offsets fit 31 bits; the register-staged kernel otherwise.
-  s.dma = offsets_fit;
+  s.dma = rows_fit;  // the register-staged kernel takes any strides
   s.kv_parts = 1;
   if (!s.dma) {
     s.n_wg = cdiv(waves, Dh == 64 ? kMaxWaves64 : kMaxWaves128);
@@ -1215,7 +1222,7 @@ static int sparse_query_attention_impl(const uint16_t* q, int64_t qrs, int64_t B
                  "sparse_query_attention: N or T too large");
   const float scale_log2 = scale * 1.4426950408889634f;
   // The row log-sum-exp comes from the register-staged kernel.
-  const AttnShape s = attn_shape(B, T, H, Dh, N, !lse && N * kvn * 2 < ((int64_t)1 << 31));
+  const AttnShape s = attn_shape(B, T, H, Dh, N, !lse && buffer_rows_fit(N, kvn, Dh));
   const int w = s.w;
   dim3 grid((unsigned)s.n_wg, (unsigned)H, (unsigned)B);
   hipStream_t st = as_stream(stream);
@@ -1342,7 +1349,7 @@ extern "C" int oudjat_sparse_query_attention_fp8(const uint16_t* q, int64_t qrs,
                  "4-byte aligned output rows required");
   OUDJAT_REQUIRE(B <= 65535 && H <= 65535 && N < ((int64_t)1 << 30) && T < ((int64_t)1 << 30), OUDJAT_ERR_TOO_LARGE,
                  "sparse_query_attention_fp8: too large");
-  const AttnShape s = attn_shape(B, T, H, Dh, N, N * kvn * 2 < ((int64_t)1 << 31));
+  const AttnShape s = attn_shape(B, T, H, Dh, N, buffer_rows_fit(N, kvn, Dh));
   const float scale_log2 = scale * 1.4426950408889634f;
   if (s.dma)
     return launch_attention128<true>(s, q, qrs, B, T, H, kv, kvb, kvn, kvkv, kvh, N, scale_log2, nullptr, ors, out,
@@ -1361,4 +1368,18 @@ extern "C" int64_t oudjat_sparse_query_attention_workspace_elems(int64_t B, int6
     return 0;
   const AttnShape s = attn_shape(B, T, H, Dh, N, true);
   return s.dma ? attn_workspace_elems(B, T, H, s.kv_parts) : 0;
+}
+
+// The launch a sparse_query_attention call of this shape and key row stride takes (with the workspace it asks
+// for): buffer loads or not, query workgroups per (image, head), query waves and waves per workgroup, light
+// parts, key parts.
+extern "C" int oudjat_sparse_query_attention_shape(int64_t B, int64_t T, int64_t H, int64_t Dh, int64_t N, int64_t kvn,
+                                                   int64_t* shape) {
+  OUDJAT_REQUIRE(shape && B > 0 && T > 0 && H > 0 && N > 0 && B <= 65535 && H <= 65535 && N < ((int64_t)1 << 30) &&
+                     T < ((int64_t)1 << 30) && (Dh == 64 || Dh == 128),
+                 OUDJAT_ERR_INVALID_ARGUMENT, "sparse_query_attention_shape: bad arguments");
+  const AttnShape s = attn_shape(B, T, H, Dh, N, buffer_rows_fit(N, kvn, Dh));
+  const int64_t v[6] = {s.dma, s.n_wg, s.w, s.dma ? s.waves : s.w, s.split, s.kv_parts};
+  for (int i = 0; i < 6; ++i) shape[i] = v[i];
+  return OUDJAT_OK;
 }

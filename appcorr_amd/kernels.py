@@ -1050,6 +1050,14 @@ def sparse_query_attention(q: torch.Tensor, kv_cache: torch.Tensor, T: int, scal
     return out
 
 
+def sparse_query_attention_shape(B: int, T: int, H: int, Dh: int, N: int, kv_stride_n: int) -> tuple:
+    """The launch `sparse_query_attention` takes for this shape, on the host alone: (buffer loads, query
+    workgroups per (image, head), query waves, waves per workgroup, light parts, key parts)."""
+    shape = (ctypes.c_int64 * 6)()
+    call("oudjat_sparse_query_attention_shape", B, T, H, Dh, N, kv_stride_n, ctypes.addressof(shape))
+    return (bool(shape[0]), *shape[1:])
+
+
 def sparse_query_attention_fp8(q: torch.Tensor, kv_cache: torch.Tensor, T: int, scale: float,
                                act_inv_scale: torch.Tensor) -> torch.Tensor:
     """sparse_query_attention's output as the e4m3fn codes (uint8 [B*T, H*Dh]) of FastFP8Linear's

@@ -508,6 +508,14 @@ int oudjat_sparse_query_attention_fp8(const uint16_t* q, int64_t q_row_stride, i
 int64_t oudjat_sparse_query_attention_workspace_elems(int64_t B, int64_t T, int64_t H, int64_t Dh,
                                                       int64_t N);
 
+/* Introspection, no counterpart in the reference: the launch that oudjat_sparse_query_attention_ws takes for
+ * this shape with the workspace it asks for, on the host alone. shape[0] 1: buffer loads, 0: the register-staged
+ * kernel (keys whose rows overlap, run backwards or lie past 31-bit byte offsets); [1] query workgroups per
+ * (image, head); [2] query waves and [3] all waves of a workgroup; [4] waves that share a light last query
+ * wave (0: none); [5] key parts. */
+int oudjat_sparse_query_attention_shape(int64_t B, int64_t T, int64_t H, int64_t Dh, int64_t N,
+                                        int64_t kv_stride_n, int64_t* shape);
+
 /* Approximate-pass server score with one query per (image, head) -- cls_attn_prob and, with the
  * pseudo query of oudjat_pseudo_query, patch_pseudo_attn_prob (the cache producer,
  * appcorr/models/dinov3/layers/attention.py:254-273):

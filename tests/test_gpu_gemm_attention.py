@@ -526,6 +526,39 @@ def test_attention_launch_shapes(dev, B, T, N, H):
     _check_attention(got.cpu(), qb, kv, D ** -0.5, o64.transpose(1, 2).reshape(B * T, H * D), f"shape {B},{T},{N},{H}")
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("stride", ["broadcast", "overlapping", "backwards"])
+@pytest.mark.parametrize("B,T,N,H", [(2, 40, 130, 3), (1, 300, 261, 2), (2, 107, 1029, 4)])
+def test_attention_key_row_strides(dev, B, T, N, H, stride, D):
+    """Key rows that no descriptor of N row strides covers: one row broadcast over N (stride 0), rows that
+    overlap (stride 8) and, through the C entry, rows that run backwards; few and many query waves, with and
+    without a workspace, against the float64 reference of the same keys."""
+    print(f"attention key strides {stride} {B},{T},{N},{H} D={D}", flush=True)
+    q = _rand((B * T, H, D), 50)
+    if stride == "backwards":
+        kv = _rand((B, N, 2, H, D), 51).to(dev)
+        view, used = kv, kv.flip(1)
+    else:
+        step = 0 if stride == "broadcast" else 8
+        image = (N - 1) * step + 2 * H * D  # elements one image's rows span
+        store = _rand((B * image,), 51).to(dev)
+        view = used = store.as_strided((B, N, 2, H, D), (image, step, H * D, D, 1))
+    qd = q.to(dev)
+    if stride == "backwards":
+        got = torch.empty((B * T, H * D), device=dev, dtype=torch.bfloat16)
+        last = view.data_ptr() + (N - 1) * view.stride(1) * 2
+        rc = _lib.load().oudjat_sparse_query_attention(
+            qd.data_ptr(), qd.stride(0), B, T, H, D, last, view.stride(0), -view.stride(1), view.stride(2),
+            view.stride(3), N, D ** -0.5, got.data_ptr(), got.stride(0), torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, _lib.load().oudjat_last_error()
+    else:
+        got = K.sparse_query_attention(qd, view, T, D ** -0.5)
+    kvc = used.cpu().contiguous()
+    qb = q.reshape(B, T, H, D).transpose(1, 2)
+    o64 = F64.sdpa(qb, kvc[:, :, 0].transpose(1, 2), kvc[:, :, 1].transpose(1, 2), D ** -0.5)
+    _check_attention(got.cpu(), qb, kvc, D ** -0.5, o64.transpose(1, 2).reshape(B * T, H * D), f"{stride} {B},{T},{N},{H}")
+
+
 @pytest.mark.parametrize("B,T,N,H,pad", [(1, 200, 261, 7, 0), (2, 257, 65, 3, 8), (1, 128, 64, 9, 0), (3, 700, 129, 5, 0),
                                          (16, 257, 193, 16, 0), (1, 1, 1, 1, 0), (1, 40, 130, 1, 1 << 23)])
 def test_attention_dh128_buffer_loads(dev, B, T, N, H, pad):

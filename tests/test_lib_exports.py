@@ -230,3 +230,18 @@ def test_fp8_gemm_entry_points_reject_bad_arguments():
     assert K.linear_fp8_kernel_name(1656, 12288, 4096, 5) == "oudjat::gemm_bf16_pp_kernel<192, 256, 5, true>"
     assert K.linear_fp8_kernel_name(1656, 4096, 8192, 3) == "oudjat::gemm_bf16_pp_kernel<128, 256, 3, true>"
     assert K.fp8_gemm_supported(4096, 12288) and not K.fp8_gemm_supported(384, 1152)
+
+
+@pytest.mark.parametrize("Dh", [64, 128])
+def test_attention_buffer_loads_only_for_rows_the_descriptor_covers(Dh):
+    """The buffer-load kernel's descriptor is N row strides long from the first key: broadcast (stride 0),
+    overlapping and backward key rows are outside it and take the register-staged kernel, at every query count."""
+    from appcorr_amd import kernels as K
+    H, N = 4, 300
+    for T in (1, 33, 300, 1000):
+        for B in (1, 16, 100):
+            assert K.sparse_query_attention_shape(B, T, H, Dh, N, 2 * H * Dh)[0]
+            assert K.sparse_query_attention_shape(B, T, H, Dh, N, Dh)[0]          # one head's rows back to back
+            for kvn in (0, 8, Dh - 8, -2 * H * Dh):
+                assert not K.sparse_query_attention_shape(B, T, H, Dh, N, kvn)[0], (T, B, kvn)
+            assert not K.sparse_query_attention_shape(B, T, H, Dh, 1 << 20, 1 << 10)[0]   # 2^31 bytes of keys
