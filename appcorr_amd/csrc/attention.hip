@@ -1092,9 +1092,11 @@ static double attn_wg_us(int64_t wgs, int64_t streams, int w, int waves, bool li
 
 // The buffer-load kernel reads the keys of a pair through a descriptor of N * kvn elements from its first key:
 // it covers the N rows of Dh elements only where they lie forwards and do not overlap (a key row broadcast
-// over N has kvn = 0 and an empty descriptor), and its byte offsets must fit 31 bits.
+// over N has kvn = 0 and an empty descriptor), and its byte offsets must fit 31 bits. The rows of the last tile
+// past N must lie past the descriptor, so that they load as zeros: their 32-bit offsets may not wrap (a single
+// key with a stride of 2^29 elements would have row 4 back at offset 0, and others anywhere in 2^30 bytes).
 static bool buffer_rows_fit(int64_t N, int64_t kvn, int64_t Dh) {
-  return kvn >= Dh && N * kvn * 2 < ((int64_t)1 << 31);
+  return kvn >= Dh && N * kvn * 2 < ((int64_t)1 << 31) && (N + kKeyTile) * kvn * 2 <= ((int64_t)1 << 32);
 }
 
 // rows_fit: buffer_rows_fit of the call's keys (and no row log-sum-exp is asked for).

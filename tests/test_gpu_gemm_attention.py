@@ -559,6 +559,20 @@ def test_attention_key_row_strides(dev, B, T, N, H, stride, D):
     _check_attention(got.cpu(), qb, kvc, D ** -0.5, o64.transpose(1, 2).reshape(B * T, H * D), f"{stride} {B},{T},{N},{H}")
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("T", [3, 300])
+def test_attention_one_key_with_a_large_row_stride(dev, T, D):
+    """One key whose row stride would wrap the buffer loads' 32-bit offsets inside the tile: the value row of
+    that key, in every query's output."""
+    print(f"attention one key T={T} D={D}", flush=True)
+    H = 2
+    q = _rand((T, H, D), 52).to(dev)
+    store = _rand((2 * H * D,), 53).to(dev)
+    kv = store.as_strided((1, 1, 2, H, D), (0, (1 << 29) + 8, H * D, D, 1))
+    got = K.sparse_query_attention(q, kv, T, D ** -0.5)
+    assert_bits_equal(got.cpu(), store[H * D:].expand(T, -1).contiguous().cpu(), "value row")
+
+
 @pytest.mark.parametrize("B,T,N,H,pad", [(1, 200, 261, 7, 0), (2, 257, 65, 3, 8), (1, 128, 64, 9, 0), (3, 700, 129, 5, 0),
                                          (16, 257, 193, 16, 0), (1, 1, 1, 1, 0), (1, 40, 130, 1, 1 << 23)])
 def test_attention_dh128_buffer_loads(dev, B, T, N, H, pad):

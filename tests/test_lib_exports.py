@@ -245,3 +245,19 @@ def test_attention_buffer_loads_only_for_rows_the_descriptor_covers(Dh):
             for kvn in (0, 8, Dh - 8, -2 * H * Dh):
                 assert not K.sparse_query_attention_shape(B, T, H, Dh, N, kvn)[0], (T, B, kvn)
             assert not K.sparse_query_attention_shape(B, T, H, Dh, 1 << 20, 1 << 10)[0]   # 2^31 bytes of keys
+
+
+@pytest.mark.parametrize("Dh", [64, 128])
+def test_attention_buffer_load_offsets_of_a_last_tile_do_not_wrap(Dh):
+    """Rows N .. of the last 64-key tile are addressed too and must lie past the descriptor (N strides) modulo
+    2^32: few keys with a large stride take the register-staged kernel; the same rule by brute force."""
+    from appcorr_amd import kernels as K
+    for N, kvn in ((1, 1 << 29), (1, 1 << 25), (1, (1 << 25) - 8), (3, 40000000), (63, 16777208), (64, 16777208),
+                   (65, 16000000), (100, 10000000), (129, 8000000), (1029, 2048)):
+        last = -(-N // 64) * 64
+        clear = all((r * kvn * 2) % (1 << 32) >= N * kvn * 2 for r in range(N, last))
+        got = K.sparse_query_attention_shape(2, 40, 3, Dh, N, kvn)[0]
+        assert clear or not got, (N, kvn)
+    assert not K.sparse_query_attention_shape(2, 40, 3, Dh, 1, 1 << 29)[0]
+    assert K.sparse_query_attention_shape(2, 40, 3, Dh, 1029, 2048)[0]
+    assert K.sparse_query_attention_shape(2, 40, 3, Dh, 100, 10000000)[0]
