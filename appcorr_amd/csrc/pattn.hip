@@ -224,7 +224,8 @@ __global__ __launch_bounds__(kStWaves * 64) void pattn_stats_kernel(const uint16
 static constexpr int kDnTile = 128;
 
 // Two workgroups per CU at DH = 64 (LDS 66 KB each, so the registers are held to 128); one at DH = 128.
-// OFF: the type of a lane's element offset from its tile's first row (32 bits while 128 rows span less).
+// OFF: the type of a lane's element offset from its tile's first row (uint32_t while 128 rows run forwards and
+// span less).
 template <int DH, int FORM, typename OFF>
 __global__ __launch_bounds__(512, DH == 64 ? 4 : 2) void pattn_colsum_kernel(const uint16_t* __restrict__ q, int64_t qrs,
                                                            const uint16_t* __restrict__ kv, int64_t kvb, int64_t kvn,
@@ -528,7 +529,8 @@ void launch_pattn(const uint16_t* q, int64_t qrs, const uint16_t* kv, int64_t kv
     float* part = ws + 2 * (int64_t)B * H * N;
     const int nqb = (int)cdiv(N, kDnTile);
     const unsigned g2 = (unsigned)(nqb * nqb * B);
-    if (std::max(std::abs(qrs), std::abs(kvn)) < ((int64_t)1 << 24))
+    // 32-bit offsets within a tile are unsigned: rows that run backwards (kvn < 0) take 64-bit ones.
+    if (qrs >= 0 && kvn >= 0 && std::max(qrs, kvn) < ((int64_t)1 << 24))
       pattn_colsum_kernel<DH, FORM, uint32_t>
           <<<g2, 512, 0, st>>>(q, qrs, kv, kvb, kvn, kvh, N, H, scale, row, part);
     else

@@ -18,6 +18,7 @@ import numpy as np
 import pytest
 import torch
 
+from appcorr_amd import _lib
 from appcorr_amd import kernels as K
 from appcorr_amd.dinov3 import SelfAttentionBlock
 from oracle import model as OM
@@ -212,6 +213,26 @@ def test_patch_score_of_a_few_keys(dev, N, D, scale, mode):
     assert bool(torch.isfinite(got).all()), got
     u = _bf16_ulps(got, ref)
     assert u.max() <= 1.0, u.max()
+
+
+@pytest.mark.parametrize("mode", [K.PATTN_DENSE, K.PATTN_LSE])
+@pytest.mark.parametrize("B,H,N,D", [(1, 2, 5, 64), (2, 3, 150, 64), (1, 4, 300, 128)])
+def test_patch_score_of_backward_key_rows(dev, B, H, N, D, mode):
+    """Key rows in the opposite order, through the C entry with a negative row stride: the bits of the call on
+    a reversed copy of the keys."""
+    print(f"patch score backward rows B={B} H={H} N={N} D={D} mode={mode}", flush=True)
+    _, _, qd, kvd = _qkv(B, H, N, D, 60 + N, dev)
+    qp = qd.reshape(B * N, H, D)
+    want = K.patch_attention_prob(qp, kvd.flip(1).contiguous(), D ** -0.5, mode)
+    lib = _lib.load()
+    ws = torch.empty(int(lib.oudjat_patch_attention_prob_workspace_elems(B, N, H, mode)), device=dev)
+    got = torch.empty((B, N), device=dev, dtype=torch.bfloat16)
+    rc = lib.oudjat_patch_attention_prob(
+        qp.data_ptr(), qp.stride(0), B, N, H, D, kvd.data_ptr() + (N - 1) * kvd.stride(1) * 2, kvd.stride(0),
+        -kvd.stride(1), kvd.stride(3), D ** -0.5, mode, ws.data_ptr(), got.data_ptr(), N,
+        torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.oudjat_last_error()
+    assert_bits_equal(got.cpu(), want.cpu(), "backward key rows")
 
 
 def test_patch_attention_prob_vit7b_mass(dev):
