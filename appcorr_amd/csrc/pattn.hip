@@ -11,7 +11,7 @@
 //
 // Rounding modes (the two paths of attention.py:241-253 and triton_kernels/attention_pscore.py):
 //   kDense: s = bf16(bf16(q.k) * scale), p = bf16(exp(s - m) / l) (torch softmax of a bf16 tensor;
-//           formed as exp2 of one exponent that holds the max and the sum),
+//           formed as exp2((s - m) log2 e) times 1 / l, max and sum held apart in fp32),
 //           head mean hm = bf16(sum_h p * fl(1/H)), score = bf16(sum_q hm * fl(1/N));
 //   kLse:   s = (q.k) in fp32, lse = m + log(l), p = exp2(s * (scale log2e) - lse * log2e) in fp32,
 //           score = bf16(sum_{q,h} p * fl(1/(H N))) -- the fused kernel's key-side sum from the row
@@ -47,17 +47,38 @@ __device__ __forceinline__ void round2_bf16(float& a, float& b) {
 
 static constexpr float kLog2e = 1.4426950408889634f;
 
-// How a kernel forms its scores from the fp32 products a = q.k (scale > 0 for kDenseP2):
+// How a kernel forms its scores from the fp32 products a = q.k (0 < scale <= 1/2 for kDenseP2):
 //   kDense     s = bf16(bf16(a) * scale)
 //   kDenseP2   the same for a power-of-two scale, whose second rounding changes nothing: the kernel keeps
 //              v = bf16(a) and the scale moves into the exponent's factor
 //   kLse       s = a * scale
-// In all of them exp(s - m) = exp2(v * kf - m * kf) with v and m in the kernel's own units and kf =
-// score_factor: one FMA and one v_exp_f32 per score.
+// In all of them exp(s - m) = exp2((v - m) * kf) with v and m in the kernel's own units and kf = score_factor;
+// `row_exp` takes it relative to the row's reference r (`row_ref`):
+//   kDense, kLse  r = m: a subtraction, exact for scores near m, and a product;
+//   kDenseP2      r = fl(m kf): one FMA, exp2(v kf - r), whose missing factor exp2(r - m kf), the same for every
+//                 score of the row, multiplies the sum or the probabilities' 1 / l (`ref_error`). m kf must not
+//                 overflow: kf <= 1 (scale <= 1/2), while kDense's kf = log2 e would from m = 2.4e38 on.
+// So the exponent is rounded relative to itself and not to the row's maximum: p is off by 2e-7 (rms, before its
+// bf16 rounding; 9e-7 at most) at row maxima of 1 to 16000. With m kf + log2 l folded into one float it
+// was 6e-7 at a maximum of 4, 2.6e-5 at 1000 and 3e-4 at 16000. That form took 216 us for 16 x 16 heads x
+// 1029^2 at scale 1/8 where this one takes 225, and 249 against 267 at scale 0.1 (kDense).
 static constexpr int kDenseP2 = 2;
 
 __host__ __device__ __forceinline__ float score_factor(int form, float scale) {
   return form == kDenseP2 ? scale * kLog2e : kLog2e;
+}
+
+template <int FORM>
+__device__ __forceinline__ float row_ref(float m, float kf) {
+  return FORM == kDenseP2 ? m * kf : m;
+}
+template <int FORM>
+__device__ __forceinline__ float ref_error(float m, float kf) {
+  return FORM == kDenseP2 ? __builtin_amdgcn_exp2f(-fmaf(m, kf, -m * kf)) : 1.0f;
+}
+template <int FORM>
+__device__ __forceinline__ float row_exp(float v, float r, float kf) {
+  return __builtin_amdgcn_exp2f(FORM == kDenseP2 ? fmaf(v, kf, -r) : (v - r) * kf);
 }
 
 // The scores of one 32 x 32 MFMA block in place, in the kernel's units.
@@ -91,9 +112,9 @@ __device__ __forceinline__ int xcd_band(int bid, int n) {
 // each lane keeps the running max of its half of the keys and the sum of exp(s - max), rescaled per tile
 // (the max is exact in any order; a tile's terms are summed apart and then added, which rounds less than
 // one long chain); the two lanes of a query merge at the end. Bound by the VALU (one exponential per
-// score): two passes over the keys with expf before, 266 -> 101 us at 16 images x 16 heads x 1029^2.
-// Output: kLse the row log-sum-exp (natural log), dense the row's exponent offset m kf + log2(l), so that
-// a probability is exp2(v kf - offset). Waves whose queries lie past N still stage tiles and meet every
+// score): two passes over the keys with expf before, 266 -> 97 us at 16 images x 16 heads x 1029^2.
+// Output: kLse the row log-sum-exp (natural log) in ref_out; dense the row's reference there and its
+// ref_error / l in w_out, so that a probability is row_exp(v) * w. Waves whose queries lie past N still stage tiles and meet every
 // barrier.
 static constexpr int kStWaves = 8;
 static constexpr int kStKeys = 64;
@@ -102,7 +123,8 @@ template <int DH, int FORM>
 __global__ __launch_bounds__(kStWaves * 64) void pattn_stats_kernel(const uint16_t* __restrict__ q, int64_t qrs,
                                                                     const uint16_t* __restrict__ kv, int64_t kvb,
                                                                     int64_t kvn, int64_t kvh, int N, int H,
-                                                                    float scale, float* __restrict__ row_out) {
+                                                                    float scale, float* __restrict__ ref_out,
+                                                                    float* __restrict__ w_out) {
   constexpr int KS = DH / 16;
   constexpr int CPR = DH / 8;
   constexpr int CHUNKS = kStKeys * CPR;
@@ -188,15 +210,15 @@ __global__ __launch_bounds__(kStWaves * 64) void pattn_stats_kernel(const uint16
         for (int v = 1; v < 8; ++v) mx[c4] = fmaxf(mx[c4], acc[c4 >> 1][8 * (c4 & 1) + v]);
       }
       const float m_new = fmaxf(fmaxf(m, fmaxf(mx[0], mx[1])), fmaxf(mx[2], mx[3]));
-      const float ref = m_new == -INFINITY ? 0.0f : m_new;
-      const float alpha = __builtin_amdgcn_exp2f((m - ref) * kf);
-      const float off = ref * kf;
+      const float mf = m_new == -INFINITY ? 0.0f : m_new;
+      const float alpha = __builtin_amdgcn_exp2f((m - mf) * kf);
+      const float ref = row_ref<FORM>(mf, kf);
       float ts[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int kb2 = 0; kb2 < 2; ++kb2)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) ts[v & 3] += __builtin_amdgcn_exp2f(fmaf(acc[kb2][v], kf, -off));
-      l = fmaf(l, alpha, (ts[0] + ts[1]) + (ts[2] + ts[3]));
+        for (int v = 0; v < 16; ++v) ts[v & 3] += row_exp<FORM>(acc[kb2][v], ref, kf);
+      l = fmaf(l, alpha, ref_error<FORM>(mf, kf) * ((ts[0] + ts[1]) + (ts[2] + ts[3])));
       m = m_new;
     }
     if (t + 1 < ntiles) store(buf ^ 1);
@@ -206,20 +228,23 @@ __global__ __launch_bounds__(kStWaves * 64) void pattn_stats_kernel(const uint16
   const float mt = fmaxf(m, m2);
   l = l * __builtin_amdgcn_exp2f((m - mt) * kf) + l2 * __builtin_amdgcn_exp2f((m2 - mt) * kf);
   const int qi = q0 + l32;
-  if (active && g == 0 && qi < N)
-    row_out[((int64_t)b * H + h) * N + qi] = FORM == kLse ? mt + logf(l) : fmaf(mt, kf, log2f(l));
+  if (active && g == 0 && qi < N) {
+    const int64_t o = ((int64_t)b * H + h) * N + qi;
+    ref_out[o] = FORM == kLse ? mt + logf(l) : row_ref<FORM>(mt, kf);
+    if (FORM != kLse) w_out[o] = ref_error<FORM>(mt, kf) / l;
+  }
 }
 
 // Dense key-side score: workgroup = (128-query block, 128-key block, image), 8 waves; wave w takes
 // queries 32 (w % 4) .. + 31 and keys 64 (w / 4) .. + 63 of the tile (two 32-key MFMA blocks, S = Q . K^T
 // so a key's column sits in one lane pair). For every head the Q and K tiles (128 x DH each, swizzled
-// 16-byte chunks) and the 128 queries' exponent offsets (pattn_stats_kernel) are staged once in LDS,
-// double-buffered through registers; p = bf16(exp2(v kf - offset)) is summed over heads per (query, key)
+// 16-byte chunks) and the 128 queries' references and weights (pattn_stats_kernel) are staged once in LDS,
+// double-buffered through registers; p = bf16(row_exp(v) * w) is summed over heads per (query, key)
 // in registers. After the last head each (query, key) takes bf16(sum * fl(1/H)); the tile's column sums
 // over its queries (four query waves added in order in LDS) go to part[b][query block][key], and
 // pattn_dense_reduce_kernel adds the query blocks in order. Waves wholly past N compute nothing
 // (N = 1029 is 8 tiles and 5 rows). Bound by the VALU (one exponential and two to three bf16
-// roundings per score and head): with expf and a divided quotient before, 344 -> 123 us at 16 images x 16
+// roundings per score and head): with expf and a divided quotient before, 344 -> 129 us at 16 images x 16
 // heads x 1029^2.
 static constexpr int kDnTile = 128;
 
@@ -230,7 +255,8 @@ template <int DH, int FORM, typename OFF>
 __global__ __launch_bounds__(512, DH == 64 ? 4 : 2) void pattn_colsum_kernel(const uint16_t* __restrict__ q, int64_t qrs,
                                                            const uint16_t* __restrict__ kv, int64_t kvb, int64_t kvn,
                                                            int64_t kvh, int N, int H, float scale,
-                                                           const float* __restrict__ row_in,
+                                                           const float* __restrict__ ref_in,
+                                                           const float* __restrict__ w_in,
                                                            float* __restrict__ part) {
   constexpr int KS = DH / 16;
   constexpr int CPR = DH / 8;
@@ -241,7 +267,7 @@ __global__ __launch_bounds__(512, DH == 64 ? 4 : 2) void pattn_colsum_kernel(con
   constexpr int IT = CHUNKS / NT;
   static_assert(CHUNKS % NT == 0, "whole chunks per thread");
   __shared__ __align__(16) unsigned char tiles[2][2 * TILEB];
-  __shared__ __align__(16) float st[2][kDnTile];  // row offsets
+  __shared__ __align__(16) float st[2][2][kDnTile];  // row references, weights
   __shared__ float colp[4][kDnTile];
   const int nb = (N + kDnTile - 1) / kDnTile;  // query blocks = key blocks
   const int item = xcd_band((int)blockIdx.x, (int)gridDim.x);
@@ -267,13 +293,14 @@ __global__ __launch_bounds__(512, DH == 64 ? 4 : 2) void pattn_colsum_kernel(con
                          : (OFF)min(r, N - 1 - kt0) * (OFF)kvn + (OFF)(ch * 8);
   }
   u32x4_t rq[IT];
-  float rs = INFINITY;
+  float rs = 1.0f;
   auto load = [&](int h) __attribute__((always_inline)) {
     const uint16_t* qh = qbase + (int64_t)h * DH;
     const uint16_t* kh = kbase + (int64_t)h * kvh;
 #pragma unroll
     for (int i = 0; i < IT; ++i) rq[i] = *reinterpret_cast<const u32x4_t*>((i < IT / 2 ? qh : kh) + off_[i]);
-    if (tid < kDnTile && qt0 + tid < N) rs = row_in[((int64_t)b * H + h) * N + qt0 + tid];
+    if (tid < 2 * kDnTile && qt0 + (tid & (kDnTile - 1)) < N)
+      rs = (tid < kDnTile ? ref_in : w_in)[((int64_t)b * H + h) * N + qt0 + (tid & (kDnTile - 1))];
   };
   auto store = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
@@ -282,7 +309,7 @@ __global__ __launch_bounds__(512, DH == 64 ? 4 : 2) void pattn_colsum_kernel(con
       const int r = c / CPR, ch = c - r * CPR;
       *reinterpret_cast<u32x4_t*>(&tiles[buf][(i < IT / 2 ? 0 : TILEB) + r * ROWB + ((ch ^ (r & (CPR - 1))) << 4)]) = rq[i];
     }
-    if (tid < kDnTile) st[buf][tid] = rs;
+    if (tid < 2 * kDnTile) st[buf][tid / kDnTile][tid & (kDnTile - 1)] = rs;
   };
 
   float hs[2][16];
@@ -322,11 +349,12 @@ __global__ __launch_bounds__(512, DH == 64 ? 4 : 2) void pattn_colsum_kernel(con
         block_scores<FORM>(acc, scale);
 #pragma unroll
         for (int a = 0; a < 4; ++a) {
-          const float4 o4 = *reinterpret_cast<const float4*>(&st[buf][wq + 8 * a + 4 * g]);
-          const float off[4] = {o4.x, o4.y, o4.z, o4.w};
+          const float4 r4 = *reinterpret_cast<const float4*>(&st[buf][0][wq + 8 * a + 4 * g]);
+          const float4 w4 = *reinterpret_cast<const float4*>(&st[buf][1][wq + 8 * a + 4 * g]);
+          const float ref[4] = {r4.x, r4.y, r4.z, r4.w}, w[4] = {w4.x, w4.y, w4.z, w4.w};
           float pv[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) pv[e] = __builtin_amdgcn_exp2f(fmaf(acc[4 * a + e], kf, -off[e]));
+          for (int e = 0; e < 4; ++e) pv[e] = row_exp<FORM>(acc[4 * a + e], ref[e], kf) * w[e];
           round2_bf16(pv[0], pv[1]);
           round2_bf16(pv[2], pv[3]);
 #pragma unroll
@@ -515,15 +543,16 @@ void launch_colsum_lse(const uint16_t* q, int64_t qrs, const uint16_t* kv, int64
                                                                   1.0f / (float)((int64_t)H * N), out, osb);
 }
 
-// FORM kLse, kDense or kDenseP2 (the dense mode with a positive power-of-two scale, e.g. 64^-0.5 = 1/8).
+// FORM kLse, kDense or kDenseP2 (the dense mode with a power-of-two scale of at most 1/2, e.g. 64^-0.5 = 1/8).
 template <int DH, int FORM>
 void launch_pattn(const uint16_t* q, int64_t qrs, const uint16_t* kv, int64_t kvb, int64_t kvn, int64_t kvh, int B,
                   int N, int H, float scale, float* ws, uint16_t* out, int64_t osb, hipStream_t st) {
-  float* row = ws;  // the row log-sum-exp, or the dense mode's exponent offset
+  float* ref = ws;                      // the rows' references, or log-sum-exp mode's row log-sum-exp
+  float* w = ws + (int64_t)B * H * N;   // the rows' weights, or log-sum-exp mode's partial column sums
   const unsigned g1 = (unsigned)(cdiv(N, 32 * kStWaves) * H * B);
-  pattn_stats_kernel<DH, FORM><<<g1, kStWaves * 64, 0, st>>>(q, qrs, kv, kvb, kvn, kvh, N, H, scale, row);
+  pattn_stats_kernel<DH, FORM><<<g1, kStWaves * 64, 0, st>>>(q, qrs, kv, kvb, kvn, kvh, N, H, scale, ref, w);
   if constexpr (FORM == kLse) {
-    launch_colsum_lse<DH>(q, qrs, kv, kvb, kvn, kvh, B, N, H, scale, row, ws + (int64_t)B * H * N, out, osb, st);
+    launch_colsum_lse<DH>(q, qrs, kv, kvb, kvn, kvh, B, N, H, scale, ref, w, out, osb, st);
   } else {
     // Partial column sums per 128-query block after the statistics.
     float* part = ws + 2 * (int64_t)B * H * N;
@@ -532,9 +561,9 @@ void launch_pattn(const uint16_t* q, int64_t qrs, const uint16_t* kv, int64_t kv
     // 32-bit offsets within a tile are unsigned: rows that run backwards (kvn < 0) take 64-bit ones.
     if (qrs >= 0 && kvn >= 0 && std::max(qrs, kvn) < ((int64_t)1 << 24))
       pattn_colsum_kernel<DH, FORM, uint32_t>
-          <<<g2, 512, 0, st>>>(q, qrs, kv, kvb, kvn, kvh, N, H, scale, row, part);
+          <<<g2, 512, 0, st>>>(q, qrs, kv, kvb, kvn, kvh, N, H, scale, ref, w, part);
     else
-      pattn_colsum_kernel<DH, FORM, int64_t><<<g2, 512, 0, st>>>(q, qrs, kv, kvb, kvn, kvh, N, H, scale, row, part);
+      pattn_colsum_kernel<DH, FORM, int64_t><<<g2, 512, 0, st>>>(q, qrs, kv, kvb, kvn, kvh, N, H, scale, ref, w, part);
     const int64_t n = (int64_t)B * N;
     pattn_dense_reduce_kernel<<<(unsigned)cdiv(n, 256), 256, 0, st>>>(part, B, N, nqb, out, osb);
   }
@@ -544,7 +573,7 @@ template <int DH>
 void launch_pattn_mode(const uint16_t* q, int64_t qrs, const uint16_t* kv, int64_t kvb, int64_t kvn, int64_t kvh, int B,
                        int N, int H, float scale, int mode, float* ws, uint16_t* out, int64_t osb, hipStream_t st) {
   int e = 0;
-  const bool pow2 = scale > 0.0f && std::isfinite(scale) && std::frexp(scale, &e) == 0.5f && std::abs(e) < 64;
+  const bool pow2 = scale > 0.0f && std::frexp(scale, &e) == 0.5f && e <= 0 && e > -64;
   if (mode == kLse) launch_pattn<DH, kLse>(q, qrs, kv, kvb, kvn, kvh, B, N, H, scale, ws, out, osb, st);
   else if (pow2) launch_pattn<DH, kDenseP2>(q, qrs, kv, kvb, kvn, kvh, B, N, H, scale, ws, out, osb, st);
   else launch_pattn<DH, kDense>(q, qrs, kv, kvb, kvn, kvh, B, N, H, scale, ws, out, osb, st);
@@ -556,8 +585,8 @@ using namespace oudjat;
 
 extern "C" int64_t oudjat_patch_attention_prob_workspace_elems(int64_t B, int64_t N, int64_t H, int mode) {
   if (B <= 0 || N <= 0 || H <= 0) return 0;
-  // row statistics (max or log-sum-exp, sum), then the dense mode's per-query-block column sums (the
-  // log-sum-exp mode's per-head-group sums reuse the second array)
+  // two arrays of row statistics (dense: references and weights; log-sum-exp mode: the row log-sum-exp, and its
+  // per-head-group column sums in the second), then the dense mode's per-query-block column sums
   return 2 * B * H * N + (mode == kDense ? B * cdiv(N, kDnTile) * N : 0);
 }
 

@@ -567,9 +567,10 @@ int oudjat_pseudo_query(const uint16_t* q, int64_t q_stride_b, int64_t q_stride_
  *     p = exp2(s log2e - lse log2e) from the row log-sum-exp, out = bf16(fl(sum_{t,h} p) * fl(1/(H N))).
  * q [B * N, H, Dh] packed rows (row stride q_row_stride elements, after RoPE); K [b, n, h, :] at
  * kv + b*kv_stride_b + n*kv_stride_n + h*kv_stride_h (the K half of {tag}_kv). q . k is an fp32 MFMA
- * accumulation and exp is the fp32 device exponential: agreement with an exact evaluation is to fp32
- * rounding before each bf16 rounding. workspace: oudjat_patch_attention_prob_workspace_elems(B, N, H,
- * mode) fp32 (row statistics, then partial column sums). out [B, N] bf16 (row stride out_stride_b).
+ * accumulation and exp is the fp32 device exponential of the score's distance from its row maximum:
+ * agreement with an exact evaluation is to fp32 rounding before each bf16 rounding, whatever the scores'
+ * magnitude. workspace: oudjat_patch_attention_prob_workspace_elems(B, N, H, mode) fp32 (two arrays of row
+ * statistics, then partial column sums). out [B, N] bf16 (row stride out_stride_b).
  * Dh in {64, 128}; 16-byte aligned rows. */
 int oudjat_patch_attention_prob(const uint16_t* q, int64_t q_row_stride, int64_t B, int64_t N, int64_t H,
                                 int64_t Dh, const uint16_t* kv, int64_t kv_stride_b, int64_t kv_stride_n,

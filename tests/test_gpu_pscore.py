@@ -215,6 +215,28 @@ def test_patch_score_of_a_few_keys(dev, N, D, scale, mode):
     assert u.max() <= 1.0, u.max()
 
 
+@pytest.mark.parametrize("logit", [0, 300, 1000, 4000, 16000])
+@pytest.mark.parametrize("D,scale", [(64, 0.125), (64, 0.1), (64, 1.0), (128, 128 ** -0.5)])
+@pytest.mark.parametrize("H,N", [(1, 640), (3, 261)])
+def test_dense_score_of_large_logits(dev, H, N, D, scale, logit):
+    """Rows whose scores are some hundreds to thousands: the probabilities' exponents are relative to the row's
+    maximum, so as few scores as at ordinary magnitudes move by a bf16 step (measured 0 to 0.6 %; an exponent
+    that holds the maximum is off by 3e-4 at 16000 and moves 4 to 16 %)."""
+    print(f"dense score of logits near {logit} H={H} N={N} D={D} scale={scale}", flush=True)
+    g = torch.Generator().manual_seed(logit + N)
+    q = torch.randn(1, N, H, D, generator=g) * 2.0
+    kv = torch.randn(1, N, 2, H, D, generator=g)
+    if logit:
+        q[..., 0] = kv[:, :, 0, :, 0] = (logit / scale) ** 0.5
+        q[..., 1:] *= logit ** 0.5 / 4
+    q, kv = q.to(torch.bfloat16), kv.to(torch.bfloat16)
+    got = K.patch_attention_prob(q.reshape(N, H, D).to(dev), kv.to(dev), scale, K.PATTN_DENSE).cpu()
+    qh = np.ascontiguousarray(q.float().numpy().transpose(0, 2, 1, 3))
+    ref = torch.from_numpy(PS.patch_attn_prob(qh, kv[:, :, 0].float().numpy(), scale)).to(torch.bfloat16)
+    differ = float((got != ref).float().mean())
+    assert differ <= 0.01, differ
+
+
 @pytest.mark.parametrize("mode", [K.PATTN_DENSE, K.PATTN_LSE])
 @pytest.mark.parametrize("B,H,N,D", [(1, 2, 5, 64), (2, 3, 150, 64), (1, 4, 300, 128)])
 def test_patch_score_of_backward_key_rows(dev, B, H, N, D, mode):
