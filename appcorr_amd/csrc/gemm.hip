@@ -2085,6 +2085,7 @@ extern "C" int oudjat_linear_swiglu_nvfp4(const uint16_t* A, int64_t M, int64_t 
   ea.b1 = b1;
   ea.b2 = b2;
   ea.xh_ts = tensor_scale;
+  OUDJAT_REQUIRE(!far_operands(M, lda, N, ldw), OUDJAT_ERR_TOO_LARGE, "%s: operands beyond 4 GiB", what);
   // The epilogue exists on the ping-pong tiles; shapes whose choice is another family take 192 x 256.
   int ci = choose_cfg(M, N, K, true);
   if (kCfgs[ci].fn[kEpiSwigluXh] == nullptr) ci = kPp192x256;
@@ -2104,6 +2105,7 @@ extern "C" int oudjat_linear_splitk_partial(const uint16_t* A, int64_t M, int64_
                  OUDJAT_ERR_UNSUPPORTED_LAYOUT, "linear_splitk_partial: operands must be 16-byte aligned, ld %% 8 == 0");
   OUDJAT_REQUIRE(M < ((int64_t)1 << 31) && N < ((int64_t)1 << 31) && K < ((int64_t)1 << 31), OUDJAT_ERR_TOO_LARGE,
                  "linear_splitk_partial: dimensions must fit in int32");
+  OUDJAT_REQUIRE(!far_operands(M, lda, N, ldw), OUDJAT_ERR_TOO_LARGE, "linear_splitk_partial: operands beyond 4 GiB");
   int S = 1;
   const int ci = choose_splitk(M, N, K, OUDJAT_EPI_BIAS_LS, &S);
   OUDJAT_REQUIRE(ci >= 0 && S > 1 && (int64_t)S * M * N <= workspace_elems, OUDJAT_ERR_UNSUPPORTED_SHAPE,
@@ -2120,14 +2122,15 @@ extern "C" int oudjat_linear_splitk_partial(const uint16_t* A, int64_t M, int64_
 extern "C" int64_t oudjat_linear_workspace_elems(int64_t M, int64_t N, int64_t K, int epi) {
   epi &= ~OUDJAT_EPI_RAW_BF16;
   int S = 1;
-  if (M <= 0 || N <= 0 || K <= 0 || choose_splitk(M, N, K, epi, &S) < 0 || S <= 1) return 0;
+  if (M <= 0 || N <= 0 || K <= 0 || far_operands(M, K, N, K) || choose_splitk(M, N, K, epi, &S) < 0 || S <= 1)
+    return 0;
   return (int64_t)S * M * N;
 }
 
 extern "C" int64_t oudjat_linear_warm_slots(int64_t M, int64_t N, int64_t K, int epi) {
   epi &= ~OUDJAT_EPI_RAW_BF16;
   if (M <= 0 || N <= 0 || K <= 0 || N % 64 != 0 || K % kBK != 0 || epi < OUDJAT_EPI_BIAS ||
-      epi > OUDJAT_EPI_BIAS_SILU_MUL)
+      epi > OUDJAT_EPI_BIAS_SILU_MUL || far_operands(M, K, N, K))
     return 0;
   int S = 1;
   if (choose_splitk(M, N, K, epi, &S) >= 0 && S > 1) return 0;  // split launches take none
@@ -2223,11 +2226,12 @@ extern "C" int oudjat_linear_qkv_rope_kv_nvfp4(const uint16_t* A, int64_t M, int
 static int kernel_name_of(const GemmCfg& c, int epi, char* buf, int64_t buflen);
 
 // Kernel a linear_bf16 call of this shape would launch, as the demangled name profilers print
-// (aligned operands assumed). For matching profile summaries to the running build.
+// (aligned operands with contiguous rows assumed). For matching profile summaries to the running build.
 extern "C" int oudjat_linear_kernel_name(int64_t M, int64_t N, int64_t K, int epi, char* buf, int64_t buflen) {
   OUDJAT_REQUIRE(buf && buflen > 0, OUDJAT_ERR_INVALID_ARGUMENT, "linear_kernel_name: no buffer");
   OUDJAT_REQUIRE(M > 0 && N > 0 && K > 0 && epi >= 0 && epi <= kEpiQkv, OUDJAT_ERR_INVALID_ARGUMENT,
                  "linear_kernel_name: bad arguments");
+  if (far_operands(M, K, N, K)) return kernel_name_of(kCfgs[far_cfg(N)], epi, buf, buflen);
   int S = 1;
   const int sk = epi == kEpiQkv ? -1 : choose_splitk(M, N, K, epi, &S);
   if (sk >= 0 && S > 1) epi = kEpiPartial;  // split K (with a workspace): the partial kernel, then the reduce

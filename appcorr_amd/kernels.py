@@ -288,11 +288,11 @@ def linear_ls_packed_residual(h: torch.Tensor, weight: torch.Tensor, bias: torch
     """mlp = bf16(bf16(h . W^T + bias) * gamma) split K, its reduce fused with packed_residual_persist_ln
     (or packed_residual_persist when `ln` is None): returns (x_new, LN(x_new) or None), bit-identical to
     linear(..., EPI_BIAS_LS) followed by that residual step. `ln` = (weight, bias, eps) of the next block's
-    norm1. Returns None when the product does not split K or an operand is not 16-byte aligned (the
-    caller then runs the two steps)."""
+    norm1. Returns None when the product does not split K, or an operand is not 16-byte aligned or spans
+    4 GiB (the caller then runs the two steps)."""
     M, Kd = h.shape
     N = weight.shape[0]
-    if not linear_splits_k(M, N, Kd):
+    if not linear_splits_k(M, N, Kd) or M * h.stride(0) * 2 >= 1 << 32 or N * weight.stride(0) * 2 >= 1 << 32:
         return None
     tensors = [h, weight, gamma, x_act, x_attn] + ([bias] if bias is not None else [])
     if ln is not None:

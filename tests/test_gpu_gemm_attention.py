@@ -220,6 +220,26 @@ def test_linear_small_tiles(dev, M, N, Kd, kernel):
                       what="small + swiglu")
 
 
+def _far(t, stride):
+    """t [M, K] with rows `stride` elements apart (only its own rows of the store are touched)."""
+    store = torch.empty(((t.shape[0] - 1) * stride + t.shape[1],), device=t.device, dtype=t.dtype)
+    v = store.as_strided(t.shape, (stride, 1))
+    v.copy_(t)
+    return v
+
+
+@pytest.mark.parametrize("M,N,Kd,lda,ldw", [(3, 384, 256, (1 << 30) + 8, 0), (103, 384, 1536, 1 << 25, 0),
+                                            (9, 128, 256, 0, 1 << 24), (5, 192, 128, 0, 1 << 24)])
+def test_linear_operands_of_4_gib(dev, M, N, Kd, lda, ldw):
+    """A few rows so far apart that the operand spans 4 GiB: past 32-bit buffer offsets the direct-to-LDS tiles
+    run, also where the shape would split K or run on 16-row tiles, within the accumulation bound of the oracle."""
+    print(f"far operands {M}x{N}x{Kd} lda {lda} ldw {ldw}", flush=True)
+    x, w, b = _rand((M, Kd), 90), _rand((N, Kd), 91, 0.02), _rand((N,), 92, 0.1)
+    xd, wd = x.to(dev), w.to(dev)
+    got = K.linear(_far(xd, lda) if lda else xd, _far(wd, ldw) if ldw else wd, b.to(dev))
+    _check_gemm(dev, got, x, w, b, "far operands")
+
+
 def test_linear_without_workspace_does_not_split(dev):
     """The C ABI without a workspace runs the one-launch kernel: same bound, and the workspace size
     query is 0 for a shape that fills the GPU."""
@@ -373,6 +393,17 @@ def test_qkv_rope_kv_scatter_bit_exact(dev, B, T, H, D):
                                         (16, 107, 16, 64, 1024), (16, 517, 16, 64, 1024), (4, 414, 32, 128, 4096),
                                         (1, 414, 32, 128, 4096), (16, 1029, 16, 64, 1024), (4, 1029, 32, 128, 4096)])
 def test_linear_qkv_rope_kv_fused_equals_unfused(dev, B, T, H, D, Kd):
+    _check_fused_qkv(dev, B, T, H, D, Kd)
+
+
+def test_linear_qkv_rope_kv_operands_of_4_gib(dev):
+    """The fused QKV product with input rows, and weight rows, that span 4 GiB."""
+    print("fused qkv, far operands", flush=True)
+    _check_fused_qkv(dev, 1, 7, 2, 64, 128, far=lambda x: _far(x, 1 << 29))
+    _check_fused_qkv(dev, 1, 7, 2, 64, 128, far_w=lambda w: _far(w, 1 << 23))
+
+
+def _check_fused_qkv(dev, B, T, H, D, Kd, far=lambda x: x, far_w=lambda w: w):
     """The fused QKV GEMM (qkv never materialised). Its raw bf16(acc + bias) values, taken from a run
     with no patch rows (no RoPE), are checked against the fp64 oracle like every GEMM; the pinned
     unfused RoPE kernel applied to those same values must then give the fused kernel's q and K/V
@@ -387,8 +418,8 @@ def test_linear_qkv_rope_kv_fused_equals_unfused(dev, B, T, H, D, Kd):
     tok = torch.from_numpy(toks.reshape(-1).astype(np.int64)).to(dev)
     bi = torch.arange(B).repeat_interleave(T).to(dev)
     pm, ri = tok >= 5, (tok - 5).clamp_min(0)
-    x = _rand((M, Kd), 40).to(dev)
-    w = _rand((3 * H * D, Kd), 41, 0.02).to(dev)
+    x = far(_rand((M, Kd), 40).to(dev))
+    w = far_w(_rand((3 * H * D, Kd), 41, 0.02).to(dev))
     b = _rand((3 * H * D,), 42, 0.1).to(dev)
     kv0 = _rand((B, N, 2, H, D), 43).to(dev)
     rope = (sin.to(dev), cos.to(dev))

@@ -261,3 +261,20 @@ def test_attention_buffer_load_offsets_of_a_last_tile_do_not_wrap(Dh):
     assert not K.sparse_query_attention_shape(2, 40, 3, Dh, 1, 1 << 29)[0]
     assert K.sparse_query_attention_shape(2, 40, 3, Dh, 1029, 2048)[0]
     assert K.sparse_query_attention_shape(2, 40, 3, Dh, 100, 10000000)[0]
+
+
+def test_gemm_entry_points_with_32_bit_offsets_refuse_far_operands():
+    """The 16-row and ping-pong tiles address their operands by 32-bit buffer offsets: the entry points that run
+    on them alone refuse operands of 4 GiB and more, before any launch."""
+    p16, slices = ctypes.c_void_p(16), ctypes.c_int64(0)
+    for M, lda, N, ldw in ((3, 1 << 30, 256, 64), (300, 64, 256, 1 << 23)):
+        _expect("OUDJAT_ERR_TOO_LARGE", "oudjat_linear_swiglu_nvfp4", p16, M, 64, lda, p16, N, ldw, p16, 256, 1.0, NULL,
+                1.0, NULL, p16, p16, 256, NULL)
+    for lda, ldw in ((1 << 25, 1536), (1536, 1 << 23)):
+        _expect("OUDJAT_ERR_TOO_LARGE", "oudjat_linear_splitk_partial", p16, 103, 1536, lda, p16, 384, ldw, p16, 1 << 40,
+                ctypes.addressof(slices), NULL)
+    from appcorr_amd import kernels as K
+    far = K.linear_kernel_name(1 << 20, 1024, 4096, _lib.EPI_BIAS)  # 8 GiB of input rows
+    assert "gemm_bf16_dma_kernel<128, 128" in far and "gemm_bf16_dma_kernel" not in K.linear_kernel_name(
+        1 << 18, 1024, 4096, _lib.EPI_BIAS)
+    assert K.linear_warm_slots(1 << 20, 1024, 4096, _lib.EPI_BIAS) == 0
