@@ -1776,11 +1776,20 @@ static int choose_small(int64_t M, int64_t N, int64_t K, int64_t head_dim, float
   return best < 0 ? kReg128x64 : best;
 }
 
-// Operands of 4 GiB and more are out of reach of the 32-bit buffer offsets of the 16-row and ping-pong
-// kernels: those products run on the direct-to-LDS tiles, which take 64-bit addresses.
-static bool far_operands(int64_t M, int64_t lda, int64_t N, int64_t ldw) {
+// The 16-row and ping-pong kernels read an operand [rows, K] (ld elements of eb bytes apart) by 32-bit buffer
+// offsets from a descriptor of rows * ld elements, and count on a tile's rows past the end (up to kTileRows - 1)
+// to lie past it and load as zeros. Out of reach: operands of 4 GiB and more, and rows with a gap whose offsets
+// past the end wrap, since those can land in the last row's gap, which need not be mapped (contiguous rows wrap
+// onto rows of their own; what they give is never stored).
+static constexpr int64_t kTileRows = 384;
+static bool buffer_operand(int64_t rows, int64_t ld, int64_t K, int64_t eb) {
   const int64_t limit = (int64_t)1 << 32;
-  return M * lda * 2 >= limit || N * ldw * 2 >= limit;
+  return rows * ld * eb < limit && (ld == K || (rows + kTileRows) * ld * eb <= limit);
+}
+
+// Such products run on the direct-to-LDS tiles, which take 64-bit addresses.
+static bool far_operands(int64_t M, int64_t lda, int64_t N, int64_t ldw, int64_t K) {
+  return !buffer_operand(M, lda, K, 2) || !buffer_operand(N, ldw, K, 2);
 }
 static int far_cfg(int64_t N) { return N % 128 == 0 ? kDma128x128 : kDma128x64; }
 
@@ -2027,7 +2036,7 @@ static int linear_bf16_impl(const uint16_t* A, int64_t M, int64_t K, int64_t lda
     ea.acc_scale = 1.0f;
     ea.bias = nullptr;
   }
-  if (aligned_io && far_operands(M, lda, N, ldw))
+  if (aligned_io && far_operands(M, lda, N, ldw, K))
     return launch_gemm(far_cfg(N), A, M, K, lda, W, N, ldw, epi, ea, C, ldc, as_stream(stream), "linear_bf16");
   if (workspace && aligned_io && aligned(workspace, 16)) {
     int S = 1;
@@ -2085,7 +2094,8 @@ extern "C" int oudjat_linear_swiglu_nvfp4(const uint16_t* A, int64_t M, int64_t 
   ea.b1 = b1;
   ea.b2 = b2;
   ea.xh_ts = tensor_scale;
-  OUDJAT_REQUIRE(!far_operands(M, lda, N, ldw), OUDJAT_ERR_TOO_LARGE, "%s: operands beyond 4 GiB", what);
+  OUDJAT_REQUIRE(!far_operands(M, lda, N, ldw, K), OUDJAT_ERR_TOO_LARGE, "%s: operands beyond 4 GiB (rows past the end of a tile too)",
+                 what);
   // The epilogue exists on the ping-pong tiles; shapes whose choice is another family take 192 x 256.
   int ci = choose_cfg(M, N, K, true);
   if (kCfgs[ci].fn[kEpiSwigluXh] == nullptr) ci = kPp192x256;
@@ -2105,7 +2115,8 @@ extern "C" int oudjat_linear_splitk_partial(const uint16_t* A, int64_t M, int64_
                  OUDJAT_ERR_UNSUPPORTED_LAYOUT, "linear_splitk_partial: operands must be 16-byte aligned, ld %% 8 == 0");
   OUDJAT_REQUIRE(M < ((int64_t)1 << 31) && N < ((int64_t)1 << 31) && K < ((int64_t)1 << 31), OUDJAT_ERR_TOO_LARGE,
                  "linear_splitk_partial: dimensions must fit in int32");
-  OUDJAT_REQUIRE(!far_operands(M, lda, N, ldw), OUDJAT_ERR_TOO_LARGE, "linear_splitk_partial: operands beyond 4 GiB");
+  OUDJAT_REQUIRE(!far_operands(M, lda, N, ldw, K), OUDJAT_ERR_TOO_LARGE,
+                 "linear_splitk_partial: operands beyond 4 GiB (rows past the end of a tile too)");
   int S = 1;
   const int ci = choose_splitk(M, N, K, OUDJAT_EPI_BIAS_LS, &S);
   OUDJAT_REQUIRE(ci >= 0 && S > 1 && (int64_t)S * M * N <= workspace_elems, OUDJAT_ERR_UNSUPPORTED_SHAPE,
@@ -2122,7 +2133,7 @@ extern "C" int oudjat_linear_splitk_partial(const uint16_t* A, int64_t M, int64_
 extern "C" int64_t oudjat_linear_workspace_elems(int64_t M, int64_t N, int64_t K, int epi) {
   epi &= ~OUDJAT_EPI_RAW_BF16;
   int S = 1;
-  if (M <= 0 || N <= 0 || K <= 0 || far_operands(M, K, N, K) || choose_splitk(M, N, K, epi, &S) < 0 || S <= 1)
+  if (M <= 0 || N <= 0 || K <= 0 || far_operands(M, K, N, K, K) || choose_splitk(M, N, K, epi, &S) < 0 || S <= 1)
     return 0;
   return (int64_t)S * M * N;
 }
@@ -2130,7 +2141,7 @@ extern "C" int64_t oudjat_linear_workspace_elems(int64_t M, int64_t N, int64_t K
 extern "C" int64_t oudjat_linear_warm_slots(int64_t M, int64_t N, int64_t K, int epi) {
   epi &= ~OUDJAT_EPI_RAW_BF16;
   if (M <= 0 || N <= 0 || K <= 0 || N % 64 != 0 || K % kBK != 0 || epi < OUDJAT_EPI_BIAS ||
-      epi > OUDJAT_EPI_BIAS_SILU_MUL || far_operands(M, K, N, K))
+      epi > OUDJAT_EPI_BIAS_SILU_MUL || far_operands(M, K, N, K, K))
     return 0;
   int S = 1;
   if (choose_splitk(M, N, K, epi, &S) >= 0 && S > 1) return 0;  // split launches take none
@@ -2180,7 +2191,7 @@ static int linear_qkv_rope_kv_impl(const uint16_t* A, int64_t M, int64_t K, int6
   }
   ea.qkv = QkvArgs{(int)H, (int)Dh, sin_table, cos_table, table_stride, patch_mask, rope_idx, batch_idx, token_idx,
                    kv, kv_stride_b, kv_stride_n, q_out};
-  const int ci = far_operands(M, lda, N, ldw) ? far_cfg(N) : choose_qkv_cfg(M, N, K, Dh);
+  const int ci = far_operands(M, lda, N, ldw, K) ? far_cfg(N) : choose_qkv_cfg(M, N, K, Dh);
   return launch_gemm(ci, A, M, K, lda, W, N, ldw, kEpiQkv, ea, nullptr, 0, as_stream(stream), "linear_qkv_rope_kv", 1,
                      warm, warm_bytes);
 }
@@ -2231,7 +2242,7 @@ extern "C" int oudjat_linear_kernel_name(int64_t M, int64_t N, int64_t K, int ep
   OUDJAT_REQUIRE(buf && buflen > 0, OUDJAT_ERR_INVALID_ARGUMENT, "linear_kernel_name: no buffer");
   OUDJAT_REQUIRE(M > 0 && N > 0 && K > 0 && epi >= 0 && epi <= kEpiQkv, OUDJAT_ERR_INVALID_ARGUMENT,
                  "linear_kernel_name: bad arguments");
-  if (far_operands(M, K, N, K)) return kernel_name_of(kCfgs[far_cfg(N)], epi, buf, buflen);
+  if (far_operands(M, K, N, K, K)) return kernel_name_of(kCfgs[far_cfg(N)], epi, buf, buflen);
   int S = 1;
   const int sk = epi == kEpiQkv ? -1 : choose_splitk(M, N, K, epi, &S);
   if (sk >= 0 && S > 1) epi = kEpiPartial;  // split K (with a workspace): the partial kernel, then the reduce
@@ -2279,9 +2290,9 @@ static int check_fp8_operands(const uint8_t* A, int64_t M, int64_t K, int64_t ld
                  "%s: need K %% 128 == 0 and N %% 256 == 0 (K=%lld, N=%lld)", what, (long long)K, (long long)N);
   OUDJAT_REQUIRE(lda % 16 == 0 && ldw % 16 == 0 && lda >= K && ldw >= K && aligned(A, 16) && aligned(W, 16),
                  OUDJAT_ERR_UNSUPPORTED_LAYOUT, "%s: 16-byte aligned operand rows required", what);
-  OUDJAT_REQUIRE(M < ((int64_t)1 << 31) && N < ((int64_t)1 << 31) && M * lda < ((int64_t)1 << 32) &&
-                     N * ldw < ((int64_t)1 << 32),
-                 OUDJAT_ERR_TOO_LARGE, "%s: operands beyond 4 GiB or 2^31 rows", what);
+  OUDJAT_REQUIRE(M < ((int64_t)1 << 31) && N < ((int64_t)1 << 31) && buffer_operand(M, lda, K, 1) &&
+                     buffer_operand(N, ldw, K, 1),
+                 OUDJAT_ERR_TOO_LARGE, "%s: operands beyond 4 GiB (rows past the end of a tile too) or 2^31 rows", what);
   return OUDJAT_OK;
 }
 

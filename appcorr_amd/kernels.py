@@ -292,8 +292,8 @@ def linear_ls_packed_residual(h: torch.Tensor, weight: torch.Tensor, bias: torch
     4 GiB (the caller then runs the two steps)."""
     M, Kd = h.shape
     N = weight.shape[0]
-    if not linear_splits_k(M, N, Kd) or M * h.stride(0) * 2 >= 1 << 32 or N * weight.stride(0) * 2 >= 1 << 32:
-        return None
+    if not linear_splits_k(M, N, Kd) or any((r + 384) * t.stride(0) * 2 > 1 << 32 for t, r in ((h, M), (weight, N))):
+        return None  # 32-bit operand offsets, those of a tile's rows past the end too
     tensors = [h, weight, gamma, x_act, x_attn] + ([bias] if bias is not None else [])
     if ln is not None:
         tensors += [ln[0], ln[1]]

@@ -446,7 +446,8 @@ int oudjat_linear_qkv_rope_kv_nvfp4(const uint16_t* A, int64_t M, int64_t K, int
  * and xhat [M, N] (row stride ldc) receives the NVFP4 operand of h with tensor scale *tensor_scale --
  * bit-identical to oudjat_linear_bf16 (w2, OUDJAT_EPI_BIAS) followed by oudjat_swiglu_scaled_nvfp4 when
  * both run the same tiles. b1, b2: both or neither. K % 64 == 0, N % 256 == 0; 16-byte aligned
- * operands and rows; operands of 4 GiB and more (M * lda or N * ldw) are OUDJAT_ERR_TOO_LARGE. */
+ * operands and rows; operands of 4 GiB and more (M * lda or N * ldw, with 384 rows added where rows have gaps) are
+ * OUDJAT_ERR_TOO_LARGE. */
 int oudjat_linear_swiglu_nvfp4(const uint16_t* A, int64_t M, int64_t K, int64_t lda, const uint16_t* W, int64_t N,
                                int64_t ldw, const uint16_t* x1, int64_t ld1, float s1, const uint16_t* b1,
                                float s2, const uint16_t* b2, const float* tensor_scale, uint16_t* xhat, int64_t ldc,

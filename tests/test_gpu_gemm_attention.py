@@ -229,7 +229,9 @@ def _far(t, stride):
 
 
 @pytest.mark.parametrize("M,N,Kd,lda,ldw", [(3, 384, 256, (1 << 30) + 8, 0), (103, 384, 1536, 1 << 25, 0),
-                                            (9, 128, 256, 0, 1 << 24), (5, 192, 128, 0, 1 << 24)])
+                                            (9, 128, 256, 0, 1 << 24), (5, 192, 128, 0, 1 << 24),
+                                            # 3 * 10^9 bytes: the tile's rows past the end would wrap
+                                            (3, 384, 256, 500000000, 0), (103, 384, 1536, 16000000, 0)])
 def test_linear_operands_of_4_gib(dev, M, N, Kd, lda, ldw):
     """A few rows so far apart that the operand spans 4 GiB: past 32-bit buffer offsets the direct-to-LDS tiles
     run, also where the shape would split K or run on 16-row tiles, within the accumulation bound of the oracle."""

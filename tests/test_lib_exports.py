@@ -278,3 +278,20 @@ def test_gemm_entry_points_with_32_bit_offsets_refuse_far_operands():
     assert "gemm_bf16_dma_kernel<128, 128" in far and "gemm_bf16_dma_kernel" not in K.linear_kernel_name(
         1 << 18, 1024, 4096, _lib.EPI_BIAS)
     assert K.linear_warm_slots(1 << 20, 1024, 4096, _lib.EPI_BIAS) == 0
+
+
+def test_gemm_buffer_offsets_of_rows_past_the_end_do_not_wrap():
+    """Operands below 4 GiB whose rows have gaps: a tile's rows past the end would wrap 32 bits into the last
+    row's gap (row 7 of rows of 10^9 bytes lands 2.7 * 10^9 bytes in, past the third and last row). Refused where
+    no 64-bit tile exists, bf16 and FP8."""
+    p16, slices = ctypes.c_void_p(16), ctypes.c_int64(0)
+    gap = 500000000
+    assert 2 * gap * 2 < (7 * gap * 2) % (1 << 32) < 3 * gap * 2 < 1 << 32
+    for M, lda, N, ldw in ((3, gap, 256, 64), (300, 64, 256, 4000000)):
+        _expect("OUDJAT_ERR_TOO_LARGE", "oudjat_linear_swiglu_nvfp4", p16, M, 64, lda, p16, N, ldw, p16, 256, 1.0, NULL,
+                1.0, NULL, p16, p16, 256, NULL)
+    _expect("OUDJAT_ERR_TOO_LARGE", "oudjat_linear_splitk_partial", p16, 103, 1536, 8000000, p16, 384, 1536, p16, 1 << 40,
+            ctypes.addressof(slices), NULL)
+    for lda, ldw in ((2 * gap, 128), (128, 8000000)):
+        _expect("OUDJAT_ERR_TOO_LARGE", "oudjat_linear_fp8", p16, 3, 128, lda, p16, 256, ldw, NULL, _lib.EPI_BIAS, NULL,
+                NULL, 0, p16, 256, 1.0, NULL)
