@@ -615,7 +615,8 @@ class SelfAttentionBlock(nn.Module):
     def _candidate_scores(self, B: int, N: int, cache_feature: Dict, tag: str, kw: dict, dind: Tensor,
                           num_pretokens: int) -> "K.CandidateScores | None":
         """The same scores as the plan kernels' source, or None where they do not apply: scores that are not
-        fp32 rows on dindice's device, a hint of a width that the elementwise path refuses, no candidates."""
+        fp32 rows on dindice's device, a hint of a width that the elementwise path refuses, no images or no
+        candidates."""
         hint, fusion, hint_off = None, _lib.FUSION_SERVER, 0
         if (kw["mobile_pscore"] in self._MOBILE_HINT_PSCORE_ALIASES and kw["mobile_pscore_weight"] != 0.0
                 and kw["mobile_pscore_hint"] is not None):
@@ -633,7 +634,7 @@ class SelfAttentionBlock(nn.Module):
         server = None
         if kw["server_pscore_weight"] != 0.0:
             server = self._resolve_server_token_scores(cache_feature, tag, kw["server_pscore"])
-        if dind.dtype != torch.long or dind.dim() != 2 or dind.shape[1] <= num_pretokens or not (
+        if dind.dtype != torch.long or dind.dim() != 2 or dind.shape[0] == 0 or dind.shape[1] <= num_pretokens or not (
                 dind.is_cuda and K.CandidateScores.takes(server, B, dind.device)
                 and K.CandidateScores.takes(hint, B, dind.device)):
             return None

@@ -169,3 +169,31 @@ def test_plan_scores_equal_elementwise_steps(dev, B, P, gh, k, fusion, server, h
                  "active_rope_idx", "keep_mask", "row_slot"):
         assert torch.equal(getattr(tp, name), getattr(ref, name)), name
     assert bool(valid.all()) and valid.shape == (B, npre + k)
+
+
+@pytest.mark.parametrize("B", [0, 1])
+@pytest.mark.parametrize("kw", [dict(), dict(server_pscore_weight=0.0), dict(token_keep_thres=-1.0, token_keep_cap=16),
+                                dict(server_pscore_weight=0.0, token_keep_thres=-1.0, token_keep_cap=16),
+                                dict(server_pscore_weight=0.0, token_keep_thres=-1.0),
+                                dict(server_pscore_weight=0.0, mobile_pscore="residual_energy",
+                                     mobile_pscore_weight=1.0)])
+def test_correction_of_no_images(dev, B, kw):
+    """An empty batch corrects to an empty batch with every kind of selection, with scores and without; one image
+    of zero tokens beside it."""
+    from appcorr_amd.dinov3 import SelfAttentionBlock
+    N, C = 201, 384
+    print(f"correction of {B} images {sorted(kw)}", flush=True)
+    blk = SelfAttentionBlock(C, 6, ffn_ratio=4.0, qkv_bias=True, init_values=1.0, mask_k_bias=True)
+    blk = blk.to(device=dev, dtype=torch.bfloat16)
+    for t in (*blk.parameters(), *blk.buffers()):  # they come uninitialised
+        t.data.zero_()
+    x = torch.zeros(B, N, C, device=dev, dtype=torch.bfloat16)
+    rope = (torch.zeros(N - 5, 64, device=dev), torch.ones(N - 5, 64, device=dev))
+    cache = {"layer0_kv": x.new_zeros(B, N, 2, 6, 64), "layer0_blocks_out_sum": torch.zeros_like(x),
+             "layer0_server_pscore": torch.zeros(B, N, device=dev)}
+    dind = torch.arange(N, device=dev).unsqueeze(0).expand(B, -1).contiguous()
+    if "mobile_pscore" in kw:
+        kw = dict(kw, mobile_pscore_hint=torch.zeros(B, N - 5, device=dev))
+    with torch.no_grad():
+        y, _ = blk.correct(x, dind, rope, cache, "layer0", token_keep_ratio=0.5, **kw)
+    assert y.shape == x.shape and bool(torch.isfinite(y).all())
