@@ -1105,20 +1105,26 @@ static AttnShape attn_shape(int64_t B, int64_t T, int64_t H, int64_t Dh, int64_t
   const int64_t waves = cdiv(T, 32);
   s.dma = rows_fit;  // the register-staged kernel takes any strides
   s.kv_parts = 1;
+  // Dh = 128, at most four query waves, more pairs than CUs: the register-staged kernel, whose 64 KB of LDS put two
+  // workgroups on a CU where the buffer loads' 128 KB put one. Measured (buffer loads -> staged, us; B x 32
+  // heads, T of N): 9 x 30 of 4101 203 -> 127, 12 x 62 of 1605 92 -> 68, 16 x 126 of 4101 254 -> 212; up to
+  // one workgroup per CU the buffer loads win (8 x 126 of 1605 45.8 -> 42.0), and with five waves and more.
+  if (Dh == 128 && waves <= kMinWaves && B * H > kNumCus) s.dma = false;
   if (!s.dma) {
     s.n_wg = cdiv(waves, Dh == 64 ? kMaxWaves64 : kMaxWaves128);
     s.w = (int)std::max<int64_t>(cdiv(waves, s.n_wg), kMinWaves);
     return s;
   }
   if (Dh == 128) {
-    // One workgroup per CU (128 KB of LDS). A key tile takes about 1.2 us with one wave per SIMD and 1.7 to
-    // 1.9 with two (five to eight waves), measured over 17 .. 65 tiles; the fewest rounds of those wins.
+    // One workgroup per CU (128 KB of LDS). A key tile takes about 1.25 us with one wave per SIMD and 1.7 to
+    // 1.85 with two (five to eight waves), measured over 17 .. 65 tiles; the fewest rounds of those wins.
     // 1 x 32 heads, 200 queries of 1029 keys: two workgroups of four waves 25.4 us, one of seven 33.1;
-    // 3 x 32, 700 of 1029: five of five 65.6, three of eight 71.5.
+    // 3 x 32, 700 of 1029: five of five 65.6, three of eight 71.5; 9 .. 12 x 32, 256 of 4101: two rounds of
+    // eight waves 242 .. 262, three of four waves 300 .. 316.
     double best = -1.0;
     for (int w = kMinWaves; w <= kMaxWaves128; ++w) {
       const int64_t n = cdiv(waves, w);
-      const double us = (double)cdiv(B * H * n, kNumCus) * (w == kMinWaves ? 1.2 : 1.7 + 0.05 * (w - 5));
+      const double us = (double)cdiv(B * H * n, kNumCus) * (w == kMinWaves ? 1.25 : 1.7 + 0.05 * (w - 5));
       if (best >= 0.0 && us >= best) continue;
       best = us;
       s.n_wg = n;

@@ -607,10 +607,12 @@ def test_attention_one_key_with_a_large_row_stride(dev, T, D):
 
 
 @pytest.mark.parametrize("B,T,N,H,pad", [(1, 200, 261, 7, 0), (2, 257, 65, 3, 8), (1, 128, 64, 9, 0), (3, 700, 129, 5, 0),
-                                         (16, 257, 193, 16, 0), (1, 1, 1, 1, 0), (1, 40, 130, 1, 1 << 23)])
+                                         (16, 257, 193, 16, 0), (1, 1, 1, 1, 0), (1, 40, 130, 1, 1 << 23),
+                                         (9, 97, 129, 32, 0), (9, 222, 65, 32, 0)])
 def test_attention_dh128_buffer_loads(dev, B, T, N, H, pad):
     """Dh = 128: four and eight loader waves, one to 256 pairs, one key past a tile, padded key rows; the
-    last case's key rows lie past the 31-bit byte offsets (the register-staged kernel). The output equals
+    case of padding 2^23 has its key rows past the 31-bit byte offsets, and 288 pairs of four query waves take the
+    register-staged kernel too. The output equals
     the register-staged kernel's (the log-sum-exp entry) bit for bit, and that one is within the bound of
     the float64 reference."""
     D = 128

@@ -239,7 +239,7 @@ def test_attention_buffer_loads_only_for_rows_the_descriptor_covers(Dh):
     from appcorr_amd import kernels as K
     H, N = 4, 300
     for T in (1, 33, 300, 1000):
-        for B in (1, 16, 100):
+        for B in (1, 16, 60):
             assert K.sparse_query_attention_shape(B, T, H, Dh, N, 2 * H * Dh)[0]
             assert K.sparse_query_attention_shape(B, T, H, Dh, N, Dh)[0]          # one head's rows back to back
             for kvn in (0, 8, Dh - 8, -2 * H * Dh):
@@ -295,3 +295,21 @@ def test_gemm_buffer_offsets_of_rows_past_the_end_do_not_wrap():
     for lda, ldw in ((2 * gap, 128), (128, 8000000)):
         _expect("OUDJAT_ERR_TOO_LARGE", "oudjat_linear_fp8", p16, 3, 128, lda, p16, 256, ldw, NULL, _lib.EPI_BIAS, NULL,
                 NULL, 0, p16, 256, 1.0, NULL)
+
+
+def test_attention_dh128_shapes_where_pairs_outnumber_the_cus():
+    """Dh = 128: calls of at most four query waves and more than 256 (image, head) pairs take the register-staged
+    kernel (two workgroups per CU); seven or eight query waves of 257 .. 384 pairs stay in one workgroup (two
+    rounds) and are not split into three rounds of four waves."""
+    from appcorr_amd import kernels as K
+
+    def shape(B, T, N=4101, H=32):
+        return K.sparse_query_attention_shape(B, T, H, 128, N, 2 * H * 128)[:4]
+
+    for T in (1, 30, 62, 97, 128):
+        assert shape(8, T) == (True, 1, 4, 4), T
+        for B in (9, 12, 16):
+            assert shape(B, T) == (False, 1, 4, 4), (B, T)
+    for B in (9, 10, 12):
+        assert shape(B, 222) == (True, 1, 7, 7) and shape(B, 256) == (True, 1, 8, 8)
+        assert shape(B, 150) == (True, 1, 5, 5)
