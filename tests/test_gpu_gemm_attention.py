@@ -398,6 +398,36 @@ def test_linear_qkv_rope_kv_fused_equals_unfused(dev, B, T, H, D, Kd):
     _check_fused_qkv(dev, B, T, H, D, Kd)
 
 
+# Every tile below the ping-pong ones that the fused QKV choice can return (the kernel's name is part of the
+# case), row counts off a multiple of the tile's.
+QKV_TILES = [(2, 33, 2, 64, 192, "dma_kernel<64, 64, 2, 2, 5>"), (5, 131, 24, 64, 128, "dma_kernel<128, 64, 2, 2, 5>"),
+             (16, 517, 6, 64, 192, "dma_kernel<128, 128, 2, 2, 5>"),
+             (1, 33, 2, 64, 128, "r16_kernel<32, 64, 1, 4, 2, 128, 2, false, 5>"),
+             (1, 103, 6, 64, 1024, "r16_kernel<32, 64, 1, 4, 2, 128, 2, false, 5>"),
+             (1, 700, 4, 64, 384, "r16_kernel<64, 64, 1, 4, 2, 128, 2, false, 5>"),
+             (2, 45, 2, 64, 1536, "r16_kernel<64, 64, 1, 4, 2, 128, 3, false, 5>"),
+             (1, 331, 16, 64, 512, "r16_kernel<96, 64, 1, 4, 2, 128, 2, false, 5>"),
+             (2, 33, 2, 64, 1216, "r16_kernel<64, 128, 1, 4, 2, 64, 4, true, 5>"),
+             (9, 103, 24, 64, 512, "r16_kernel<144, 128, 1, 4, 2, 128, 2, false, 5>"),
+             (5, 261, 16, 64, 1024, "r16_kernel<144, 128, 1, 4, 2, 128, 2, false, 5>"),
+             (5, 261, 24, 64, 2048, "r16_kernel<128, 256, 2, 4, 1, 64, 3, false, 5>")]
+
+
+@pytest.mark.parametrize("B,T,H,D,Kd,kernel", QKV_TILES)
+def test_linear_qkv_rope_kv_tiles(dev, B, T, H, D, Kd, kernel):
+    print(f"fused qkv tile {B}x{T} {H}x{D} K={Kd} {kernel}", flush=True)
+    name = K.linear_kernel_name(B * T, 3 * H * D, Kd, 5)
+    assert kernel in name, name
+    _check_fused_qkv(dev, B, T, H, D, Kd)
+
+
+@pytest.mark.parametrize("B,T,H,Kd", [(1, 33, 2, 128), (2, 45, 3, 1216), (3, 131, 5, 512), (9, 61, 8, 256)])
+def test_linear_qkv_rope_kv_small_tiles_of_128_wide_heads(dev, B, T, H, Kd):
+    """Dh = 128: of the small tiles only those that hold a whole head."""
+    print(f"fused qkv {B}x{T} {H}x128 K={Kd}", flush=True)
+    _check_fused_qkv(dev, B, T, H, 128, Kd)
+
+
 def test_linear_qkv_rope_kv_operands_of_4_gib(dev):
     """The fused QKV product with input rows, and weight rows, that span 4 GiB."""
     print("fused qkv, far operands", flush=True)
