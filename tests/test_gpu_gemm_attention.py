@@ -589,6 +589,32 @@ def test_attention_launch_shapes(dev, B, T, N, H):
     _check_attention(got.cpu(), qb, kv, D ** -0.5, o64.transpose(1, 2).reshape(B * T, H * D), f"shape {B},{T},{N},{H}")
 
 
+# One case per kind of launch the shape model gives at Dh = 64, with the launch it must be: (query workgroups per
+# pair, query waves, waves, light parts, key parts), every number of key parts among them.
+LAUNCHES = [(8, 1, 450, 12, (1, 1, 4, 0, 2)), (5, 1, 450, 16, (1, 1, 4, 0, 3)), (1, 1, 201, 1, (1, 1, 4, 0, 4)),
+            (1, 33, 300, 1, (2, 1, 4, 0, 5)), (1, 33, 700, 1, (2, 1, 4, 0, 6)), (1, 33, 833, 1, (2, 1, 4, 0, 7)),
+            (1, 33, 450, 1, (2, 1, 4, 0, 8)), (3, 130, 580, 6, (2, 3, 4, 0, 5)), (3, 200, 580, 16, (2, 4, 4, 0, 2)),
+            (16, 70, 1, 12, (1, 3, 4, 0, 1)), (5, 150, 833, 16, (1, 5, 5, 0, 2)), (5, 517, 201, 12, (4, 5, 5, 0, 1)),
+            (8, 330, 300, 12, (2, 6, 6, 0, 1)), (16, 200, 201, 12, (1, 7, 7, 0, 1)), (2, 400, 4101, 12, (2, 7, 7, 0, 5)),
+            (5, 700, 450, 16, (3, 8, 8, 0, 1)), (5, 1029, 1, 12, (4, 9, 9, 0, 1)), (16, 261, 1, 12, (1, 9, 9, 0, 1)),
+            (16, 300, 1, 12, (1, 10, 10, 0, 1)), (8, 300, 1029, 12, (1, 10, 10, 0, 2)), (8, 700, 1, 12, (2, 11, 11, 0, 1)),
+            (5, 1500, 1, 12, (4, 12, 12, 0, 1)), (16, 103, 700, 16, (1, 4, 7, 4, 1)), (5, 103, 2305, 16, (1, 4, 7, 4, 3)),
+            (16, 130, 130, 12, (1, 5, 8, 4, 1)), (5, 130, 833, 16, (1, 5, 8, 4, 2)), (16, 261, 130, 12, (1, 9, 12, 4, 1))]
+
+
+@pytest.mark.parametrize("B,T,N,H,launch", LAUNCHES)
+def test_attention_each_launch_shape(dev, B, T, N, H, launch):
+    """Every kind of launch, pinned, against the float64 reference."""
+    D = 64
+    print(f"attention launch {B},{T},{N},{H} {launch}", flush=True)
+    assert K.sparse_query_attention_shape(B, T, H, D, N, 2 * H * D) == (True, *launch)
+    q, kv = _rand((B * T, H, D), 54), _rand((B, N, 2, H, D), 55)
+    got = K.sparse_query_attention(q.to(dev), kv.to(dev), T, D ** -0.5)
+    qb = q.reshape(B, T, H, D).transpose(1, 2)
+    o64 = F64.sdpa(qb, kv[:, :, 0].transpose(1, 2), kv[:, :, 1].transpose(1, 2), D ** -0.5)
+    _check_attention(got.cpu(), qb, kv, D ** -0.5, o64.transpose(1, 2).reshape(B * T, H * D), f"launch {launch}")
+
+
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("stride", ["broadcast", "overlapping", "backwards"])
 @pytest.mark.parametrize("B,T,N,H", [(2, 40, 130, 3), (1, 300, 261, 2), (2, 107, 1029, 4)])
