@@ -402,8 +402,8 @@ __global__ __launch_bounds__((DH == 64 ? kMaxWaves64 : kMaxWaves128) * 64) void 
 // The arithmetic (MFMA order, softmax, P rounding) is that of sq_attention_kernel, so both give
 // bit-identical outputs.
 // Dh = 128, measured against the register-staged kernel (two stages, a barrier with nothing issued across
-// it, two-way bank conflicts of the V reads): 4 x 32 heads, 4101 of 4101 1343 -> 1100 us, 414 of 4101 150 ->
-// 128. The matrix cores are busy half of the cycles there and the VALU (softmax) half, and the clock falls
+// it, two-way bank conflicts of the V reads): 4 x 32 heads, 4101 of 4101 1259 -> 1068 us, 414 of 4101 146 ->
+// 133. The matrix cores are busy half of the cycles there and the VALU (softmax) half, and the clock falls
 // from 1.9 to 1.75 GHz as they overlap more.
 // ------------------------------------------------------------------------------------------------
 
@@ -428,7 +428,7 @@ __device__ __forceinline__ int tile_slot(int row, int chunk) {
 
 // light_split: 0, or kLightParts when the launch has one workgroup per (image, head) whose last
 // query wave is light; that wave's work is then done by kLightParts waves (the last ones), part p
-// taking the key tiles t with t % NST == p, and merged at the end (see the light path below).
+// taking keys 16 p .. 16 p + 15 of every tile, and merged at the end (see the light path below).
 // Key-part workspace of a split launch, per (image, head, part): the running max of each query
 // (kv_part_rows(T) floats, T rounded up to 4 so the rows below stay 16-byte aligned), its sum (as
 // many), then its unnormalised 64-dim output rows (T x 64).
@@ -1072,8 +1072,11 @@ struct AttnShape {
 // when a light one is split) over L key tiles each, reading `streams` distinct K/V ranges; light: the last
 // query wave has 1..16 queries. Up to four waves, a wave runs alone on its SIMD and two workgroups share a
 // CU; above, one workgroup holds the CU and the SIMD with the most waves sets the pace per tile (a step at
-// every multiple of four). Fitted to sweeps over 100 shapes of 4 .. 65 tiles (below one round of workgroups
-// of up to four waves, 640 points, within 3 % rms); it only ranks the shapes of one call.
+// every multiple of four). Fitted to sweeps over 100 shapes of 4 .. 65 tiles, within 3 % rms below one round
+// of workgroups of up to four waves and less closely above; it only ranks the shapes of one call. Against every
+// other launch of 110 shapes (B 1 .. 16, 6 .. 16 heads, 200 .. 4101 keys) its choice is 1.5 % off the fastest
+// in the geometric mean, 4 % at the 90th percentile, 30 % at most (4 x 12 heads, 264 of 1041: 20.2 us in two
+// key parts, 15.6 as five workgroups of two waves).
 static double attn_wg_us(int64_t wgs, int64_t streams, int w, int waves, bool light, int64_t L) {
   if (waves <= 4) {
     const double u = std::min(1.0, (double)streams / kNumCus), lt = light ? 0.08 : 0.0;
@@ -1118,8 +1121,8 @@ static AttnShape attn_shape(int64_t B, int64_t T, int64_t H, int64_t Dh, int64_t
   if (Dh == 128) {
     // One workgroup per CU (128 KB of LDS). A key tile takes about 1.25 us with one wave per SIMD and 1.7 to
     // 1.85 with two (five to eight waves), measured over 17 .. 65 tiles; the fewest rounds of those wins.
-    // 1 x 32 heads, 200 queries of 1029 keys: two workgroups of four waves 25.4 us, one of seven 33.1;
-    // 3 x 32, 700 of 1029: five of five 65.6, three of eight 71.5; 9 .. 12 x 32, 256 of 4101: two rounds of
+    // 1 x 32 heads, 200 queries of 1029 keys: two workgroups of four waves 25.4 us, one of seven 33.1 (39.4
+    // register-staged); 3 x 32, 700 of 1029: five of five 65.6, three of eight 71.5 (81.6 register-staged); 9 .. 12 x 32, 256 of 4101: two rounds of
     // eight waves 242 .. 262, three of four waves 300 .. 316.
     double best = -1.0;
     for (int w = kMinWaves; w <= kMaxWaves128; ++w) {
@@ -1139,11 +1142,12 @@ static AttnShape attn_shape(int64_t B, int64_t T, int64_t H, int64_t Dh, int64_t
   // parts: the key tiles of each query workgroup dealt to 2 .. kMaxKvParts workgroups in contiguous ranges,
   // whose fp32 rows a merge launch combines (2 us and their bytes); always for few pairs of up to ten waves
   // and many tiles, else where it is modelled faster.
-  // Measured (HIP graph, before -> after; B x heads, queries of keys): 16 x 16, 1029 of 1029 132 -> 110 us
-  // (four workgroups of nine waves -> three of eleven); 16 x 16, 330 of 1029 65.5 -> 38.8 (two of six -> one of
-  // eleven); 3 x 12, 384 of 764 21.2 -> 12.1 (two of six, register-staged -> six of two); 1 x 16, 1500 of 4101
-  // 96 -> 50; 16 x 16, 107 of 1029 25.0 -> 19.9 (two waves per full query wave -> one); 2 x 6, 200 of 1000
-  // 26.2 -> 10.0 (four key parts); 1 x 6, 103 of 201 8.3 -> 6.0 (one of four -> four of one).
+  // Measured (HIP graph, evenly filled workgroups of four to ten waves -> this choice, in turn on one card; B x
+  // heads, queries of keys): 16 x 16, 1029 of 1029 122 -> 104 us (four workgroups of nine waves -> nine of four;
+  // three of eleven are level with those); 16 x 16, 330 of 1029 62.2 -> 34.7 (two of six -> one of eleven);
+  // 3 x 12, 384 of 764 20.8 -> 11.7 (two of six, register-staged -> six of two); 1 x 16, 1500 of 4101 95.6 ->
+  // 46.6; 16 x 16, 107 of 1029 23.9 -> 18.4 (two waves per full query wave -> one); 2 x 6, 200 of 1000 26.2 ->
+  // 10.0 (four key parts); 1 x 6, 103 of 201 8.3 -> 5.9 (one of four -> four of one).
   const int64_t pairs = B * H, L = cdiv(N, kKeyTile);
   const int64_t few = std::min<int64_t>(std::min<int64_t>(kNumCus / std::max<int64_t>(pairs, 1), L), kMaxKvParts);
   const bool must_split = waves <= 10 && 2 * pairs <= kNumCus && few >= 2 && L - cdiv(L, few) >= kMinTilesSaved;

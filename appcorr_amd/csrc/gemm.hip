@@ -5,13 +5,13 @@
 // row of A and one row of W, i.e. one 16-byte LDS read per operand per MFMA.
 //
 // Kernel families (templates over the workgroup tile BM x BN and the WGM x WGN wave grid):
-//   * gemm_bf16_pp_kernel: 288-row tiles (M = B (5 + k) = 4176 = 14.5 x 288 at the headline shape)
-//     with 8 waves in two groups that alternate between MFMA-only and LDS-read phases; fc1 and the
-//     fused QKV projection.
-//   * gemm_bf16_r16_kernel: 144- and 288-row tiles on 16x16x32 MFMAs with optional split K inside
-//     the workgroup; the N = C projections.
-//   * gemm_bf16_dma_kernel: direct-to-LDS loads, K tiles of 64; 64- to 128-wide tiles with 4 waves,
-//     several workgroups per CU.
+//   * gemm_bf16_pp_kernel: 192- to 288-row tiles (FP8 operands also 128; M = B (5 + k) = 4176 = 14.5 x 288 at the headline
+//     shape) with 8 waves in two groups that alternate between MFMA-only and LDS-read phases; one round or
+//     more of large tiles (fc1 and the fused QKV projection of the headline).
+//   * gemm_bf16_r16_kernel: 32- to 144-row tiles on 16x16x32 MFMAs with optional split K inside
+//     the workgroup; the headline's N = C projections and products below a round of large tiles.
+//   * gemm_bf16_dma_kernel: direct-to-LDS loads, K tiles of 64; 32- to 128-wide tiles with 4 waves,
+//     several workgroups per CU; small products, and operands past 32-bit offsets.
 //   * gemm_bf16_kernel: register-staged loads with 16-byte-aligned fallbacks (any N % 64 == 0, any
 //     output alignment).
 // Common to all:
@@ -774,16 +774,16 @@ __global__ __launch_bounds__(WGM * WGN * 64) void gemm_bf16_dma_kernel(const uin
 }
 
 // ------------------------------------------------------------------------------------------------
-// 16-row-block kernel for M = 144 k-multiples. The correction pass's GEMMs have M = B * (5 + k)
-// rows (4176 = 29 x 144 at the headline shape), which 256-row tiles cover badly (17 tile rows, the
-// last one 31 % full). Tiles of 144 rows (9 blocks of 16) on v_mfma_f32_16x16x32_bf16 cover it
-// exactly: fc1 as 29 x 8 tiles of 144 x 512, the N = C GEMMs as 29 x 8 tiles of 144 x 128 -- 232
-// workgroups, one round on 256 CUs.
+// 16-row-block kernel: tiles of 32, 64, 96, 128 or 144 rows on v_mfma_f32_16x16x32_bf16. The correction pass's
+// GEMMs have M = B * (5 + k) rows (4176 = 29 x 144 at the headline shape), which 256-row tiles cover badly (17
+// tile rows, the last one 31 % full); tiles of 144 rows (9 blocks of 16) cover it exactly, the N = C GEMMs as
+// 29 x 8 tiles of 144 x 128 -- 232 workgroups, one round on 256 CUs. The smaller tiles fill the CUs where M is
+// small (choose_small).
 //   * Waves form a WGM x WGN grid of BM / WGM-row, BN / WGN-column wave tiles; with KSPLIT = 2 two
 //     such grids take alternate 32-deep halves of each K tile (doubling the waves per CU for the
-//     narrow N = C tiles) and are summed through LDS at the end. With WGM = 2 (288-row tiles of two
-//     144-row halves) the epilogue stages one half at a time through LDS.
-//   * K tiles of BK (32 or 64) in NST LDS stages, direct-to-LDS loads issued NST - 1 tiles ahead,
+//     narrow tiles) and are summed through LDS at the end. With WGM = 2 (128 x 256 tiles of two
+//     64-row halves) the epilogue stages one half at a time through LDS.
+//   * K tiles of BK (64 or 128) in NST LDS stages, direct-to-LDS loads issued NST - 1 tiles ahead,
 //     fragments read one K tile ahead of their MFMAs, one barrier per K tile.
 //   * Rows are 2 * BK bytes; chunk c of row r sits at 16-byte slot c ^ ((r / L) % CPRW) with
 //     L = rows per 256-byte bank line and CPRW = chunks per row, so a fragment read (16 rows at one
@@ -1528,8 +1528,8 @@ typedef void (*gemm_fn)(const uint16_t*, int, int, int64_t, const uint16_t*, int
 
 struct GemmCfg {
   int bm, bn, wgm, wgn, pf;  // pf: register prefetch depth; 0 = direct-to-LDS; -2 = 16-row; -3 / -4 = ping-pong
-  gemm_fn fn[kNumEpi];       // by epilogue; fn[kEpiQkv] only for the direct-to-LDS families, fn[kEpiPartial]
-                             // only for the 16-row-block family
+  gemm_fn fn[kNumEpi];       // by epilogue (null: none); fn[kEpiQkv] for all but the register-staged kernel,
+                             // fn[kEpiPartial] for the 16-row and ping-pong kernels
   int bk, nst, ks;           // 16-row kernel: K tile depth, LDS stages, K groups
   int fb;                    // 16-row kernel: fragments read one K tile ahead
 };
@@ -1721,11 +1721,16 @@ static int choose_large(int64_t M, int64_t N, int64_t K) {
 // one whose time comes out least in
 //     us = fix[n] + (per_k[n] + fill[n] * (w / 256 - (n - 1))) * depth,   n = ceil(w / 256) rounds,
 // w = workgroups (output tiles x K slices), depth = K / slices. The figures are fits over 24 row counts
-// (64 .. 16464) x the 16 layer shapes of the four backbones (weights from HBM, activations cached), 3-9 %
-// off the single measurement; several workgroups share a CU where their LDS allows, hence one row per n.
-// Over those 384 products the choice is 1.19x faster in the geometric mean than the earlier rule (128 x 128
-// tiles for most of them) and 4 % off the fastest tile measured for each: 1152 x 768 x 3072 35.6 -> 14.7 us,
-// 800 x 768 x 768 12.0 -> 6.9, 224 x 3072 x 1024 14.3 -> 8.1, 400 x 4096 x 4096 32.4 -> 28.9.
+// (64 .. 16464) x the 16 layer shapes of the four backbones (weights from HBM, activations cached); several
+// workgroups share a CU where their LDS allows, hence one row per n. Over those 384 products the choice is
+// 1.19x faster in the geometric mean than the earlier rule (128 x 128 tiles for most of them): 1152 x 768 x
+// 3072 35.6 -> 14.7 us, 800 x 768 x 768 12.0 -> 6.9, 224 x 3072 x 1024 14.3 -> 8.1, 400 x 4096 x 4096 32.4 ->
+// 28.9. Measured again over 20 row counts (64 .. 12001) with every tile and slice count the model puts within
+// twice its best: the choice is 3.7 % off the fastest in the geometric mean (level at the median, 14 % at the
+// 90th percentile, 27 % at most: 2500 x 768 x 3072, always split, 29.3 us against 23.0), and the model's times
+// are 0.84 (64 x 64 direct-to-LDS) to 1.00 of the measured ones with a spread of 4 to 9 % per tile.
+// The tiles differ in the order of their fp32 sums over K (K groups, slices), so the choice moves an output by
+// a bf16 step here and there; the error against 64 bits is that of the 128 x 128 tiles.
 struct SmallTile {
   int ci, max_n;
   float fix[4], per_k[4], fill[4];
@@ -1810,9 +1815,9 @@ static int choose_cfg(int64_t M, int64_t N, int64_t K, bool aligned_io) {
 //   * 288 x 256 ping-pong tiles in slices at least 4096 deep (ViT-7B w3, 1656 x 4096 x 8192: 138 -> 128 us;
 //     with shallower slices the partial stores and the reduce cost more than the halved operand stream
 //     saves: ViT-L fc2 49 -> 68 us, ViT-7B proj 78 -> 90 us);
-//   * K in two to four slices at least 1024 deep of a product of 33 to 127 tiles of 144 x 128 (the fc2 of
-//     ViT-B, and of ViT-L at keep 10 %, whose reduce runs in the residual step), on the tile and slice count
-//     of least modelled time;
+//   * products of 33 to 127 tiles of 144 x 128 that two to four slices at least 1024 deep would bring to 160 to
+//     256 (the fc2 of ViT-B, and of ViT-L at keep 10 %, whose reduce runs in the residual step): always split,
+//     on the small tile and the slice count (2 to 16, two K tiles deep or more) of least modelled time;
 //   * any other product with K >= 1024 whose split is modelled faster than its one launch (ViT-S at B = 1
 //     fc2, 103 x 384 x 1536: 13.5 us in 12 slices of 144 x 128 tiles, 8.6 in 6 of 32 x 64).
 static int choose_splitk(int64_t M, int64_t N, int64_t K, int epi, int* S_out) {
@@ -1820,7 +1825,7 @@ static int choose_splitk(int64_t M, int64_t N, int64_t K, int epi, int* S_out) {
   if (N % 128 != 0 || epi >= kEpiQkv) return -1;
   const int64_t t288 = N % 256 == 0 ? cdiv(M, 288) * (N / 256) : 0;
   const int64_t t144 = cdiv(M, 144) * (N / 128);
-  int deep = 1, mid = 1;  // the slice counts the first two rules find
+  int deep = 1, mid = 1;  // the slice count of the first rule; the second rule applies when mid > 1
   for (int S = 4; S >= 2; --S) {
     if (deep == 1 && t288 > 0 && t288 < 128 && S * t288 <= kNumCus && S * t288 >= 160 && K % (S * 64) == 0 &&
         K / S >= 4096)
@@ -1903,16 +1908,17 @@ static int choose_cfg_fp8(int64_t M, int64_t N) {
   return kPp8_128x256;
 }
 
-// Launches configuration `ci` with epilogue `epi` (arguments already validated).
-// Warming workgroups a launch of configuration `cfg` with this many tiles (unsplit) carries: one per
-// CU its tiles leave idle, for the 16-row and ping-pong kernels (one workgroup per CU).
+// Warming workgroups a launch of configuration `cfg` with this many tiles (unsplit) carries, for the 16-row and
+// ping-pong kernels: one per CU that a round of one workgroup each leaves idle (the small 16-row tiles may
+// share a CU; dispatch fills idle CUs first, and a warming workgroup that shares one only reads).
 static int64_t warm_slots(const GemmCfg& cfg, int64_t tiles) {
   return (cfg.pf == -2 || cfg.pf == -3) && tiles < kNumCus ? kNumCus - tiles : 0;
 }
 
+// Launches configuration `ci` with epilogue `epi` (arguments already validated).
 // warm / warm_bytes: a region (4-byte aligned) to read into the caches from the CUs an unsplit launch
-// of fewer tiles than CUs leaves idle (one workgroup per CU: the kernels that take it hold a CU's
-// registers or LDS), for the launch after the next that reads it; ignored by the other kernels.
+// of fewer tiles than CUs leaves idle (warm_slots), for a later launch that reads it; ignored by the
+// other kernels.
 static int launch_gemm(int ci, const uint16_t* A, int64_t M, int64_t K, int64_t lda, const uint16_t* W, int64_t N,
                        int64_t ldw, int epi, const EpiArgs& ea_in, uint16_t* C, int64_t ldc, hipStream_t stream,
                        const char* what, int splits = 1, const void* warm = nullptr, int64_t warm_bytes = 0) {

@@ -466,8 +466,8 @@ int oudjat_sparse_query_attention(const uint16_t* q, int64_t q_row_stride, int64
                                   oudjat_stream_t stream);
 
 /* Row 10 with a workspace (the same SDPA call site, attention.py:456-532): the same result as
- * oudjat_sparse_query_attention, except that when few (image, head) pairs would leave most CUs idle
- * (Dh = 64, B*H at most half the CU count) the keys are split into contiguous ranges over several
+ * oudjat_sparse_query_attention, except that where its workgroups would leave CUs idle (Dh = 64, a measured
+ * time model decides) the keys are split into contiguous ranges over several
  * workgroups per pair, whose fp32 partial outputs, running maxima and sums go to `workspace` and
  * are merged by a second launch (deterministic, in range order; within the unsplit kernel's error
  * bound, since each range rounds its probabilities to bf16 relative to its own running max, results
