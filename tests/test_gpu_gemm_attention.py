@@ -538,8 +538,8 @@ def _attention_call(entry, q, kv, B, T, H, N, out, *ws):
 def test_attention_key_split(dev, B, T, N, H, scale_up):
     """Few (image, head) pairs with many key tiles (ViT-B at B = 8: 96 pairs of 17 tiles): the keys are
     dealt in contiguous tile ranges to several workgroups per pair, whose fp32 partials a second
-    launch merges (with the light-wave split, the 16-query light wave, the two-wave split of few
-    query waves, a ragged last tile of one key, and large logits inside the parts).
+    launch merges (with the light-wave split, one and several query workgroups per pair, a ragged last
+    tile of one key, and large logits inside the parts).
     Both the split and the unsplit kernel against the float64 reference with the same bound (each
     part rounds its probabilities to bf16 relative to its own running max, so the two differ by about
     a P rounding, which the bound covers); deterministic; and with a workspace one element short the
@@ -666,11 +666,10 @@ def test_attention_one_key_with_a_large_row_stride(dev, T, D):
                                          (16, 257, 193, 16, 0), (1, 1, 1, 1, 0), (1, 40, 130, 1, 1 << 23),
                                          (9, 97, 129, 32, 0), (9, 222, 65, 32, 0)])
 def test_attention_dh128_buffer_loads(dev, B, T, N, H, pad):
-    """Dh = 128: four and eight loader waves, one to 256 pairs, one key past a tile, padded key rows; the
-    case of padding 2^23 has its key rows past the 31-bit byte offsets, and 288 pairs of four query waves take the
-    register-staged kernel too. The output equals
-    the register-staged kernel's (the log-sum-exp entry) bit for bit, and that one is within the bound of
-    the float64 reference."""
+    """Dh = 128: four and eight loader waves, one to 288 pairs, one key past a tile, padded key rows; the case
+    of padding 2^23 has its key rows past the 31-bit byte offsets, and 288 pairs of four query waves take the
+    register-staged kernel too. The output equals the register-staged kernel's (the log-sum-exp entry) bit for
+    bit, and that one is within the bound of the float64 reference."""
     D = 128
     print(f"attention dh128 {B},{T},{N},{H} pad {pad}", flush=True)
     q = _rand((B * T, H, D), 48).to(dev)

@@ -300,7 +300,7 @@ def test_approx_block_caches_the_dense_score(dev, kind):
 @pytest.mark.parametrize("B,H,N,D", [(1, 32, 1029, 128), (2, 4, 77, 64), (1, 8, 300, 64)])
 def test_attention_row_lse_and_fused_score(dev, B, H, N, D):
     """sparse_query_attention(..., lse=) over all N queries of an image: the output equals the call
-    without lse (bit for bit at Dh = 128, where both run the register-staged kernel), lse is the float64
+    without lse (bit for bit at Dh = 128, on whichever kernel that call runs), lse is the float64
     row log-sum-exp of the same bf16 q and K within 2e-4 (fp32 score accumulation, fp32 exponentials and
     an fp32 sum of up to N probabilities; a wrong log base or a dropped max is off by > 0.1), and the
     key-side score computed from it is within the fused score's bound of the oracle."""
