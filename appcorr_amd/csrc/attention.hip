@@ -994,7 +994,8 @@ __global__ __launch_bounds__((DH == 64 && LW == 8 ? kDmaMaxWaves : 8) * 64) void
 static constexpr int kAttnStages = 4;
 static constexpr int kNumCus = 256;     // MI355X
 static constexpr int kMaxKvParts = 8;
-static constexpr int kMinTilesSaved = 8;
+static constexpr int kMinTilesSaved = 8;   // key tiles a workgroup is spared where a split is always taken,
+static constexpr int kMinTilesSplit = 5;   // and at the least
 
 // Merge of the key parts of a split launch. Per (row, head) part p left its running (reference) max
 // m_p, its sum l_p and its unnormalised output o_p, both relative to m_p; with m = max_p m_p and
@@ -1141,7 +1142,10 @@ static AttnShape attn_shape(int64_t B, int64_t T, int64_t H, int64_t Dh, int64_t
   // (1..16 queries) over kLightParts waves (the merge area, 3 parts of 18 x 64 floats, fits the stages). Key
   // parts: the key tiles of each query workgroup dealt to 2 .. kMaxKvParts workgroups in contiguous ranges,
   // whose fp32 rows a merge launch combines (2 us and their bytes); always for few pairs of up to ten waves
-  // and many tiles, else where it is modelled faster.
+  // and many tiles, else where it is modelled faster, in at most two rounds of workgroups, where it spares each
+  // at least five key tiles, and from as many pairs as CUs on only with a light last wave (beyond that the model
+  // flatters the split: 8 x 6 heads, 10 of 300 keys 6.8 us in five parts, 5.8 unsplit; 1 x 12, 33 of 300 7.1, 6.3;
+  // 16 x 16, 52 of 1500 25.2 in two parts, 21.3 unsplit, but 33 of 1500 23.6, 25.9).
   // Measured (HIP graph, evenly filled workgroups of four to ten waves -> this choice, in turn on one card; B x
   // heads, queries of keys): 16 x 16, 1029 of 1029 122 -> 104 us (four workgroups of nine waves -> nine of four;
   // three of eleven are level with those); 16 x 16, 330 of 1029 62.2 -> 34.7 (two of six -> one of eleven);
@@ -1161,7 +1165,9 @@ static AttnShape attn_shape(int64_t B, int64_t T, int64_t H, int64_t Dh, int64_t
     const int all = std::max(split ? w - 1 + kLightParts : w, kMinWaves);
     for (int64_t p = must_split ? 2 : 1; p <= std::min<int64_t>(L, kMaxKvParts); ++p) {
       const int64_t per = cdiv(L, p);
-      if (cdiv(L, per) != p) continue;
+      if (cdiv(L, per) != p || (p > 1 && L - per < kMinTilesSplit)) continue;
+      if (p > 1 && !must_split && ((pairs >= kNumCus && !(n == 1 && last <= 16)) || pairs * n * p > 2 * kNumCus))
+        continue;
       double us = attn_wg_us(pairs * n * p, pairs * p, w, all, n == 1 && last <= 16, per);
       if (p > 1) us += 2.0 + (double)pairs * T * p * (64 + 2) * 4 * 2 / 3e6;
       if (best >= 0.0 && us >= best) continue;

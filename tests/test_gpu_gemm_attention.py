@@ -591,8 +591,8 @@ def test_attention_launch_shapes(dev, B, T, N, H):
 
 # One case per kind of launch the shape model gives at Dh = 64, with the launch it must be: (query workgroups per
 # pair, query waves, waves, light parts, key parts), every number of key parts among them.
-LAUNCHES = [(8, 1, 450, 12, (1, 1, 4, 0, 2)), (5, 1, 450, 16, (1, 1, 4, 0, 3)), (1, 1, 201, 1, (1, 1, 4, 0, 4)),
-            (1, 33, 300, 1, (2, 1, 4, 0, 5)), (1, 33, 700, 1, (2, 1, 4, 0, 6)), (1, 33, 833, 1, (2, 1, 4, 0, 7)),
+LAUNCHES = [(8, 1, 450, 12, (1, 1, 4, 0, 4)), (5, 1, 450, 16, (1, 1, 4, 0, 3)), (1, 1, 201, 1, (1, 1, 4, 0, 1)),
+            (1, 33, 300, 1, (2, 1, 4, 0, 1)), (1, 1, 513, 1, (1, 1, 4, 0, 5)), (1, 33, 700, 1, (2, 1, 4, 0, 6)), (1, 33, 833, 1, (2, 1, 4, 0, 7)),
             (1, 33, 450, 1, (2, 1, 4, 0, 8)), (3, 130, 580, 6, (2, 3, 4, 0, 5)), (3, 200, 580, 16, (2, 4, 4, 0, 2)),
             (16, 70, 1, 12, (1, 3, 4, 0, 1)), (5, 150, 833, 16, (1, 5, 5, 0, 2)), (5, 517, 201, 12, (4, 5, 5, 0, 1)),
             (8, 330, 300, 12, (2, 6, 6, 0, 1)), (16, 200, 201, 12, (1, 7, 7, 0, 1)), (2, 400, 4101, 12, (2, 7, 7, 0, 5)),

@@ -313,3 +313,21 @@ def test_attention_dh128_shapes_where_pairs_outnumber_the_cus():
     for B in (9, 10, 12):
         assert shape(B, 222) == (True, 1, 7, 7) and shape(B, 256) == (True, 1, 8, 8)
         assert shape(B, 150) == (True, 1, 5, 5)
+
+
+def test_attention_dh64_key_parts_spare_five_tiles_or_are_not_taken():
+    """Dh = 64: keys are split only where each workgroup is spared five 64-key tiles or more, and from 256
+    (image, head) pairs on only where the last query wave has 1 to 16 queries (otherwise the merge launch costs
+    more than it saves), at every query count."""
+    from appcorr_amd import kernels as K
+    split = 0
+    for N in (1, 64, 201, 300, 321, 400, 450, 640, 1029, 4101):
+        tiles = -(-N // 64)
+        for B in (1, 2, 4, 8, 16):
+            for H in (1, 6, 12, 16):
+                for T in (1, 10, 33, 64, 130, 261, 1029):
+                    parts = K.sparse_query_attention_shape(B, T, H, 64, N, 2 * H * 64)[5]
+                    assert parts == 1 or tiles - -(-tiles // parts) >= 5, (B, T, N, H, parts)
+                    assert parts == 1 or B * H < 256 or (T - 1) % 32 < 16, (B, T, N, H, parts)
+                    split += parts > 1
+    assert split > 100
